@@ -110,6 +110,10 @@ struct fg_model {
   // first use; w16_inv = 1 / w16_scale; wmax = max |w| of those weights
   bool fwd_f16 = false;
   uint16_t* w16 = nullptr;
+  // the GEMM weights (layers and lm_head, the arena's offsets) in the MFMA
+  // operand layout (tile_at); w16 is in it too. The row-major arena serves
+  // the GEMV, the embedding and the persistent decode's own copy.
+  bf16_t* wt = nullptr;
   float w16_scale = 1.f, w16_inv = 1.f, wmax = 0.f;
   std::string fused_why = "not set up";
   // the single-term fp16 passes' overflow flag (device, one word): set by
@@ -401,13 +405,26 @@ int32_t upload_weights(fg_model* m, const float* const st[8]) {
   HIPCHK(hipStreamSynchronize(m->stream));
   w.lm = w.base + w.layer_stride * d.L;
   w.wte = w.lm + V * D;
+  HIPCHK(hipMalloc((void**)&m->wt, (w.layer_stride * d.L + V * D) * sizeof(bf16_t)));
+  auto tiled = [&](const bf16_t* p, size_t N, size_t K) {
+    launch_tile_weights(m->stream, p, m->wt + (p - w.base), (int64_t)N, (int)K);
+  };
+  for (int l = 0; l < d.L; ++l) {
+    tiled(w.qkv(l), d.nqkv(), D);
+    tiled(w.proj(l), D, qd);
+    tiled(w.fc(l), dff, D);
+    tiled(w.proj2(l), D, dff);
+  }
+  tiled(w.lm, V, D);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(m->stream));
   return setup_fused(m, h.data());
 }
 
 void free_work(fg_model* m) {
   Work& ws = m->ws;
   void* ptrs[] = {ws.x, ws.q, ws.ao, ws.h, ws.logits, ws.ids, ws.tgt, ws.nll, ws.stat, ws.amax,
-                  ws.xs, ws.aos, ws.hs, ws.ssq, ws.part, ws.nllp, m->qs};
+                  ws.xs, ws.aos, ws.hs, ws.ssq, ws.nllp, m->qs};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   ws = Work();
@@ -554,21 +571,12 @@ int32_t ensure_work(fg_model* m, int64_t rows) {
   RCCHK(alloc((void**)&ws.stat, rows * 4));
   RCCHK(alloc((void**)&ws.amax, rows * 4));
   RCCHK(alloc((void**)&m->qs, rows * d.qd() * 2 * 2));
-  RCCHK(alloc((void**)&ws.xs, rows * d.D * 2 * 2));
-  RCCHK(alloc((void**)&ws.aos, rows * d.qd() * 2 * 2));
-  RCCHK(alloc((void**)&ws.hs, rows * d.dff * 2 * 2));
-  RCCHK(alloc((void**)&ws.ssq, rows * (d.D / 64) * 4));
+  const int64_t prow = tile_rows(rows);  // (operand planes hold whole 16-row tiles)
+  RCCHK(alloc((void**)&ws.xs, prow * d.D * 2 * 2));
+  RCCHK(alloc((void**)&ws.aos, prow * d.qd() * 2 * 2));
+  RCCHK(alloc((void**)&ws.hs, prow * d.dff * 2 * 2));
+  RCCHK(alloc((void**)&ws.ssq, rows * (d.D / 16) * 4));
   if (d.V % 256 == 0) RCCHK(alloc((void**)&ws.nllp, rows * (d.V / NLL_GROUP_COLS) * 2 * 4));
-  // split-K partials of the small-M GEMMs: the largest any row count up to
-  // `rows` needs over the five GEMM shapes
-  int64_t part = 0;
-  for (int64_t r = 1; r <= rows && r <= 128; ++r) {
-    const int64_t shapes[5][2] = {{d.nqkv(), d.D}, {d.D, d.qd()}, {d.dff, d.D}, {d.D, d.dff},
-                                  {d.V, d.D}};
-    for (auto& sh : shapes)
-      part = std::max(part, gemm_splitk_floats(r, (int)sh[0], (int)sh[1]));
-  }
-  if (part > 0) RCCHK(alloc((void**)&ws.part, part * 4));
   HIPCHK(hipStreamSynchronize(m->stream));  // the clears, before any caller stream's work
   ws.rows = rows;
   m->work_bytes = total;
@@ -636,7 +644,6 @@ void linear(fg_model* m, hipStream_t s, GemvEpi epi, const GemvArgs& a, const in
 GemvArgs base_args(fg_model* m, const Work& ws) {
   GemvArgs a;
   memset(&a, 0, sizeof a);
-  a.part = ws.part;
   a.eps = m->d.eps;
   a.cosb = m->d_cos;
   a.sinb = m->d_sin;
@@ -681,15 +688,19 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
   const bool gm = !o.rows_single && use_gemm(d, rows);
   // the single-term fp16 pass: MFMA GEMMs of more than 128 rows (no split K)
   const bool f16 = o.f16 && gm && rows > 128 && m->w16;
-  auto W = [&](const bf16_t* p) { return f16 ? m->w16 + (p - m->w.base) : p; };
+  // the GEMMs' weights: the operand-layout copies; the GEMV's: row-major
+  auto W = [&](const bf16_t* p) {
+    return !gm ? p : (f16 ? m->w16 : m->wt) + (p - m->w.base);
+  };
   const int pos_host = o.pos_host < 0 ? pos0 : o.pos_host;
   const bool embed = o.embed;
   // causal (query, key) pairs per (sequence, head) and the attention traffic
   const double pairs = (double)T * pos_host + 0.5 * (double)T * (T + 1);
   const double at_flops = 4.0 * d.hd * d.H * B * pairs;
   const double at_bytes = (double)B * (2.0 * T * d.qd() + 2.0 * (pos_host + T) * d.kvd()) * 4;
-  const int64_t xplane = (int64_t)rows * d.D, aplane = (int64_t)rows * d.qd();
-  const int64_t hplane = (int64_t)rows * d.dff;
+  const int64_t prow = tile_rows(rows);
+  const int64_t xplane = prow * d.D, aplane = prow * d.qd(), hplane = prow * d.dff;
+  const int64_t qplane = (int64_t)rows * d.qd();
   // ssq partials per row after the attention-output RESID
   const int nt_resid = gemm_ssq_parts(rows, d.D, d.qd());
   const int64_t pos_items = o.pos_cnt ? attn_items(d, B, T, pos0) : 0;
@@ -720,7 +731,7 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
     const int npos = npos_pad(pos0 + T);
     if (!one) {
       a.qs = m->qs;
-      a.q_plane = aplane;
+      a.q_plane = qplane;
       a.ks = m->ks;
       a.vt = m->vt;
       a.npos = npos;
@@ -731,33 +742,7 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
     a.ovf = f16 ? m->d_ovf : nullptr;
     a.wscale = m->w16_inv;
     a.w = W(m->w.qkv(l)); a.N = d.nqkv(); a.K = d.D; a.norm = 1; a.y = ws.q;
-    // Batched cached steps (split-K GEMM, one query row per sequence): the
-    // decode attention finishes the QKV's split-K sums itself (row norm,
-    // RoPE, the k/v append) in place of the reduce launch
-    QkvFold qf;
-    bool fold = false;
-    if (one && gm && T == 1 && !o.d_rows && !f16 &&
-        attn_decode_takes_qkv(d, B, maxT, d_pos != nullptr, pos0 + 1, o.kv16)) {
-      int sp = 0;
-      const double M = a.M, N = a.N, K = a.K;  // (linear()'s units)
-      timed(m, s, FG_K_GEMM, 2.0 * M * N * K, N * K * 2 + M * K * 4 + M * N * 4, [&] {
-        sp = launch_gemm_partials(s, GV_QKV, a, d_pos);
-      });
-      if (sp > 0) {
-        fold = true;
-        qf.part = a.part;
-        qf.splits = sp;
-        qf.rows = rows;
-        qf.N = a.N;
-        qf.K = a.K;
-        qf.ssq_n = a.ssq_n;
-        qf.ssq_in = a.ssq_in;
-        qf.eps = a.eps;
-        qf.cosb = a.cosb;
-        qf.sinb = a.sinb;
-      }
-    }
-    if (!fold) linear(m, s, GV_QKV, a, d_pos, gm);
+    linear(m, s, GV_QKV, a, d_pos, gm);
     a.qs = nullptr;
     a.ks = a.vt = nullptr;
     uint16_t* aos = gm ? ws.aos : nullptr;
@@ -765,7 +750,7 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
       timed(m, s, FG_K_ATTN_DECODE, at_flops, at_bytes, [&] {
         launch_attn_decode_pos(s, d, ws.q, lk, lv, o.kv16, B, maxT, d_pos, pos0 + 1, dec_part,
                                o.dec_cnt, ws.ao, aos,
-                               aplane, T, o.d_rows, fold ? &qf : nullptr);
+                               aplane, T, o.d_rows);
       });
     } else {
       if (pos0 > 0)  // earlier cache positions enter the chunk's key planes
@@ -775,7 +760,7 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
                              m->ks, m->vt);
         });
       timed(m, s, FG_K_ATTN_CHUNK, at_flops, at_bytes, [&] {
-        launch_attn_mfma(s, d, m->qs, m->ks, m->vt, B, T, npos, pos0, aplane,
+        launch_attn_mfma(s, d, m->qs, m->ks, m->vt, B, T, npos, pos0, qplane,
                          (int64_t)B * npos * d.kvd(), m->attn_part, ws.ao, aos, aplane, f16,
                          o.pos_cnt ? o.pos_cnt + l * pos_items : nullptr);
       });
@@ -912,6 +897,7 @@ extern "C" int32_t fg_model_destroy(fg_model* m) {
   if (m->w.base) (void)hipFree(m->w.base);
   if (m->fused_w) (void)hipFree(m->fused_w);
   if (m->w16) (void)hipFree(m->w16);
+  if (m->wt) (void)hipFree(m->wt);
   if (m->fused_slots) (void)hipFree(m->fused_slots);
   if (m->fused_err) (void)hipFree(m->fused_err);
   if (m->d_cos) (void)hipFree(m->d_cos);
@@ -2038,10 +2024,10 @@ int32_t ensure_w16(fg_model* m) {
   if (m->wmax * std::ldexp(1.0f, k) > 32768.f)
     return seterr(FG_EARG, "weights up to %g exceed what fp16 holds", (double)m->wmax);
   const size_t n = m->w.layer_stride * m->d.L + (size_t)m->d.V * m->d.D;  // layers + lm_head
-  HIPCHK(hipMalloc((void**)&m->w16, m->w.bytes));  // (the arena's size: offsets stay valid)
+  HIPCHK(hipMalloc((void**)&m->w16, n * 2));  // (the arena's offsets, in the operand layout)
   m->w16_scale = std::ldexp(1.0f, k);
   m->w16_inv = std::ldexp(1.0f, -k);
-  launch_to_f16(m->stream, m->w.base, m->w16, (int64_t)n, m->w16_scale);
+  launch_to_f16(m->stream, m->wt, m->w16, (int64_t)n, m->w16_scale);
   HIPCHK(hipStreamSynchronize(m->stream));
   return FG_OK;
 }

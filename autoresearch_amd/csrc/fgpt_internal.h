@@ -67,6 +67,22 @@ __host__ __device__ inline int pair_dim(int s, int hd) {
   return (s & 1) ? (hd / 2 + (s >> 1)) : (s >> 1);
 }
 
+// Layout of the MFMA GEMM operands (weights and activation planes alike), a
+// matrix of R rows (padded to a multiple of 16) by K columns: 16-row x
+// 32-column tiles of 1 KB, a row block's tiles in column order, and within a
+// tile 16-byte chunks of 8 columns, the 16 rows of one chunk next to each
+// other. Lane l's operand of a 16x16x32 MFMA is then chunk l of a tile, so a
+// wavefront's load is 1 KB of consecutive memory (row-major, it is 16
+// half-used cache lines: a CU then took in ~20 bytes a clock, M = 64 token
+// rows through a [3072][768] matrix 8.0 us against 4.5 in tiles), a 1 KB DMA
+// lands in LDS in the order the MFMA reads it, and those reads meet no bank
+// conflict. Element offset of (r, k):
+__host__ __device__ __forceinline__ int64_t tile_at(int64_t r, int k, int K) {
+  return ((r >> 4) * (K >> 5) + (k >> 5)) * 512 + ((k >> 3) & 3) * 128 + (r & 15) * 8 + (k & 7);
+}
+// Rows of an operand plane for M token rows.
+__host__ __device__ __forceinline__ int64_t tile_rows(int64_t M) { return (M + 15) / 16 * 16; }
+
 // Columns of one log-sum-exp partial of lm_head's cross-entropy epilogue
 // (one wavefront row of the 128x256 register-epilogue tile).
 constexpr int NLL_GROUP_COLS = 128;
@@ -84,14 +100,13 @@ struct Work {
   float* nll = nullptr;     // [rows]
   float* stat = nullptr;    // [rows] per-row scratch (argmax values etc.)
   int32_t* amax = nullptr;  // [rows]
-  // the MFMA path's activations in the split format (hi plane, lo plane
-  // rows*width elements later) and the residual's per-row partial sums of
-  // squares [rows][D/64]
+  // the MFMA path's activations in the split format (hi plane, then lo
+  // plane; each in the GEMM operand layout, tile_at, its rows padded to 16)
+  // and the residual's per-row partial sums of squares, up to [rows][D/16]
   uint16_t* xs = nullptr;   // residual [rows][D]
   uint16_t* aos = nullptr;  // attention output [rows][H*hd]
   uint16_t* hs = nullptr;   // relu2(fc) [rows][4D]
   float* ssq = nullptr;
-  float* part = nullptr;    // split-K partial sums of the small-M GEMMs
   float* nllp = nullptr;    // lm_head's log-sum-exp partials [rows][V/NLL_GROUP_COLS][2]
 };
 
@@ -147,7 +162,8 @@ struct GemvArgs {
   int npos;
   int64_t q_plane, kv_plane;  // elements between the hi and lo planes
   // MFMA GEMM operands in the split format (bf16 hi plane, lo plane
-  // `*_plane` elements later). xs: A rows [M][K]. ssq_in: per-row partial
+  // `*_plane` elements later), every plane and w in the operand layout of
+  // tile_at. xs: A rows [M][K]. ssq_in: per-row partial
   // sums of squares of A, [M][ssq_n] (the row norm). ys: split output
   // (RESID: the updated residual, RELU2: relu^2). ssq_out: RESID only,
   // per-row partial sums of squares of the updated residual, one per
@@ -159,12 +175,7 @@ struct GemvArgs {
   uint16_t* ys;
   int64_t ys_plane;
   float* ssq_out;
-  // split-K scratch for small-M GEMMs (nullable): the K-split partial sums,
-  // [splits][M][N] fp32, reduced in split order by a second kernel that
-  // applies the norm and the epilogue (RESID then writes one ssq partial per
-  // row and 512 columns). Sized by gemm_splitk_floats.
-  float* part;
-  // single-term fp16 pass (MFMA GEMM only, more than 128 rows): A is one fp16
+  // single-term fp16 pass (MFMA GEMM only): A is one fp16
   // plane (xs), W the fp16 copy of the weights scaled by 1 / wscale (a power
   // of 2), the outputs' operand planes fp16 too
   int f16;
@@ -183,11 +194,19 @@ void launch_gemv(hipStream_t s, GemvEpi epi, const GemvArgs& a);
 // MFMA GEMM, C[M][N] = epi(rowscale * (A[M][K] . W[N][K]^T)), A in the
 // split format (xs), W bf16, fp32 accumulation. K must be a multiple of 128.
 void launch_gemm(hipStream_t s, GemvEpi epi, const GemvArgs& a);
-// Number of ssq_out partials per row that a RESID GEMM of M x N x K
-// writes (when it is given split-K scratch, if it splits).
+// Number of ssq_out partials per row that a RESID GEMM of M x N x K writes
+// (at most N / 16).
 int gemm_ssq_parts(int64_t M, int N, int K);
-// Floats of split-K scratch an M x N x K GEMM needs (0: it does not split).
-int64_t gemm_splitk_floats(int64_t M, int N, int K);
+// The same GEMM for few token rows (kern_rows.hip); gemm_rows_tile: the tile
+// it takes for M x N outputs, in units of 16 rows and columns (tm = 0: the
+// pass is not its).
+struct RowsTile {
+  int tm, tn;
+};
+RowsTile gemm_rows_tile(int64_t M, int N);
+void launch_gemm_rows(hipStream_t s, GemvEpi epi, const GemvArgs& a, const int32_t* d_pos);
+// dst = the GEMM operand layout (tile_at) of the row-major matrix src [N][K].
+void launch_tile_weights(hipStream_t s, const bf16_t* src, bf16_t* dst, int64_t N, int K);
 
 // Causal chunk attention of T queries at positions pos0..pos0+T-1 against
 // keys 0..pos0+t, on MFMA from the bf16 hi/lo planes (layouts of
@@ -241,29 +260,11 @@ void launch_gemm_pos(hipStream_t s, GemvEpi epi, const GemvArgs& a, const int32_
 // launch (of B*qpr), on the device.
 int64_t attn_decode_scratch_floats(const Dims& d, int B, int maxT);
 inline int64_t attn_decode_counters(const Dims& d, int rows) { return (int64_t)rows * d.H; }
-// The QKV GEMM's split-K partial sums, left for the single-query attention
-// to finish (sum in split order, row norm, RoPE, the k/v append) instead of
-// a reduce launch: part [splits][rows][N], N = (H + 2 KH) hd in the stored
-// column order; the norm from ssq_in [rows][ssq_n] over K inputs.
-struct QkvFold {
-  const float* part = nullptr;
-  int splits = 0, rows = 0, N = 0, K = 0, ssq_n = 0;
-  const float* ssq_in = nullptr;
-  float eps = 0.f;
-  const float* cosb = nullptr;
-  const float* sinb = nullptr;
-};
-// Whether launch_attn_decode_pos for one query row per sequence (no
-// d_rows; replayed: d_len set) runs the kernel that takes a QkvFold.
-bool attn_decode_takes_qkv(const Dims& d, int B, int maxT, bool replayed, int len, bool kv16);
-// The split-K GEMM alone (no reduce): its partial sums into a.part. Returns
-// the split count, or 0 (nothing launched) when this GEMM is not split.
-int launch_gemm_partials(hipStream_t s, GemvEpi epi, const GemvArgs& a, const int32_t* d_pos);
 void launch_attn_decode_pos(hipStream_t s, const Dims& d, const float* q, const void* kc,
                             const void* vc, bool kv16, int B, int maxT, const int32_t* d_len,
                             int len, float* scratch, uint32_t* cnt, float* y,
                             uint16_t* ys = nullptr, int64_t ys_plane = 0, int qpr = 1,
-                            const int32_t* d_rows = nullptr, const QkvFold* qf = nullptr);
+                            const int32_t* d_rows = nullptr);
 // argmax into out; with d_len/d_len0 set, also into out2[(len-len0)*rows +
 // row] (and the logits row into lgs_out at that slot, when set), then
 // *d_len += 1.

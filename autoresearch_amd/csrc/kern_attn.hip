@@ -103,11 +103,11 @@ __device__ __forceinline__ void split8(const float* v, bf16x8_t& h, bf16x8_t& l)
 // four consecutive output dims (d % 4 == 0): fp32, or the bf16 hi/lo planes
 // the next GEMM reads, one 8-byte store per plane
 template <int HD, bool P16>
-__device__ __forceinline__ void store_out(const AttnArgs& p, int64_t yo, int d, const float (&v)[4]) {
+__device__ __forceinline__ void store_out(const AttnArgs& p, int64_t row, int col, const float (&v)[4]) {
   if (p.ys) {
-    put4<P16>(v, p.ys + yo + d, p.ys_plane);
+    put4<P16>(v, p.ys + tile_at(row, col, p.H * HD), p.ys_plane);
   } else {
-    *(float4*)(p.y + yo + d) = make_float4(v[0], v[1], v[2], v[3]);
+    *(float4*)(p.y + row * p.H * HD + col) = make_float4(v[0], v[1], v[2], v[3]);
   }
 }
 
@@ -331,7 +331,6 @@ __global__ __launch_bounds__(512) void k_attn_mfma(AttnArgs p) {
     xo[ND * 16 * 64 + 64 + lane] = l_run;
   }
   __syncthreads();
-  const int64_t yrow = (int64_t)p.H * HD;
   if (kp == 0 && wact) {
     const float m1 = xo[ND * 16 * 64 + lane], l1 = xo[ND * 16 * 64 + 64 + lane];
     const float m = fmaxf(m_run, m1);
@@ -340,7 +339,7 @@ __global__ __launch_bounds__(512) void k_attn_mfma(AttnArgs p) {
     if (nch == 1) {
       if (tok) {
         const float inv = 1.0f / l;
-        const int64_t yo = ((int64_t)b * p.T + t) * yrow + h * HD;
+        const int64_t yo = (int64_t)b * p.T + t;
 #pragma unroll
         for (int i = 0; i < ND; ++i)
 #pragma unroll
@@ -349,7 +348,7 @@ __global__ __launch_bounds__(512) void k_attn_mfma(AttnArgs p) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
               v[e] = (o[i][4 * r4 + e] * a0 + xo[(i * 16 + 4 * r4 + e) * 64 + lane] * a1) * inv;
-            store_out<HD, P16>(p, yo, 32 * i + 8 * r4 + 4 * g, v);
+            store_out<HD, P16>(p, yo, h * HD + 32 * i + 8 * r4 + 4 * g, v);
           }
       }
     } else {
@@ -393,7 +392,6 @@ __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs p) {
   int base = 0;
   for (int i = p.nqb - 1; i > j; --i) base += chunk_count(i, p.T, p.pos0, p.nvalid, p.ck);
   const int b = bh / p.H, h = bh % p.H;
-  const int64_t yrow = (int64_t)p.H * HD;
   const float* P0 = p.part + ((int64_t)bh * p.iph + base) * PSTR;
   float m = -FLT_MAX;
   if (nch > 8) {
@@ -434,7 +432,7 @@ __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs p) {
   }
   const float inv = 1.0f / l;
   const float v[4] = {acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv};
-  store_out<HD, P16>(p, ((int64_t)b * p.T + tt) * yrow + h * HD, d, v);
+  store_out<HD, P16>(p, (int64_t)b * p.T + tt, h * HD + d, v);
 }
 
 // Cache positions [0, n) of one layer, [B][maxT][KH*hd] -> hi/lo planes

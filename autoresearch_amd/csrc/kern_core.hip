@@ -85,7 +85,7 @@ __global__ __launch_bounds__(256) void k_embed_norm(const bf16_t* __restrict__ w
   for (int k = threadIdx.x; k < D; k += 256) {
     const float v = bf16_to_f32(row[k]) * inv;
     x[r * D + k] = v;
-    if (xs) put1<P16>(v, xs + r * D + k, plane);
+    if (xs) put1<P16>(v, xs + tile_at(r, k, D), plane);
     s2 += v * v;
   }
   if (ssq) {
@@ -365,8 +365,6 @@ struct DecArgs {
                 // floats, so every partial row starts 16-byte aligned)
   uint32_t* cnt;  // (nullable) arrival counters, one per head group, zero
                   // between launches: k_attn_dec merges its own chunks
-  int fold;       // k_attn_dec_loop: q, k, v from qf's split-K sums (qpr == 1)
-  QkvFold qf;
 };
 
 // Floats per partial row of the single-query attention: O (HD), max, sum,
@@ -374,12 +372,13 @@ struct DecArgs {
 __host__ __device__ constexpr int dec_pstride(int hd) { return hd + 4; }
 
 template <int HD>
-__device__ __forceinline__ void dec_store(const DecArgs& a, int64_t o, int d, float4 v) {
+__device__ __forceinline__ void dec_store(const DecArgs& a, int64_t bh, int d, float4 v) {
   if (a.ys) {  // d % 4 == 0: one 8-byte store per plane
     const float w[4] = {v.x, v.y, v.z, v.w};
-    split_bf16x4(w, a.ys + o + d, a.ys_plane);
+    const int r = (int)bh / a.H, h = (int)bh % a.H;
+    split_bf16x4(w, a.ys + tile_at(r, h * HD + d, a.H * HD), a.ys_plane);
   } else {
-    *(float4*)(a.y + o + d) = v;
+    *(float4*)(a.y + bh * HD + d) = v;
   }
 }
 
@@ -488,7 +487,7 @@ __device__ void dec_fold_merge(const DecArgs& a, int row, int h0, int nch, float
       L += w * gml[1][g0 + i];
     }
     const float inv = 1.0f / L;
-    dec_store<HD>(a, ((int64_t)row * a.H + h0 + jj) * HD, d,
+    dec_store<HD>(a, (int64_t)row * a.H + h0 + jj, d,
                   make_float4(t.x * inv, t.y * inv, t.z * inv, t.w * inv));
   }
 }
@@ -609,7 +608,7 @@ __global__ __launch_bounds__(256) void k_attn_dec(DecArgs a) {
     const int64_t bh = (int64_t)row * a.H + h0 + j;
     if (nch == 1) {
       const float inv = 1.0f / lj;
-      dec_store<HD>(a, bh * HD, d, make_float4(t.x * inv, t.y * inv, t.z * inv, t.w * inv));
+      dec_store<HD>(a, bh, d, make_float4(t.x * inv, t.y * inv, t.z * inv, t.w * inv));
     } else {
       float* P = a.part + (bh * a.nchunk + c) * dec_pstride(HD);
       const float mj = fmaxf(fmaxf(red[0][0][j], red[0][1][j]), fmaxf(red[0][2][j], red[0][3][j]));
@@ -639,138 +638,6 @@ __global__ __launch_bounds__(256) void k_attn_dec(DecArgs a) {
   dec_fold_merge<HD, GH>(a, row, h0, nch, &so[0][0][0], gml);
 }
 
-// The QKV projection's tail for one query row, done by the attention that
-// consumes it (a batched cached step whose QKV GEMM split K): the split
-// partial sums added in split order, eight at a time, the row's rmsnorm
-// scale, RoPE at position pos, as k_splitk_reduce and the QKV epilogue have
-// it (stored column pair 2i, 2i+1 of a head holds dims i and i + hd/2).
-// Thread t takes item t: pair t of the GH query heads h0.., then, with kv
-// set, pair t - GH*HD/2 of the KV head's k and then v (at most (GH+2)*HD/2
-// items, no more than the workgroup's threads). fold_load issues every load
-// the item needs at once (the first eight splits, four of the row's
-// sum-of-squares partials, the RoPE pair), ahead of the kernel's first K
-// rows; fold_pin, after those, marks where the values must have arrived;
-// fold_finish adds them (and any further splits and partials), and leaves q
-// in sq and the new k and v (their cached values: bf16-rounded for a bf16
-// cache) in skv, and with put set also in the cache at pos.
-struct FoldIn {
-  float2 pv[8];
-  float ss[4];
-  float cs, sn;
-};
-
-template <int HD, int GH>
-__device__ __forceinline__ int fold_col(const DecArgs& a, int h0, int kvh, bool kv, int& grp,
-                                        int& i) {
-  constexpr int NP = HD / 2;  // rotation pairs per head
-  const int it = threadIdx.x;
-  grp = it / NP;  // q heads 0..GH-1, then k, then v
-  i = it % NP;
-  if (it >= (GH + (kv ? 2 : 0)) * NP) return -1;
-  return grp < GH ? (h0 + grp) * HD + 2 * i
-                  : a.H * HD + (grp - GH) * a.KH * HD + kvh * HD + 2 * i;
-}
-
-// (Every load goes out, from a clamped and valid address; the unused
-// values are dropped later: conditional loads would become branches that
-// each wait for their load.)
-template <int HD, int GH>
-__device__ __forceinline__ void fold_load(const DecArgs& a, int row, int h0, int kvh, bool kv,
-                                          int pos, FoldIn& in) {
-  const QkvFold& f = a.qf;
-  int grp, i;
-  const int n = fold_col<HD, GH>(a, h0, kvh, kv, grp, i);
-  const float* P = f.part + (int64_t)row * f.N + max(n, 0);
-  const int64_t stride = (int64_t)f.rows * f.N;
-#pragma unroll
-  for (int k = 0; k < 8; ++k)
-    in.pv[k] = *reinterpret_cast<const float2*>(P + min(k, f.splits - 1) * stride);
-#pragma unroll
-  for (int t = 0; t < 4; ++t) in.ss[t] = f.ssq_in[(int64_t)row * f.ssq_n + min(t, f.ssq_n - 1)];
-  const int64_t at = (int64_t)pos * (HD / 2) + i;
-  in.cs = f.cosb[at];
-  in.sn = f.sinb[at];
-}
-
-__device__ __forceinline__ void fold_pin(FoldIn& in) {
-#pragma unroll
-  for (int k = 0; k < 8; ++k) asm volatile("" : "+v"(in.pv[k].x), "+v"(in.pv[k].y) : : "memory");
-  asm volatile("" : "+v"(in.ss[0]), "+v"(in.ss[1]), "+v"(in.ss[2]), "+v"(in.ss[3]),
-               "+v"(in.cs), "+v"(in.sn) : : "memory");
-}
-
-template <int HD, int GH, class KT>
-__device__ void fold_finish(const DecArgs& a, int row, int h0, int kvh, int pos, bool kv,
-                            bool put, const FoldIn& in, float (*sq)[HD], float (*skv)[HD]) {
-  const QkvFold& f = a.qf;
-  constexpr int NP = HD / 2;
-  int grp, i;
-  const int n = fold_col<HD, GH>(a, h0, kvh, kv, grp, i);
-  if (n < 0) return;
-  float v0 = 0.f, v1 = 0.f;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {  // split order (a zero adds nothing)
-    const float2 x = k < f.splits ? in.pv[k] : make_float2(0.f, 0.f);
-    v0 += x.x;
-    v1 += x.y;
-  }
-  const float* P = f.part + (int64_t)row * f.N + n;
-  const int64_t stride = (int64_t)f.rows * f.N;
-  for (int s0 = 8; s0 < f.splits; s0 += 8) {
-    float2 pv[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-      pv[k] = s0 + k < f.splits ? *reinterpret_cast<const float2*>(P + (s0 + k) * stride)
-                                : make_float2(0.f, 0.f);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      v0 += pv[k].x;
-      v1 += pv[k].y;
-    }
-  }
-  float ssum = 0.f;
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-    if (t < f.ssq_n) ssum += in.ss[t];
-  for (int t = 4; t < f.ssq_n; ++t) ssum += f.ssq_in[(int64_t)row * f.ssq_n + t];
-  const float inv = 1.0f / sqrtf(ssum / (float)f.K + f.eps);
-  v0 *= inv;
-  v1 *= inv;
-  float y1 = v0, y2 = v1;
-  if (grp <= GH) {  // q and k: rotated
-    const float cs = in.cs, sn = in.sn;
-    y1 = v0 * cs + v1 * sn;
-    y2 = v0 * (-sn) + v1 * cs;
-  }
-  if (grp < GH) {
-    sq[grp][i] = y1;
-    sq[grp][i + NP] = y2;
-    return;
-  }
-  const int t = grp - GH;  // 0: k, 1: v
-  // (row = sequence: one query row each; the cache operands are read-only
-  // to every other kernel of the launch)
-  const int64_t at = (int64_t)(row * a.maxT + pos) * a.KH * HD + kvh * HD;
-  if constexpr (sizeof(KT) == 2) {
-    const uint16_t h1 = f32_to_bf16_rne(y1), h2 = f32_to_bf16_rne(y2);
-    skv[t][i] = bf16_to_f32(h1);
-    skv[t][i + NP] = bf16_to_f32(h2);
-    if (put) {
-      uint16_t* c = (uint16_t*)(t ? a.vc : a.kc) + at;
-      c[i] = h1;
-      c[i + NP] = h2;
-    }
-  } else {
-    skv[t][i] = y1;
-    skv[t][i + NP] = y2;
-    if (put) {
-      float* c = (float*)(t ? a.vc : a.kc) + at;
-      c[i] = y1;
-      c[i + NP] = y2;
-    }
-  }
-}
-
 // k_attn_dec over a.iters consecutive blocks of DPC positions per
 // workgroup (NWV wavefronts, DPC / NWV positions each per block), for
 // batches with rows x KV heads enough to fill the chip without splitting
@@ -781,11 +648,8 @@ __device__ void fold_finish(const DecArgs& a, int row, int h0, int kvh, int pos,
 // rescaled to the workgroup maximum, and leave as
 // k_attn_dec's do (the output, or a partial for k_attn_dec_merge). While a
 // block's scores are formed its V rows load, and the next block's K rows
-// load while its V rows are weighed. With FOLD the kernel also finishes the
-// step's QKV projection (fold_load / fold_finish): the query comes from the
-// split-K partials, and the new position, not cached yet, is added by the
-// last chunk from the k and v it computed (and appended to the cache).
-template <int HD, int DPC, int GH, class KT, int NWV = 4, bool FOLD = false>
+// load while its V rows are weighed.
+template <int HD, int DPC, int GH, class KT, int NWV = 4>
 __global__ __launch_bounds__(64 * NWV) void k_attn_dec_loop(DecArgs a) {
   constexpr int LPP = HD / 8;        // lanes per cached row
   constexpr int PPW = 64 / LPP;      // rows per wavefront load
@@ -793,7 +657,6 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_dec_loop(DecArgs a) {
   static_assert(LPP == 8 || LPP == 16, "head dim 64 or 128");
   __shared__ float red[3][NWV][GH];
   __shared__ float so[NWV * PPW][GH][HD];
-  __shared__ float sq[FOLD ? GH : 1][HD], skv[FOLD ? 2 : 1][HD];  // (FOLD) q; new k, v
   const int G = a.H / a.KH, ng = G / GH;
   const int gi = blockIdx.x, c = blockIdx.y;
   const int row = gi / (a.KH * ng), kvh = (gi / ng) % a.KH, h0 = kvh * G + (gi % ng) * GH;
@@ -803,12 +666,8 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_dec_loop(DecArgs a) {
   const int p0 = c * span;
   if (p0 >= len) return;
   const int nch = (len + span - 1) / span;
-  // With FOLD the new position len-1 is not in the cache yet: the cached
-  // positions stop at lenc, and the last chunk adds the new one from skv.
-  const int lenc = FOLD ? len - 1 : len;
-  const int plast = max(lenc - 1, 0);  // (loads past lenc repeat a cached row)
-  const int nblk = min(a.iters, (lenc - p0 + DPC - 1) / DPC);  // blocks with positions < lenc
-  const bool last = c == nch - 1;
+  const int plast = len - 1;  // (loads past it repeat a cached row)
+  const int nblk = min(a.iters, (len - p0 + DPC - 1) / DPC);  // blocks with positions < len
   const int b = row / a.qpr;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int sub = lane / LPP, dl = lane % LPP;
@@ -825,32 +684,15 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_dec_loop(DecArgs a) {
   };
   auto pos = [&](int blk, int i) { return p0 + blk * DPC + wv * (DPC / NWV) + i * PPW + sub; };
   Row8<KT> kr[IT], vr[IT];
-  FoldIn fin;
-  if constexpr (FOLD) {
-    fold_load<HD, GH>(a, row, h0, kvh, last, len - 1, fin);
-    asm volatile("" ::: "memory");  // (those loads go out before the K rows')
-  }
 #pragma unroll
   for (int i = 0; i < IT; ++i) kr[i].load(rowp(Kb, pos(0, i)));
   float qv[GH][8];
-  if constexpr (FOLD) {
-    fold_pin(fin);
-    fold_finish<HD, GH, KT>(a, row, h0, kvh, len - 1, last, last && gi % ng == 0, fin, sq, skv);
-    __syncthreads();
 #pragma unroll
-    for (int j = 0; j < GH; ++j) {
-      const float4 u = *(const float4*)&sq[j][8 * dl], w = *(const float4*)&sq[j][8 * dl + 4];
-      qv[j][0] = u.x; qv[j][1] = u.y; qv[j][2] = u.z; qv[j][3] = u.w;
-      qv[j][4] = w.x; qv[j][5] = w.y; qv[j][6] = w.z; qv[j][7] = w.w;
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < GH; ++j) {
-      const float* qp = a.q + ((int64_t)row * a.H + h0 + j) * HD + 8 * dl;
-      const float4 u = *(const float4*)qp, w = *(const float4*)(qp + 4);
-      qv[j][0] = u.x; qv[j][1] = u.y; qv[j][2] = u.z; qv[j][3] = u.w;
-      qv[j][4] = w.x; qv[j][5] = w.y; qv[j][6] = w.z; qv[j][7] = w.w;
-    }
+  for (int j = 0; j < GH; ++j) {
+    const float* qp = a.q + ((int64_t)row * a.H + h0 + j) * HD + 8 * dl;
+    const float4 u = *(const float4*)qp, w = *(const float4*)(qp + 4);
+    qv[j][0] = u.x; qv[j][1] = u.y; qv[j][2] = u.z; qv[j][3] = u.w;
+    qv[j][4] = w.x; qv[j][5] = w.y; qv[j][6] = w.z; qv[j][7] = w.w;
   }
   // scores in log2 units (scale x log2(e)): each weight is one v_exp_f32 of
   // a difference; the maximum handed to the merge is converted back
@@ -880,7 +722,7 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_dec_loop(DecArgs a) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v += qv[j][e] * x[e];
         v = row_sum<LPP>(v);
-        sc[j][i] = p < lenc ? v * scale : -INFINITY;
+        sc[j][i] = p < len ? v * scale : -INFINITY;
         mx[j] = fmaxf(mx[j], sc[j][i]);
       }
     }
@@ -907,33 +749,6 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_dec_loop(DecArgs a) {
         l[j] += w;
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[j][e] += w * x[e];
-      }
-    }
-  }
-  if (FOLD && last && wv == 0) {  // the new position, one row of wavefront 0
-    float kx[8], vx[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      kx[e] = skv[0][8 * dl + e];
-      vx[e] = skv[1][8 * dl + e];
-    }
-#pragma unroll
-    for (int j = 0; j < GH; ++j) {
-      float v = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v += qv[j][e] * kx[e];
-      const float sc = row_sum<LPP>(v) * scale;
-      const float mn = fmaxf(m[j], sc);
-      const float alpha = __builtin_amdgcn_exp2f(m[j] - mn);
-      m[j] = mn;
-      l[j] *= alpha;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[j][e] *= alpha;
-      if (sub == 0) {
-        const float w = __builtin_amdgcn_exp2f(sc - mn);
-        l[j] += w;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[j][e] += w * vx[e];
       }
     }
   }
@@ -976,7 +791,7 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_dec_loop(DecArgs a) {
     const int64_t bh = (int64_t)row * a.H + h0 + j;
     if (nch == 1) {
       const float inv = 1.0f / lj;
-      dec_store<HD>(a, bh * HD, d, make_float4(t.x * inv, t.y * inv, t.z * inv, t.w * inv));
+      dec_store<HD>(a, bh, d, make_float4(t.x * inv, t.y * inv, t.z * inv, t.w * inv));
     } else {
       float* P = a.part + (bh * a.nchunk + c) * dec_pstride(HD);
       *(float4*)(P + d) = t;
@@ -1050,7 +865,7 @@ __global__ __launch_bounds__(256) void k_attn_dec_merge(DecArgs a, int dpc) {
     L += sl[k];
   }
   const float inv = 1.0f / L;
-  dec_store<HD>(a, (int64_t)bh * HD, 4 * tid, make_float4(t.x * inv, t.y * inv, t.z * inv, t.w * inv));
+  dec_store<HD>(a, bh, 4 * tid, make_float4(t.x * inv, t.y * inv, t.z * inv, t.w * inv));
 }
 
 int attn_decode_chunks(int maxT) { return (maxT + DPC_MIN - 1) / DPC_MIN; }
@@ -1084,30 +899,14 @@ void launch_dec_gh(hipStream_t s, const DecArgs& a, int rows, int gh) {
     if (a.iters > 1 && a.iters % 2 == 0) {
       DecArgs b2 = a;
       b2.iters = a.iters / 2;
-      if (a.fold) {
-        if (gh == 2)
-          FG_LAUNCH((k_attn_dec_loop<HD, 256, 2, KT, 8, true>), grid, dim3(512), 0, s, b2);
-        else
-          FG_LAUNCH((k_attn_dec_loop<HD, 256, 1, KT, 8, true>), grid, dim3(512), 0, s, b2);
-      } else {
-        if (gh == 2)
-          FG_LAUNCH((k_attn_dec_loop<HD, 256, 2, KT, 8>), grid, dim3(512), 0, s, b2);
-        else
-          FG_LAUNCH((k_attn_dec_loop<HD, 256, 1, KT, 8>), grid, dim3(512), 0, s, b2);
-      }
+      if (gh == 2)
+        FG_LAUNCH((k_attn_dec_loop<HD, 256, 2, KT, 8>), grid, dim3(512), 0, s, b2);
+      else
+        FG_LAUNCH((k_attn_dec_loop<HD, 256, 1, KT, 8>), grid, dim3(512), 0, s, b2);
       return;
     }
   }
   if (a.iters > 1) {  // (DPC 128 only: dec_group's options for it)
-    if constexpr (DPC == 128) {
-      if (a.fold) {
-        if (gh == 2)
-          FG_LAUNCH((k_attn_dec_loop<HD, DPC, 2, KT, 4, true>), grid, dim3(256), 0, s, a);
-        else
-          FG_LAUNCH((k_attn_dec_loop<HD, DPC, 1, KT, 4, true>), grid, dim3(256), 0, s, a);
-        return;
-      }
-    }
     if (gh == 2)
       FG_LAUNCH((k_attn_dec_loop<HD, DPC, 2, KT>), grid, dim3(256), 0, s, a);
     else
@@ -1173,15 +972,10 @@ DecPlan dec_plan(const Dims& d, int B, int maxT, bool replayed, int len, int qpr
 
 }  // namespace
 
-bool attn_decode_takes_qkv(const Dims& d, int B, int maxT, bool replayed, int len, bool kv16) {
-  return dec_plan(d, B, maxT, replayed, len, 1, kv16).iters > 1;  // k_attn_dec_loop
-}
-
 void launch_attn_decode_pos(hipStream_t s, const Dims& d, const float* q, const void* kc,
                             const void* vc, bool kv16, int B, int maxT, const int32_t* d_len,
                             int len, float* scratch, uint32_t* cnt, float* y, uint16_t* ys,
-                            int64_t ys_plane, int qpr, const int32_t* d_rows,
-                            const QkvFold* qf) {
+                            int64_t ys_plane, int qpr, const int32_t* d_rows) {
   DecArgs a;
   a.q = q;
   a.kc = kc;
@@ -1192,14 +986,6 @@ void launch_attn_decode_pos(hipStream_t s, const Dims& d, const float* q, const 
   const DecPlan pl = dec_plan(d, B, maxT, d_len != nullptr, len, qpr, kv16);
   const int dpc = pl.dpc, live = pl.live, gh = pl.gh, iters = pl.iters;
   const int rows = B * qpr;
-  // a caller passes qf only where attn_decode_takes_qkv holds for the same
-  // arguments; the QKV's sums would go unfinished otherwise
-  if (qf && (iters <= 1 || qpr != 1 || d_rows)) {
-    std::fprintf(stderr, "fgpt: internal error: QKV fold for a launch that cannot take it\n");
-    std::abort();
-  }
-  a.fold = qf ? 1 : 0;
-  if (qf) a.qf = *qf;
   a.iters = iters;
   a.nchunk = (live + dpc * iters - 1) / (dpc * iters);
   a.d_len = d_len;

@@ -114,6 +114,27 @@ __device__ __forceinline__ void put4(const float (&v)[4], uint16_t* p, int64_t p
     split_bf16x4<NT>(v, p, plane);
 }
 
+// Eight adjacent values as one 16-byte store per plane (p a multiple of 8
+// elements).
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+template <bool P16, bool NT = false>
+__device__ __forceinline__ void put8(const float (&v)[8], uint16_t* p, int64_t plane) {
+  u32x4_t h, l;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (P16) {
+      h[i] = (uint32_t)f32_to_f16_rne(v[2 * i]) | ((uint32_t)f32_to_f16_rne(v[2 * i + 1]) << 16);
+    } else {
+      const uint16_t h0 = f32_to_bf16_rne(v[2 * i]), h1 = f32_to_bf16_rne(v[2 * i + 1]);
+      h[i] = (uint32_t)h0 | ((uint32_t)h1 << 16);
+      l[i] = (uint32_t)f32_to_bf16_rne(v[2 * i] - bf16_to_f32(h0)) |
+             ((uint32_t)f32_to_bf16_rne(v[2 * i + 1] - bf16_to_f32(h1)) << 16);
+    }
+  }
+  store_v<NT>(reinterpret_cast<u32x4_t*>(p), h);
+  if constexpr (!P16) store_v<NT>(reinterpret_cast<u32x4_t*>(p + plane), l);
+}
+
 // The single-term fp16 pass stores its activations as fp16, whose largest
 // finite value is 65504: an fp32 value of magnitude 65520 or more (or one
 // that is not finite) would become inf. Such a value raises the pass's

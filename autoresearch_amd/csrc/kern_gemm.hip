@@ -18,9 +18,11 @@
 //
 // Pipeline: NST stages of BK-wide K slices (BK = 32, 64 or 128) in LDS,
 // filled by global_load_lds_dwordx4 (memory -> LDS without registers),
-// NST-1 slices in flight while the MFMAs consume the oldest. Each LDS row
-// holds its 16-byte chunks XOR-swizzled by row so the MFMA operand reads
-// (32 rows x one chunk per half-wavefront) do not collide in banks.
+// NST-1 slices in flight while the MFMAs consume the oldest. Both operands
+// are stored in 1 KB tiles of 16 rows x 32 K (tile_at), so each DMA reads 1 KB
+// of consecutive memory and a stage is a list of tiles: the MFMA operand
+// reads (32 rows x one 16-byte chunk per half-wavefront) are two runs of 256
+// consecutive bytes, free of bank conflicts without a swizzle.
 // Tiling: BM x BN per block of NWM x NWN 64-wide wavefronts, each owning
 // (BM/NWM) x (BN/NWN) as 32x32 MFMA blocks, times KG groups of such
 // wavefronts that split each slice's K steps between them. The epilogue is
@@ -42,6 +44,7 @@ constexpr bool NT_RELU2 = true, NT_RESID = true, NT_QKV = false;
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 // One 32x32x16 MFMA step: bf16 operands, or (P16) fp16 ones.
 template <bool P16>
@@ -55,17 +58,11 @@ __device__ __forceinline__ f32x16_t mma16(const bf16x8_t& a, const bf16x8_t& b, 
 
 namespace {
 
-// 16-byte chunk slot of logical chunk c in row r of a stage whose rows hold
-// BK bf16 (BK/8 chunks). gfx950's LDS has 64 banks (256 bytes a cycle), and
-// a 16-byte read is served 16 lanes at a time: the 16 rows an MFMA operand
-// read touches at one logical chunk must land on 16 different 16-byte bank
-// groups. 128 / BK rows fill 256 bytes, so the XOR pattern changes every
-// 128 / BK rows (every 4 rows of 64 bytes, every 2 rows of 128 bytes).
-template <int BK>
-__device__ __forceinline__ int swz(int r, int c) {
-  constexpr int S = BK == 32 ? 2 : BK == 64 ? 1 : 0;
-  static_assert(BK == 32 || BK == 64 || BK == 128, "stage row width");
-  return c ^ ((r >> S) & (BK / 8 - 1));
+// Byte offset within a stage (k tiles of RT row tiles each) of the 16-byte
+// chunk c of row r.
+template <int RT>
+__device__ __forceinline__ int at(int r, int c) {
+  return ((c >> 2) * RT + (r >> 4)) * 1024 + ((c & 3) * 16 + (r & 15)) * 16;
 }
 
 template <int N>
@@ -172,18 +169,17 @@ __global__ __launch_bounds__(64 * NWM * NWN * KG) void k_gemm(GemvArgs a,
                                                              const int32_t* __restrict__ d_pos) {
   constexpr int NWT = NWM * NWN, NW = NWT * KG, NT = 64 * NW;
   constexpr int WM = BM / (32 * NWM), WN = BN / (32 * NWN);  // 32x32 blocks per wave
-  // a stage: A hi rows, A lo rows, W rows of RB bytes each, loaded 1 KB
-  // (1024 / RB rows) per wavefront instruction
-  constexpr int RB = 2 * BK, CPR = BK / 8, RPG = 1024 / RB;
+  // a stage: for each 32 of K the tiles of A hi, A lo and W, one wavefront
+  // instruction each
   constexpr int AP = P16 ? 1 : 2;  // operand planes of A (hi and lo, or one fp16)
-  constexpr int ROWS = AP * BM + BN;
-  constexpr int GROUPS = ROWS / RPG;         // 1 KB load groups per stage
+  constexpr int ROWS = AP * BM + BN, RT = ROWS / 16;
+  constexpr int GROUPS = RT * (BK / 32);     // 1 KB tiles per stage
   // groups per wavefront per stage; when NW does not divide GROUPS, the
   // spare slots repeat the last group (the same bytes to the same place)
   constexpr int GPW = (GROUPS + NW - 1) / NW;
-  static_assert(ROWS % RPG == 0 && WM >= 1 && WN >= 1, "tile / wave grid mismatch");
+  static_assert(WM >= 1 && WN >= 1, "tile / wave grid mismatch");
   static_assert(KG == 1 || (BM == 64 && (BK / 16) % KG == 0), "K groups: one 64-row pass");
-  constexpr int STAGE_BYTES = ROWS * RB;
+  constexpr int STAGE_BYTES = GROUPS * 1024;
   constexpr int SSTR = BN + 4;  // epilogue staging row stride (floats)
   // NST stages of STAGE_BYTES; after the K loop the same memory (sized for
   // the larger of the two) stages the epilogue (the DMA is issued from asm, so the compiler never waits on it
@@ -202,48 +198,43 @@ __global__ __launch_bounds__(64 * NWM * NWN * KG) void k_gemm(GemvArgs a,
   if ((ntile & 7) == 0) lin = (lin & 7) * (ntile >> 3) + (lin >> 3);
   const int m0 = (lin / nbn) * BM, n0 = (lin % nbn) * BN;
   const int M = a.M, K = a.K;
-  // split-K (a.part set): this block sums K range [kz*klen, kz*klen + klen)
-  const int kz = blockIdx.z, klen = K / (int)gridDim.z, kbeg = kz * klen;
 
-  // This lane's source rows for each of its load groups (fixed for the whole
-  // K loop): group g covers stage rows RPG*g .. RPG*g+RPG-1; lane -> row
-  // RPG*g + l/CPR, LDS slot l%CPR, which holds logical chunk swz(row, slot).
+  // This lane's source of each of its load groups: chunk `lane` of tile g's
+  // 1 KB (row tiles past M repeat the last one and are never stored); a
+  // K slice further on is BK / 32 tiles (16 BK elements) away.
   const uint16_t* src[GPW];
 #pragma unroll
   for (int q = 0; q < GPW; ++q) {
-    const int g = min(wid + NW * q, GROUPS - 1);
-    const int r = RPG * g + lane / CPR, slot = lane % CPR;
-    const int c = swz<BK>(r, slot);
-    if (r < AP * BM) {  // A hi (r < BM) or A lo
-      const int ar = r < BM ? r : r - BM;
-      const int row = min(m0 + ar, M - 1);  // rows past M are never stored
-      src[q] = a.xs + (r < BM ? 0 : a.xs_plane) + (int64_t)row * K + kbeg + c * 8;
+    const int g = min(wid + NW * q, GROUPS - 1), rt = g % RT, kt = g / RT;
+    const uint16_t* base;
+    if (rt < AP * (BM / 16)) {  // A hi, then A lo
+      const int ar = rt < BM / 16 ? rt : rt - BM / 16;
+      base = a.xs + (rt < BM / 16 ? 0 : a.xs_plane) +
+             (int64_t)min((m0 >> 4) + ar, (M - 1) >> 4) * K * 16;
     } else {
-      src[q] = a.w + (int64_t)(n0 + r - AP * BM) * K + kbeg + c * 8;
+      base = a.w + (int64_t)((n0 >> 4) + rt - AP * (BM / 16)) * K * 16;
     }
+    src[q] = base + kt * 512 + lane * 8;
   }
 
-  // epilogue items (column pairs of a 64-row pass) per thread
-  constexpr int EPT = 64 * (BN / 2) / NT;
-  static_assert(EPT * NT == 64 * (BN / 2), "epilogue pass / block size mismatch");
-  // RESID row sums of squares: within the wavefront when a row's BN / 2
-  // column pairs are exactly one wavefront (BN = 128) or half of one
-  // (BN = 64), else through LDS (sqs, a padded [64][BN / 2] after the
-  // staged tile), each row summed in column order by one thread
-  constexpr bool SQ_LDS = EPI == GV_RESID && BN != 64 && BN != 128;
-  constexpr int SQS = BN / 2 + 1;
+  // epilogue items (8 columns of one row of a 64-row pass) per thread
+  constexpr int ITEMS = 64 * (BN / 8), EPT = (ITEMS + NT - 1) / NT;
+  // RESID row sums of squares: one value per item in LDS (sqs, a padded
+  // [64][BN / 8] after the staged tile), a row's summed by four threads
+  constexpr int SQS = BN / 8 + 1;
   // RESID: the residual tile is read now, so its latency hides behind the
   // K loop instead of stalling the epilogue
-  float2 xres[EPI == GV_RESID ? (BM / 64) * EPT : 1];
-  if (EPI == GV_RESID && !a.part) {
+  float4 xres[EPI == GV_RESID ? (BM / 64) * EPT : 1][2];
+  if (EPI == GV_RESID) {
 #pragma unroll
     for (int q = 0; q < BM / 64; ++q)
 #pragma unroll
       for (int k = 0; k < EPT; ++k) {
-        const int e = tid + k * NT, m = m0 + q * 64 + e / (BN / 2);
-        xres[q * EPT + k] = m < M ? *reinterpret_cast<const float2*>(
-                                        a.y + (int64_t)m * a.N + n0 + 2 * (e % (BN / 2)))
-                                  : make_float2(0.f, 0.f);
+        const int e = min(tid + k * NT, ITEMS - 1), m = min(m0 + q * 64 + e / (BN / 8), M - 1);
+        const float4* p = reinterpret_cast<const float4*>(a.y + (int64_t)m * a.N + n0 +
+                                                          8 * (e % (BN / 8)));
+        xres[q * EPT + k][0] = p[0];
+        xres[q * EPT + k][1] = p[1];
       }
   }
 
@@ -255,15 +246,15 @@ __global__ __launch_bounds__(64 * NWM * NWN * KG) void k_gemm(GemvArgs a,
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  const int nk = klen / BK;  // klen % BK == 0 (checked by the host)
-  const int klast = klen - BK;
+  const int nk = K / BK;  // K % BK == 0 (checked by the host)
+  const int klast = K - BK;
   uint32_t ldsq[GPW];  // LDS byte offset of each of this wavefront's groups
 #pragma unroll
   for (int q = 0; q < GPW; ++q)
     ldsq[q] = __builtin_amdgcn_readfirstlane(lds_off(smem) + min(wid + NW * q, GROUPS - 1) * 1024);
   auto fill = [&](int stg, int k0) {
 #pragma unroll
-    for (int q = 0; q < GPW; ++q) dma16(src[q] + k0, ldsq[q] + stg * STAGE_BYTES);
+    for (int q = 0; q < GPW; ++q) dma16(src[q] + k0 * 16, ldsq[q] + stg * STAGE_BYTES);
   };
   auto consume = [&](int si) {
     const uint8_t* stg = smem + si * STAGE_BYTES;
@@ -275,13 +266,13 @@ __global__ __launch_bounds__(64 * NWM * NWN * KG) void k_gemm(GemvArgs a,
 #pragma unroll
       for (int i = 0; i < WM; ++i) {
         const int r = (wm * WM + i) * 32 + (lane & 31);
-        ah[i] = *(const bf16x8_t*)(stg + r * RB + swz<BK>(r, c) * 16);
-        if constexpr (!P16) al[i] = *(const bf16x8_t*)(stg + (BM + r) * RB + swz<BK>(BM + r, c) * 16);
+        ah[i] = *(const bf16x8_t*)(stg + at<RT>(r, c));
+        if constexpr (!P16) al[i] = *(const bf16x8_t*)(stg + at<RT>(BM + r, c));
       }
 #pragma unroll
       for (int j = 0; j < WN; ++j) {
         const int r = AP * BM + (wn * WN + j) * 32 + (lane & 31);
-        bw[j] = *(const bf16x8_t*)(stg + r * RB + swz<BK>(r, c) * 16);
+        bw[j] = *(const bf16x8_t*)(stg + at<RT>(r, c));
       }
 #pragma unroll
       for (int i = 0; i < WM; ++i)
@@ -315,7 +306,7 @@ __global__ __launch_bounds__(64 * NWM * NWN * KG) void k_gemm(GemvArgs a,
   __syncthreads();
 
   // row scale from the producer's partial sums of squares
-  if (a.norm && !a.part) {
+  if (a.norm) {
     for (int r = tid; r < BM; r += NT) {
       float ssum = 0.f;
       if (m0 + r < M)
@@ -330,7 +321,7 @@ __global__ __launch_bounds__(64 * NWM * NWN * KG) void k_gemm(GemvArgs a,
   // Tiles holding v columns that go to the transposed bf16 layout
   // ([..][hd][npos]: positions contiguous) walk the staged tile row-fastest,
   // so a wavefront's stores cover 64 consecutive positions of one dim.
-  const bool rows_fast = EPI == GV_QKV && a.vt && !a.part && n0 + BN > (a.H + a.KH) * a.hd;
+  const bool rows_fast = EPI == GV_QKV && a.vt && n0 + BN > (a.H + a.KH) * a.hd;
   float* sqs = stage + KG * 64 * SSTR;
 #pragma unroll
   for (int q = 0; q < BM / 64; ++q) {
@@ -372,81 +363,78 @@ __global__ __launch_bounds__(64 * NWM * NWN * KG) void k_gemm(GemvArgs a,
         __syncthreads();
       }
     }
-    // BN/2 consecutive e cover one row; with BN = 128 that is one
-    // wavefront, with BN = 64 half of one (reductions stay in the wave)
     if constexpr (EPI == GV_QKV) {
-      if (!a.part) {
-        qkv_tile_pass<BN, NT, P16>(a, stage, sinv, m0, n0, q, rows_fast, pos0);
-        __syncthreads();
-        continue;
-      }
+      qkv_tile_pass<BN, NT, P16>(a, stage, sinv, m0, n0, q, rows_fast, pos0);
+      __syncthreads();
+      continue;
     }
+    // RELU2 writes planes only: items row-fastest, so 16 lanes store 256
+    // consecutive bytes; RESID and STORE also touch row-major fp32: four
+    // lanes per 128 bytes of a row
 #pragma unroll
     for (int k = 0; k < EPT; ++k) {
       const int e = tid + k * NT;
-      const int srow = rows_fast ? e % 64 : e / (BN / 2);
-      const int pc = rows_fast ? 2 * (e / 64) : 2 * (e % (BN / 2));
-      const int ml = q * 64 + srow;
-      const int m = m0 + ml, n = n0 + pc;
+      if (ITEMS % NT != 0 && e >= ITEMS) break;
+      const int srow = EPI == GV_RELU2 ? e % 64 : e / (BN / 8);
+      const int pc = 8 * (EPI == GV_RELU2 ? e / 64 : e % (BN / 8));
+      const int ml = q * 64 + srow, m = m0 + ml, n = n0 + pc;
       const bool live = m < M;
-      float v0 = stage[srow * SSTR + pc], v1 = stage[srow * SSTR + pc + 1];
-      if (a.part) {  // raw partial; the reduce kernel applies norm and epilogue
-        if (live)
-          *reinterpret_cast<float2*>(a.part + ((int64_t)kz * M + m) * a.N + n) = make_float2(v0, v1);
-        continue;
-      }
+      const float4 lo = *reinterpret_cast<const float4*>(stage + srow * SSTR + pc);
+      const float4 hi = *reinterpret_cast<const float4*>(stage + srow * SSTR + pc + 4);
+      float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
       if (a.norm) {
-        v0 *= sinv[ml];
-        v1 *= sinv[ml];
+        const float sc = sinv[ml];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] *= sc;
       }
-      if (EPI == GV_QKV) {
-        if (live) qkv_pair_epilogue<P16>(a, m, pos0, n, v0, v1);
-      } else if (EPI == GV_RESID) {
-        float2 o = make_float2(0.f, 0.f);
-        float* y = a.y + (int64_t)(live ? m : 0) * a.N + n;
+      if (EPI == GV_RESID) {
+        const float4 x0 = xres[q * EPT + k][0], x1 = xres[q * EPT + k][1];
+        const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        float sq = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          v[i] = x[i] + v[i];
+          sq += v[i] * v[i];
+        }
         if (live) {
-          o = xres[q * EPT + k];
-          o.x += v0;
-          o.y += v1;
-          store_v<NT_RESID>(reinterpret_cast<f32x2_t*>(y), f32x2_t{o.x, o.y});
-          f16_guard<P16>(a, o.x);
-          f16_guard<P16>(a, o.y);
-          put2<P16, NT_RESID>(o.x, o.y, a.ys + (int64_t)m * a.N + n, a.ys_plane);
+          f32x4_t* y = reinterpret_cast<f32x4_t*>(a.y + (int64_t)m * a.N + n);
+          store_v<NT_RESID>(y, f32x4_t{v[0], v[1], v[2], v[3]});
+          store_v<NT_RESID>(y + 1, f32x4_t{v[4], v[5], v[6], v[7]});
+#pragma unroll
+          for (int i = 0; i < 8; ++i) f16_guard<P16>(a, v[i]);
+          put8<P16, NT_RESID>(v, a.ys + tile_at(m, n, a.N), a.ys_plane);
         }
-        // the row's sum of squares over this tile
-        const float sq0 = o.x * o.x + o.y * o.y;
-        if constexpr (SQ_LDS) {
-          sqs[srow * SQS + pc / 2] = sq0;
-        } else {
-          const float sq = BN == 128 ? wave_sum(sq0) : half_sum(sq0);
-          if (live && pc == 0) a.ssq_out[(int64_t)m * (a.N / BN) + n0 / BN] = sq;
-        }
+        sqs[srow * SQS + pc / 8] = sq;
       } else if (EPI == GV_RELU2) {
-        if (live) {
-          const float t0 = v0 < 0.f ? 0.f : v0, t1 = v1 < 0.f ? 0.f : v1;
-          f16_guard<P16>(a, t0 * t0);
-          f16_guard<P16>(a, t1 * t1);
-          put2<P16, NT_RELU2>(t0 * t0, t1 * t1, a.ys + (int64_t)m * a.N + n, a.ys_plane);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float t = v[i] < 0.f ? 0.f : v[i];
+          v[i] = t * t;
+          if (live) f16_guard<P16>(a, v[i]);
         }
-      } else {
-        if (live) *reinterpret_cast<float2*>(a.y + (int64_t)m * a.N + n) = make_float2(v0, v1);
+        if (live) put8<P16, NT_RELU2>(v, a.ys + tile_at(m, n, a.N), a.ys_plane);
+      } else if (live) {
+        float4* y = reinterpret_cast<float4*>(a.y + (int64_t)m * a.N + n);
+        y[0] = make_float4(v[0], v[1], v[2], v[3]);
+        y[1] = make_float4(v[4], v[5], v[6], v[7]);
       }
     }
     __syncthreads();
-    if constexpr (SQ_LDS) {
-      // P = NT / 64 adjacent threads per row, each summing BN / 2 / P of
-      // its values in column order, then a fixed butterfly over the P
-      constexpr int P = NT / 64, VPP = (BN / 2) / P;
-      static_assert(P * VPP == BN / 2 && (P == 2 || P == 4 || P == 8), "row-sum split");
-      const int row = tid / P, part = tid % P;
-      float sum = 0.f;
+    if constexpr (EPI == GV_RESID) {
+      // four adjacent threads per row, each summing BN / 32 of its items in
+      // column order, then a fixed butterfly
+      constexpr int VPP = BN / 32;
+      static_assert(NT >= 256 && VPP * 32 == BN, "row-sum split");
+      if (tid < 256) {
+        const int row = tid >> 2, part = tid & 3;
+        float sum = 0.f;
 #pragma unroll
-      for (int v = 0; v < VPP; ++v) sum += sqs[row * SQS + part * VPP + v];
-      sum += dpp_f<0xB1>(sum);                          // lane ^ 1
-      if constexpr (P >= 4) sum += dpp_f<0x4E>(sum);    // lane ^ 2
-      if constexpr (P == 8) sum += dpp_f<0x141>(sum);   // the other quad of eight
-      if (!a.part && part == 0 && m0 + q * 64 + row < M)
-        a.ssq_out[(int64_t)(m0 + q * 64 + row) * (a.N / BN) + n0 / BN] = sum;
+        for (int v = 0; v < VPP; ++v) sum += sqs[row * SQS + part * VPP + v];
+        sum += dpp_f<0xB1>(sum);  // lane ^ 1
+        sum += dpp_f<0x4E>(sum);  // lane ^ 2
+        if (part == 0 && m0 + q * 64 + row < M)
+          a.ssq_out[(int64_t)(m0 + q * 64 + row) * (a.N / BN) + n0 / BN] = sum;
+      }
       __syncthreads();
     }
   }
@@ -457,17 +445,19 @@ __global__ __launch_bounds__(64 * NWM * NWN * KG) void k_gemm(GemvArgs a,
 // operand fragments of the next 16-deep step are read from LDS into a
 // second register set while the MFMAs of the current one run (the last
 // step of a slice runs after the next slice's barrier), so LDS latency hides
-// behind MFMA work
-// even at one wavefront per SIMD. The epilogue works straight from the
-// accumulators: lane l of a 32x32 block holds column l % 32 of rows
-// 8(r/4) + 4(l/32) + r%4, r = 0..15, so 32 lanes store 32 consecutive
-// columns of one row.
+// behind MFMA work even at one wavefront per SIMD. The epilogue works
+// straight from the accumulators, whose lane l holds column l % 32 of rows
+// 8(r/4) + 4(l/32) + r%4, r = 0..15, of a 32x32 block: for the logits (STORE)
+// 32 lanes write 32 consecutive columns of one row. For RELU2 the product is
+// formed transposed (the same sums), so a lane holds 16 columns of one token
+// row, and the two halves of a wavefront fill 16-byte chunks of the output
+// tiles, 16 rows next to each other.
 template <int WM, int WN>
 struct Frag {
   bf16x8_t h[WM], l[WM], w[WN];
 };
 
-template <int BM, int WM, int WN, bool P16, int BK = 32>
+template <int BM, int WM, int WN, bool P16, int RT>
 __device__ __forceinline__ void frag_load(Frag<WM, WN>& f, const uint8_t* stg, int kk, int wm,
                                           int wn, int lane) {
   constexpr int AP = P16 ? 1 : 2;
@@ -475,40 +465,45 @@ __device__ __forceinline__ void frag_load(Frag<WM, WN>& f, const uint8_t* stg, i
 #pragma unroll
   for (int i = 0; i < WM; ++i) {
     const int r = (wm * WM + i) * 32 + (lane & 31);
-    f.h[i] = *(const bf16x8_t*)(stg + r * (2 * BK) + swz<BK>(r, c) * 16);
-    if constexpr (!P16) f.l[i] = *(const bf16x8_t*)(stg + (BM + r) * (2 * BK) + swz<BK>(BM + r, c) * 16);
+    f.h[i] = *(const bf16x8_t*)(stg + at<RT>(r, c));
+    if constexpr (!P16) f.l[i] = *(const bf16x8_t*)(stg + at<RT>(BM + r, c));
   }
 #pragma unroll
   for (int j = 0; j < WN; ++j) {
     const int r = AP * BM + (wn * WN + j) * 32 + (lane & 31);
-    f.w[j] = *(const bf16x8_t*)(stg + r * (2 * BK) + swz<BK>(r, c) * 16);
+    f.w[j] = *(const bf16x8_t*)(stg + at<RT>(r, c));
   }
 }
 
-template <int WM, int WN, bool P16>
+// TR: the transposed product (W rows down, token rows across).
+template <int WM, int WN, bool P16, bool TR>
 __device__ __forceinline__ void frag_mma(const Frag<WM, WN>& f, f32x16_t (&acc)[WM][WN]) {
 #pragma unroll
   for (int i = 0; i < WM; ++i)
 #pragma unroll
-    for (int j = 0; j < WN; ++j) acc[i][j] = mma16<P16>(f.h[i], f.w[j], acc[i][j]);
+    for (int j = 0; j < WN; ++j)
+      acc[i][j] = TR ? mma16<P16>(f.w[j], f.h[i], acc[i][j]) : mma16<P16>(f.h[i], f.w[j], acc[i][j]);
   if constexpr (!P16) {
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
-      for (int j = 0; j < WN; ++j) acc[i][j] = mma16<false>(f.l[i], f.w[j], acc[i][j]);
+      for (int j = 0; j < WN; ++j)
+        acc[i][j] = TR ? mma16<false>(f.w[j], f.l[i], acc[i][j])
+                       : mma16<false>(f.l[i], f.w[j], acc[i][j]);
   }
 }
 
 template <int EPI, int NWM, int NWN, int WM, int WN, int NST, bool P16 = false, int BK = 32>
 __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm2(GemvArgs a,
                                                          const int32_t* __restrict__ d_pos) {
-  constexpr int RB = 2 * BK, CPR = BK / 8, RPG = 1024 / RB;
+  static_assert(EPI == GV_RELU2 || EPI == GV_STORE, "register epilogues");
+  constexpr bool TR = EPI == GV_RELU2;
   constexpr int BM = NWM * WM * 32, BN = NWN * WN * 32;
   constexpr int NW = NWM * NWN, NT = 64 * NW;
   constexpr int AP = P16 ? 1 : 2;
-  constexpr int ROWS = AP * BM + BN, GROUPS = ROWS / RPG, GPW = GROUPS / NW;
+  constexpr int ROWS = AP * BM + BN, RT = ROWS / 16, GROUPS = RT * (BK / 32), GPW = GROUPS / NW;
   static_assert(GROUPS % NW == 0, "tile / wave grid mismatch");
-  constexpr int STAGE_BYTES = ROWS * RB;
+  constexpr int STAGE_BYTES = GROUPS * 1024;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   __shared__ float sinv[BM];
 
@@ -524,16 +519,16 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm2(GemvArgs a,
   const uint16_t* src[GPW];
 #pragma unroll
   for (int q = 0; q < GPW; ++q) {
-    const int g = wid + NW * q;
-    const int r = RPG * g + lane / CPR, slot = lane % CPR;
-    const int c = swz<BK>(r, slot);
-    if (r < AP * BM) {
-      const int ar = r < BM ? r : r - BM;
-      const int row = min(m0 + ar, M - 1);  // rows past M are never stored
-      src[q] = a.xs + (r < BM ? 0 : a.xs_plane) + (int64_t)row * K + c * 8;
+    const int g = wid + NW * q, rt = g % RT, kt = g / RT;
+    const uint16_t* base;
+    if (rt < AP * (BM / 16)) {
+      const int ar = rt < BM / 16 ? rt : rt - BM / 16;
+      base = a.xs + (rt < BM / 16 ? 0 : a.xs_plane) +
+             (int64_t)min((m0 >> 4) + ar, (M - 1) >> 4) * K * 16;
     } else {
-      src[q] = a.w + (int64_t)(n0 + r - AP * BM) * K + c * 8;
+      base = a.w + (int64_t)((n0 >> 4) + rt - AP * (BM / 16)) * K * 16;
     }
+    src[q] = base + kt * 512 + lane * 8;
   }
 
   f32x16_t acc[WM][WN];
@@ -548,7 +543,7 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm2(GemvArgs a,
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_off(smem) + wid * 1024);
   auto fill = [&](int stg, int k0) {
 #pragma unroll
-    for (int q = 0; q < GPW; ++q) dma16(src[q] + k0, lds0 + stg * STAGE_BYTES + NW * q * 1024);
+    for (int q = 0; q < GPW; ++q) dma16(src[q] + k0 * 16, lds0 + stg * STAGE_BYTES + NW * q * 1024);
   };
 #pragma unroll
   for (int si = 0; si < NST - 1; ++si) fill(si, min(si * BK, klast));
@@ -560,21 +555,21 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm2(GemvArgs a,
         stage_sync<(NST - 2) * GPW>();
         fill((si + NST - 1) % NST, min((kt + si + NST - 1) * BK, klast));
         const uint8_t* stg = smem + si * STAGE_BYTES;
-        frag_load<BM, WM, WN, P16, BK>(f0, stg, 0, wm, wn, lane);
-        if (kt + si > 0) frag_mma<WM, WN, P16>(f1, acc);  // last k-step of the previous slice
-        frag_load<BM, WM, WN, P16, BK>(f1, stg, 1, wm, wn, lane);
-        frag_mma<WM, WN, P16>(f0, acc);
+        frag_load<BM, WM, WN, P16, RT>(f0, stg, 0, wm, wn, lane);
+        if (kt + si > 0) frag_mma<WM, WN, P16, TR>(f1, acc);  // last k-step of the previous slice
+        frag_load<BM, WM, WN, P16, RT>(f1, stg, 1, wm, wn, lane);
+        frag_mma<WM, WN, P16, TR>(f0, acc);
 #pragma unroll
         for (int kk = 2; kk < BK / 16; kk += 2) {
-          frag_load<BM, WM, WN, P16, BK>(f0, stg, kk, wm, wn, lane);
-          frag_mma<WM, WN, P16>(f1, acc);
-          frag_load<BM, WM, WN, P16, BK>(f1, stg, kk + 1, wm, wn, lane);
-          frag_mma<WM, WN, P16>(f0, acc);
+          frag_load<BM, WM, WN, P16, RT>(f0, stg, kk, wm, wn, lane);
+          frag_mma<WM, WN, P16, TR>(f1, acc);
+          frag_load<BM, WM, WN, P16, RT>(f1, stg, kk + 1, wm, wn, lane);
+          frag_mma<WM, WN, P16, TR>(f0, acc);
         }
       }
     }
   }
-  frag_mma<WM, WN, P16>(f1, acc);
+  frag_mma<WM, WN, P16, TR>(f1, acc);
   wait_vmcnt<0>();
 
   if (a.norm) {
@@ -587,71 +582,42 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm2(GemvArgs a,
     __syncthreads();
   }
 
-  const int pos0 = d_pos ? *d_pos : a.pos0;
   const int half = lane >> 5, cl = lane & 31;
+  if constexpr (TR) {
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+      const int ml = (wm * WM + i) * 32 + cl, m = m0 + ml;
+      if (m >= M) continue;
+      const float sc = (a.norm ? sinv[ml] : 1.f) * (P16 ? a.wscale : 1.f);  // (wscale: a power of 2)
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq) {
+          const int n = n0 + (wn * WN + j) * 32 + 8 * rq + 4 * half;
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float u = acc[i][j][4 * rq + e] * sc, t = u < 0.f ? 0.f : u;
+            v[e] = t * t;
+            f16_guard<P16>(a, v[e]);
+          }
+          put4<P16>(v, a.ys + tile_at(m, n, a.N), a.ys_plane);
+        }
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < WM; ++i) {
     const int rb = (wm * WM + i) * 32 + 4 * half;  // tile row of r = 0
-    float ssq[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) ssq[r] = 0.f;
 #pragma unroll
     for (int j = 0; j < WN; ++j) {
-      const int cb = n0 + (wn * WN + j) * 32, n = cb + cl;
-      float v[16];
+      const int n = n0 + (wn * WN + j) * 32 + cl;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int rl = rb + 8 * (r >> 2) + (r & 3);
+        const int rl = rb + 8 * (r >> 2) + (r & 3), m = m0 + rl;
         const float u = P16 ? acc[i][j][r] * a.wscale : acc[i][j][r];
-        v[r] = a.norm ? u * sinv[rl] : u;
-      }
-      if (EPI == GV_QKV) {
-        const bool vblock = cb >= (a.H + a.KH) * a.hd;  // a 32-column block never straddles
-#pragma unroll
-        for (int rq = 0; rq < 4; ++rq) {
-          const int m = m0 + rb + 8 * rq;  // rows m .. m+3
-          const int t = m % a.T;
-          const int pos = pos0 + t;
-          if (vblock && a.vt && !a.vc && m + 3 < M && t + 3 < a.T && (pos & 3) == 0) {
-            // four consecutive positions of one dim: one 8-byte store per plane
-            const int base = n - (a.H + a.KH) * a.hd;
-            const int head = base / a.hd, j2 = (base % a.hd) >> 1;
-            const int dim = (n & 1) ? j2 + a.hd / 2 : j2;
-            const int b = m / a.T;
-            uint16_t* p = a.vt + (((int64_t)b * a.KH + head) * a.hd + dim) * a.npos + pos;
-            const float w4[4] = {v[4 * rq], v[4 * rq + 1], v[4 * rq + 2], v[4 * rq + 3]};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) f16_guard<P16>(a, w4[e]);
-            put4<P16>(w4, p, a.kv_plane);
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float own = v[4 * rq + e];
-              const float other = __shfl_xor(own, 1, 64);
-              if (m + e < M) qkv_elem_epilogue<P16>(a, m + e, pos0, n, own, other);
-            }
-          }
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = m0 + rb + 8 * (r >> 2) + (r & 3);
-          if (m >= M) continue;
-          const int64_t o = (int64_t)m * a.N + n;
-          if (EPI == GV_RESID) {
-            const float x = a.y[o] + v[r];
-            a.y[o] = x;
-            f16_guard<P16>(a, x);
-            put1<P16>(x, a.ys + o, a.ys_plane);
-            ssq[r] += x * x;
-          } else if (EPI == GV_RELU2) {
-            const float t = v[r] < 0.f ? 0.f : v[r];
-            f16_guard<P16>(a, t * t);
-            put1<P16>(t * t, a.ys + o, a.ys_plane);
-          } else {
-            __builtin_nontemporal_store(v[r], a.y + o);  // logits: read once, later
-          }
-        }
+        if (m < M)  // logits: read once, later
+          __builtin_nontemporal_store(a.norm ? u * sinv[rl] : u, a.y + (int64_t)m * a.N + n);
       }
     }
     if constexpr (EPI == GV_STORE) {
@@ -696,18 +662,6 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm2(GemvArgs a,
         }
       }
     }
-    if (EPI == GV_RESID) {
-      // per-row partial over this wavefront's WN*32 columns
-      const int nparts = a.N / (WN * 32), part = (n0 + wn * WN * 32) / (WN * 32);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float sq = ssq[r];
-#pragma unroll
-        for (int off = 16; off > 0; off >>= 1) sq += __shfl_xor(sq, off, 64);
-        const int m = m0 + rb + 8 * (r >> 2) + (r & 3);
-        if (cl == 0 && m < M) a.ssq_out[(int64_t)m * nparts + part] = sq;
-      }
-    }
   }
 }
 
@@ -725,10 +679,9 @@ void launch_cfg2(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
 
 template <int EPI, int BM, int BN, int NWM, int NWN, int BK, int NST, int KG, bool P16>
 void launch_cfg(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
-  constexpr bool sq_lds = EPI == GV_RESID && BN != 64 && BN != 128;
   constexpr size_t pipe = (size_t)NST * ((P16 ? 1 : 2) * BM + BN) * 2 * BK;
   constexpr size_t epi =
-      (size_t)KG * 64 * (BN + 4) * 4 + (sq_lds ? (size_t)64 * (BN / 2 + 1) * 4 : 0);
+      (size_t)KG * 64 * (BN + 4) * 4 + (EPI == GV_RESID ? (size_t)64 * (BN / 8 + 1) * 4 : 0);
   constexpr size_t lds = pipe > epi ? pipe : epi;
   // gfx950: 160 KB of LDS per workgroup, the row scales (BM floats) included
   static_assert(lds + BM * sizeof(float) <= 160 * 1024, "tile exceeds the LDS");
@@ -766,101 +719,11 @@ bool resid_160(int64_t M, int N, int K) {
          2 * t160 > ncu;
 }
 
-// Small M (batched decode, short chunks): too few output tiles to fill the
-// chip, so K is split over blockIdx.z as well: 64x64 tiles, enough splits
-// for ~256 blocks, each split a whole number of 32-wide slices.
-constexpr int64_t SPLITK_MAX_M = 128;
-
-int splitk_count(int64_t M, int N, int K) {
-  if (M > SPLITK_MAX_M || N % 64 != 0) return 1;
-  const int nb = (int)((M + 63) / 64) * (N / 64), nsl = K / 32;
-  int sp = (256 + nb - 1) / nb;
-  if (sp > nsl) sp = nsl;
-  while (sp > 1 && nsl % sp != 0) --sp;
-  return sp;
-}
-
-// Sum of the K-split partials in split order, then the row norm and the
-// epilogue. Block = (row, 512 columns), a thread a column pair; the splits'
-// loads go out eight at a time. RESID leaves one sum-of-squares partial per
-// row and 512-column group.
-constexpr int RED_COLS = 512;
-
-template <int EPI>
-__global__ __launch_bounds__(256) void k_splitk_reduce(GemvArgs a, int splits,
-                                                       const int32_t* __restrict__ d_pos) {
-  __shared__ float red[4];
-  const int m = blockIdx.x, tid = threadIdx.x, N = a.N;
-  const int n = blockIdx.y * RED_COLS + 2 * tid;
-  float inv = 1.f;
-  if (a.norm) {
-    float ssum = 0.f;
-    for (int t = 0; t < a.ssq_n; ++t) ssum += a.ssq_in[(int64_t)m * a.ssq_n + t];
-    inv = 1.0f / sqrtf(ssum / (float)a.K + a.eps);
-  }
-  const int pos0 = d_pos ? *d_pos : a.pos0;
-  float sq = 0.f;
-  if (n < N) {
-    float v0 = 0.f, v1 = 0.f;
-    const float* P = a.part + (int64_t)m * N + n;
-    const int64_t stride = (int64_t)a.M * N;
-    for (int s0 = 0; s0 < splits; s0 += 8) {
-      float2 p[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        p[k] = s0 + k < splits ? *reinterpret_cast<const float2*>(P + (s0 + k) * stride)
-                               : make_float2(0.f, 0.f);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {  // split order (a zero adds nothing)
-        v0 += p[k].x;
-        v1 += p[k].y;
-      }
-    }
-    v0 *= inv;
-    v1 *= inv;
-    const int64_t o = (int64_t)m * N + n;
-    if (EPI == GV_QKV) {
-      qkv_pair_epilogue(a, m, pos0, n, v0, v1);
-    } else if (EPI == GV_RESID) {
-      float2 x = *reinterpret_cast<const float2*>(a.y + o);
-      x.x += v0;
-      x.y += v1;
-      *reinterpret_cast<float2*>(a.y + o) = x;
-      if (a.ys) split_bf16x2(x.x, x.y, a.ys + o, a.ys_plane);
-      sq = x.x * x.x + x.y * x.y;
-    } else if (EPI == GV_RELU2) {
-      const float t0 = v0 < 0.f ? 0.f : v0, t1 = v1 < 0.f ? 0.f : v1;
-      split_bf16x2(t0 * t0, t1 * t1, a.ys + o, a.ys_plane);
-    } else {
-      *reinterpret_cast<float2*>(a.y + o) = make_float2(v0, v1);
-    }
-  }
-  if (EPI == GV_RESID && a.ssq_out) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) sq += __shfl_xor(sq, off, 64);
-    if ((tid & 63) == 0) red[tid >> 6] = sq;
-    __syncthreads();
-    if (tid == 0)
-      a.ssq_out[(int64_t)m * gridDim.y + blockIdx.y] = red[0] + red[1] + red[2] + red[3];
-  }
-}
-
-// The K-split partial sums of a small-M GEMM into a.part (64x64 tiles,
-// blockIdx.z the split).
-template <int EPI>
-void launch_splitk_parts(hipStream_t s, const GemvArgs& a, int sp, const int32_t* d_pos) {
-  constexpr size_t lds = (size_t)4 * (2 * 64 + 64) * 64;
-  const dim3 g(a.N / 64, (unsigned)((a.M + 63) / 64), (unsigned)sp);
-  FG_LAUNCH((k_gemm<EPI, 64, 64, 2, 2, 32, 4>), g, dim3(256), lds, s, a, d_pos);
-}
-
 // Tile choice. The LDS-staged epilogue (k_gemm) serves QKV and RESID,
 // whose outputs are scattered or need per-row reductions; the register
 // epilogue (k_gemm2) serves the plain stores of RELU2 and lm_head, with
 // 128x256 tiles (wave 64x128) when there are >= 1.5 blocks per CU.
 
-// The single-term fp16 kernels (a.f16) serve passes of more than
-// SPLITK_MAX_M rows only, so they never split K.
 template <int EPI, bool P16>
 void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
   if constexpr (P16 && (EPI == GV_RELU2 || EPI == GV_STORE)) {
@@ -871,9 +734,7 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
     // barriers per K: 0.8 % of the 8 x 2048 eval forward (identical bits; at
     // 2048 rows the 128x256 tiles are 1.5 % slower with them)
     if (a.M > 4096 && a.N % 256 == 0) {
-      GemvArgs b = a;
-      b.part = nullptr;
-      launch_cfg2<EPI, 2, 4, 4, 2, 2, P16, 64>(s, b, d_pos);
+      launch_cfg2<EPI, 2, 4, 4, 2, 2, P16, 64>(s, a, d_pos);
       return;
     }
   }
@@ -881,21 +742,10 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
     // lm_head with the cross-entropy's partials: a register-epilogue tiling
     // (the only one that writes them; gemm_store_nll guarantees the shape)
     if (a.nll_part) {
-      GemvArgs b = a;
-      b.part = nullptr;
-      launch_cfg2<EPI, 2, 2, 2, 4, 2, P16>(s, b, d_pos);
+      launch_cfg2<EPI, 2, 2, 2, 4, 2, P16>(s, a, d_pos);
       return;
     }
   }
-  const int sp = a.part && !P16 ? splitk_count(a.M, a.N, a.K) : 1;
-  if (sp > 1) {
-    launch_splitk_parts<EPI>(s, a, sp, d_pos);
-    const dim3 rg((unsigned)a.M, (unsigned)((a.N + RED_COLS - 1) / RED_COLS));
-    FG_LAUNCH((k_splitk_reduce<EPI>), rg, dim3(256), 0, s, a, sp, d_pos);
-    return;
-  }
-  GemvArgs b = a;
-  b.part = nullptr;  // the kernels below write the epilogue themselves
   const int64_t mt128 = (a.M + 127) / 128;
   // fc at prefill sizes: where 128x128 tiles spill into a second, mostly
   // empty round over the CUs, 128x192 tiles fit in one (QKV stays on
@@ -904,27 +754,28 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
     const int64_t ncu = cu_count();
     if (a.N % 192 == 0 && a.K % 64 == 0 && mt128 * (a.N / 128) > ncu &&
         mt128 * (a.N / 192) <= ncu) {
-      launch_cfg<EPI, 128, 192, 4, 2, 64, 2, 1, P16>(s, b, d_pos);
+      launch_cfg<EPI, 128, 192, 4, 2, 64, 2, 1, P16>(s, a, d_pos);
       return;
     }
   }
-  if (a.N % 256 == 0 && ((EPI == GV_STORE && mt128 * (a.N / 256) >= 384) ||
-                         (EPI == GV_RELU2 && mt128 * (a.N / 256) >= 768))) {
-    launch_cfg2<EPI, 2, 2, 2, 4, 2, P16>(s, b, d_pos);
-    return;
-  }
   const bool big = a.N % 128 == 0 && mt128 * (a.N / 128) >= 256;
-  if (big && (EPI == GV_RELU2 || EPI == GV_STORE)) {
-    launch_cfg2<EPI, 4, 2, 1, 2, 3, P16>(s, b, d_pos);
-    return;
+  if constexpr (EPI == GV_RELU2 || EPI == GV_STORE) {
+    if (a.N % 256 == 0 && mt128 * (a.N / 256) >= (EPI == GV_STORE ? 384 : 768)) {
+      launch_cfg2<EPI, 2, 2, 2, 4, 2, P16>(s, a, d_pos);
+      return;
+    }
+    if (big) {
+      launch_cfg2<EPI, 4, 2, 1, 2, 3, P16>(s, a, d_pos);
+      return;
+    }
   }
   if constexpr (EPI == GV_RESID) {
     if (resid_k4(a.M, a.N, a.K)) {
-      launch_cfg<EPI, 64, 96, 2, 1, 64, 3, 4, P16>(s, b, d_pos);
+      launch_cfg<EPI, 64, 96, 2, 1, 64, 3, 4, P16>(s, a, d_pos);
       return;
     }
     if (resid_160(a.M, a.N, a.K)) {
-      launch_cfg<EPI, 64, 160, 2, 1, 64, 3, 2, P16>(s, b, d_pos);
+      launch_cfg<EPI, 64, 160, 2, 1, 64, 3, 2, P16>(s, a, d_pos);
       return;
     }
   }
@@ -934,7 +785,7 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
     // two (the depth-20 model at 2047 rows: 224 tiles against 448)
     const int64_t ncu = cu_count(), t128 = mt128 * (a.N / 128);
     if (bn == 128 && !big && t128 <= ncu && 2 * t128 > ncu) {
-      launch_cfg<EPI, 128, 128, 4, 2, 32, 3, 1, P16>(s, b, d_pos);
+      launch_cfg<EPI, 128, 128, 4, 2, 32, 3, 1, P16>(s, a, d_pos);
       return;
     }
   }
@@ -943,22 +794,26 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
     // tiles: 64-wide K slices, two stages (64 KB with one fp16 A plane):
     // 1-3 % of the GEMM time faster than 32-wide ones over 8 x 2048 rows,
     // and the depth-12 forward 0.9 % (1 x 2048) to 1.2 % (2 x 2048) faster
-    launch_cfg<EPI, 128, 128, 4, 2, 64, 2, 1, P16>(s, b, d_pos);
+    launch_cfg<EPI, 128, 128, 4, 2, 64, 2, 1, P16>(s, a, d_pos);
   else if (bn == 128 && big)
-    launch_cfg<EPI, 128, 128, 4, 2, 32, 3, 1, P16>(s, b, d_pos);  // 72 KB: two blocks per CU
+    launch_cfg<EPI, 128, 128, 4, 2, 32, 3, 1, P16>(s, a, d_pos);  // 72 KB: two blocks per CU
   else if (bn == 128 && EPI == GV_RESID && a.K % 64 == 0)
     // the residual GEMMs (proj, proj2) inside the layer stack: 64-wide slices
     // (half the stage hand-overs) measured ~4 us a launch faster than 32-wide
     // ones at any depth
-    launch_cfg<EPI, 64, 128, 2, 2, 64, 3, 1, P16>(s, b, d_pos);
+    launch_cfg<EPI, 64, 128, 2, 2, 64, 3, 1, P16>(s, a, d_pos);
   else if (bn == 128)
-    launch_cfg<EPI, 64, 128, 2, 2, 32, 4, 1, P16>(s, b, d_pos);
+    launch_cfg<EPI, 64, 128, 2, 2, 32, 4, 1, P16>(s, a, d_pos);
   else
-    launch_cfg<EPI, 64, 64, 2, 2, 32, 4, 1, P16>(s, b, d_pos);
+    launch_cfg<EPI, 64, 64, 2, 2, 32, 4, 1, P16>(s, a, d_pos);
 }
 
 template <int EPI>
 void launch_tile(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
+  if (gemm_rows_tile(a.M, a.N).tm > 0) {  // few token rows
+    launch_gemm_rows(s, (GemvEpi)EPI, a, d_pos);
+    return;
+  }
   if (a.f16)
     launch_tile_p<EPI, true>(s, a, d_pos);
   else
@@ -989,17 +844,12 @@ int cu_count() {
 // hold 64 rows a lane and the epilogue's reductions cost more than the pass.
 bool gemm_store_nll(int64_t M, int N) { return M > 1024 && M <= 4096 && N % 256 == 0; }
 
-// RESID on k_gemm: one sum-of-squares partial per row and N tile; split-K
-// RESID (given split-K scratch): one per row and 512 columns.
+// RESID: one sum-of-squares partial per row and N tile.
 int gemm_ssq_parts(int64_t M, int N, int K) {
-  if (splitk_count(M, N, K) == 1 && resid_k4(M, N, K)) return N / 96;
-  if (splitk_count(M, N, K) == 1 && resid_160(M, N, K)) return N / 160;
-  return splitk_count(M, N, K) > 1 ? (N + RED_COLS - 1) / RED_COLS : N / tile_n(M, N);
-}
-
-int64_t gemm_splitk_floats(int64_t M, int N, int K) {
-  const int sp = splitk_count(M, N, K);
-  return sp > 1 ? (int64_t)sp * M * N : 0;
+  if (const RowsTile t = gemm_rows_tile(M, N); t.tm > 0) return N / (16 * t.tn);
+  if (resid_k4(M, N, K)) return N / 96;
+  if (resid_160(M, N, K)) return N / 160;
+  return N / tile_n(M, N);
 }
 
 void launch_gemm_pos(hipStream_t s, GemvEpi epi, const GemvArgs& a, const int32_t* d_pos) {
@@ -1009,18 +859,6 @@ void launch_gemm_pos(hipStream_t s, GemvEpi epi, const GemvArgs& a, const int32_
     case GV_RELU2: launch_tile<GV_RELU2>(s, a, d_pos); break;
     default: launch_tile<GV_STORE>(s, a, d_pos); break;
   }
-}
-
-int launch_gemm_partials(hipStream_t s, GemvEpi epi, const GemvArgs& a, const int32_t* d_pos) {
-  const int sp = a.part && !a.f16 ? splitk_count(a.M, a.N, a.K) : 1;
-  if (sp <= 1) return 0;
-  switch (epi) {  // (the kernel writes raw partials whatever the epilogue)
-    case GV_QKV: launch_splitk_parts<GV_QKV>(s, a, sp, d_pos); break;
-    case GV_RESID: launch_splitk_parts<GV_RESID>(s, a, sp, d_pos); break;
-    case GV_RELU2: launch_splitk_parts<GV_RELU2>(s, a, sp, d_pos); break;
-    default: launch_splitk_parts<GV_STORE>(s, a, sp, d_pos); break;
-  }
-  return sp;
 }
 
 void launch_gemm(hipStream_t s, GemvEpi epi, const GemvArgs& a) {

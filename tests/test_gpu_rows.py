@@ -1,0 +1,65 @@
+"""The few-row MFMA GEMM (kern_rows.hip) at the edges of its tiles and of the
+row range it serves, through fg_forward and fg_step, against the CPU oracle.
+
+Rows 5..256 run on it (fewer on the GEMV, more on the LDS-tiled GEMM); its
+tiles are 16x16, 16x32, 32x32, 32x64 and 64x64, picked by the row count, and 8
+wavefronts split K (K = 128: four 32-deep steps, so half of them have none).
+Bounds: split operands carry 16 bits of an activation, so a logit is within a
+few 2^-16 of max|logit| (5e-5 asked); one fp16 term carries 11 (2e-3 asked).
+"""
+import numpy as np
+import pytest
+
+from autoresearch_amd import engine
+from autoresearch_amd.weights import Dims, rope_tables, seeded_weights, uniform_ids
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+TINY = Dims(n_layer=2, d_model=128, n_head=2, n_kv_head=1, head_dim=64, vocab=512)
+SMALL = Dims(n_layer=2, d_model=384, n_head=3, n_kv_head=3, head_dim=128, vocab=1024)
+# d_model / 16 = 136 sums of squares per row: more than a block's threads take in one pass
+WIDE = Dims(n_layer=1, d_model=2176, n_head=34, n_kv_head=2, head_dim=64, vocab=256)
+
+
+def model(d, maxpos):
+    w = seeded_weights(d, 11)
+    c, s = (t.reshape(-1) for t in rope_tables(maxpos, d.head_dim))
+    m = engine.Model(d, stacks=w)
+    m.set_rope(c, s)
+    return m, w, c, s
+
+
+def rel(a, b):
+    return float(np.abs(a - b).max() / np.abs(b).max())
+
+
+@pytest.mark.parametrize("d,B,T", [
+    (TINY, 1, 5), (TINY, 1, 16), (TINY, 1, 17), (TINY, 3, 21), (TINY, 1, 256), (TINY, 1, 257),
+    (SMALL, 1, 15), (SMALL, 2, 32), (SMALL, 1, 65), (SMALL, 1, 128), (SMALL, 1, 129),
+    (SMALL, 3, 85), (WIDE, 1, 9), (WIDE, 1, 40)])
+def test_forward_rows(d, B, T):
+    m, w, c, s = model(d, T)
+    ids = uniform_ids(21 + T, B * T, d.vocab)
+    ref = O.gpt_forward(ids, c, s, w, d, B, T)
+    lg, _ = m.forward(ids, B, T)
+    assert rel(lg, ref) <= 5e-5
+    m.set_forward_f16(True)
+    lg16, _ = m.forward(ids, B, T)
+    assert rel(lg16, ref) <= (2e-3 if B * T > 128 else 5e-5)
+    m.close()
+
+
+@pytest.mark.parametrize("B", [5, 16, 17, 40, 70])
+def test_step_rows(B):
+    d, P = SMALL, 6
+    m, w, c, s = model(d, P + 1)
+    ids = uniform_ids(31 + B, B * (P + 1), d.vocab).reshape(B, P + 1)
+    kv = m.kv(B, P + 1)
+    kv.step_multi(ids[:, :P], want_logits=False)
+    lg, nxt = kv.step(ids[:, P])
+    ref = O.gpt_forward(ids.reshape(-1), c, s, w, d, B, P + 1).reshape(B, P + 1, -1)[:, P]
+    assert rel(lg, ref) <= 5e-5
+    assert np.array_equal(nxt, lg.argmax(axis=1))
+    kv.close()
+    m.close()
