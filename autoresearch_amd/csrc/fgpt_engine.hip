@@ -424,7 +424,7 @@ int32_t upload_weights(fg_model* m, const float* const st[8]) {
 void free_work(fg_model* m) {
   Work& ws = m->ws;
   void* ptrs[] = {ws.x, ws.q, ws.ao, ws.h, ws.logits, ws.ids, ws.tgt, ws.nll, ws.stat, ws.amax,
-                  ws.xs, ws.aos, ws.hs, ws.ssq, ws.nllp, m->qs};
+                  ws.xs, ws.aos, ws.hs, ws.fkv, ws.ssq, ws.nllp, m->qs};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   ws = Work();
@@ -575,6 +575,7 @@ int32_t ensure_work(fg_model* m, int64_t rows) {
   RCCHK(alloc((void**)&ws.xs, prow * d.D * 2 * 2));
   RCCHK(alloc((void**)&ws.aos, prow * d.qd() * 2 * 2));
   RCCHK(alloc((void**)&ws.hs, prow * d.dff * 2 * 2));
+  RCCHK(alloc((void**)&ws.fkv, std::min(rows, attn_rows_most(d)) * d.kvd() * 2 * 4));
   RCCHK(alloc((void**)&ws.ssq, rows * (d.D / 16) * 4));
   if (d.V % 256 == 0) RCCHK(alloc((void**)&ws.nllp, rows * (d.V / NLL_GROUP_COLS) * 2 * 4));
   HIPCHK(hipStreamSynchronize(m->stream));  // the clears, before any caller stream's work
@@ -626,6 +627,18 @@ int npos_pad(int n) { return (n + 63) / 64 * 64; }
 // that every linear of the pass runs on the MFMA GEMM with split operands.
 bool use_gemm(const Dims& d, int64_t rows) {
   return rows > 4 || rows * (int64_t)d.dff * 4 > 65536;
+}
+
+// The single-term fp16 pass: MFMA GEMMs of more than 128 rows.
+bool pass_f16(const fg_model* m, int64_t rows, bool on) {
+  return on && use_gemm(m->d, rows) && rows > 128 && m->w16;
+}
+
+// Whether the chunk attention of a pass reads cache rows (launch_attn_rows)
+// rather than split planes. The single-term fp16 pass keeps its fp16 planes
+// (no faster from rows: 150 rows 389 us either way, 600 835 -> 845).
+bool chunk_few(const Dims& d, bool kv16, int B, int T, int pos0, bool f16) {
+  return !f16 && attn_rows_fits(d, kv16, B, T, pos0);
 }
 
 // y = epi(x W^T) on the path chosen for the pass. Algorithmic traffic:
@@ -686,8 +699,7 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
   Work& ws = ws_in ? *ws_in : m->ws;
   const int rows = B * T;
   const bool gm = !o.rows_single && use_gemm(d, rows);
-  // the single-term fp16 pass: MFMA GEMMs of more than 128 rows (no split K)
-  const bool f16 = o.f16 && gm && rows > 128 && m->w16;
+  const bool f16 = !o.rows_single && pass_f16(m, rows, o.f16);
   // the GEMMs' weights: the operand-layout copies; the GEMV's: row-major
   auto W = [&](const bf16_t* p) {
     return !gm ? p : (f16 ? m->w16 : m->wt) + (p - m->w.base);
@@ -703,7 +715,10 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
   const int64_t qplane = (int64_t)rows * d.qd();
   // ssq partials per row after the attention-output RESID
   const int nt_resid = gemm_ssq_parts(rows, d.D, d.qd());
-  const int64_t pos_items = o.pos_cnt ? attn_items(d, B, T, pos0) : 0;
+  // chunk attention from the cache rows instead of split planes
+  const bool few = chunk_few(d, o.kv16, B, T, pos0, f16) &&
+                   !((T == 1 || o.rows_single) && kc != nullptr);
+  const int64_t pos_items = o.pos_cnt ? attn_items(d, B, T, pos0, few) : 0;
 
   if (embed)  // (else x already holds the embedded rows)
     timed(m, s, FG_K_OTHER, 0, (double)rows * d.D * (gm ? 10 : 6), [&] {
@@ -729,7 +744,11 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
     // (and, for a chunk, written as bf16 hi/lo planes for the MFMA attention)
     const bool one = (T == 1 || o.rows_single) && lk != nullptr;
     const int npos = npos_pad(pos0 + T);
-    if (!one) {
+    if (few && !kc) {  // (gpt_forward: the layer's keys and values in scratch rows)
+      a.kc = ws.fkv;
+      a.vc = ws.fkv + (int64_t)rows * d.kvd();
+    }
+    if (!one && !few) {
       a.qs = m->qs;
       a.q_plane = qplane;
       a.ks = m->ks;
@@ -751,6 +770,11 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
         launch_attn_decode_pos(s, d, ws.q, lk, lv, o.kv16, B, maxT, d_pos, pos0 + 1, dec_part,
                                o.dec_cnt, ws.ao, aos,
                                aplane, T, o.d_rows);
+      });
+    } else if (few) {
+      timed(m, s, FG_K_ATTN_CHUNK, at_flops, at_bytes, [&] {
+        launch_attn_rows(s, d, ws.q, a.kc, a.vc, o.kv16, B, T, pos0, maxT, ws.ao, aos, aplane,
+                         o.pos_cnt ? o.pos_cnt + l * pos_items : nullptr);
       });
     } else {
       if (pos0 > 0)  // earlier cache positions enter the chunk's key planes
@@ -991,7 +1015,8 @@ int32_t forward_host(fg_model* m, const int32_t* ids, int32_t B, int32_t T, floa
   GUARD(m);
   RCCHK(ensure_work(m, rows));
   hipStream_t s = m->stream;
-  const int64_t items = npos ? attn_items(m->d, B, T, 0) : 0;
+  const bool few = chunk_few(m->d, false, B, T, 0, pass_f16(m, rows, m->fwd_f16));
+  const int64_t items = npos ? attn_items(m->d, B, T, 0, few) : 0;
   if (npos && items * m->d.L > m->pos_cap) {
     RCCHK(quiesce(m));
     if (m->d_pos) HIPCHK(hipFree(m->d_pos));
@@ -1260,7 +1285,7 @@ int32_t kv_pass(fg_model* m, fg_kv* kv, const int32_t* h_ids, int TB, float* log
   RCCHK(check_rope(m, kv->len + TB));
   const int64_t rows = (int64_t)B * TB;
   RCCHK(ensure_work(m, rows));
-  if (TB > 1) {
+  if (TB > 1 && !chunk_few(m->d, kv->kv16, B, TB, kv->len, false)) {
     RCCHK(ensure_split(m, (int64_t)B * npos_pad(kv->len + TB) * m->d.kvd()));
     RCCHK(ensure_attn(m, B, TB, kv->len));
   }

@@ -106,6 +106,9 @@ struct Work {
   uint16_t* xs = nullptr;   // residual [rows][D]
   uint16_t* aos = nullptr;  // attention output [rows][H*hd]
   uint16_t* hs = nullptr;   // relu2(fc) [rows][4D]
+  // one layer's key, then value rows [rows][KH*hd] of a forward without a
+  // cache that attends from rows (attn_rows_fits)
+  float* fkv = nullptr;
   float* ssq = nullptr;
   float* nllp = nullptr;    // lm_head's log-sum-exp partials [rows][V/NLL_GROUP_COLS][2]
 };
@@ -229,14 +232,22 @@ inline void raise_lds_once(const void* fn, size_t bytes, std::atomic<uint64_t>* 
   (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
   if (bit) done->fetch_or(bit, std::memory_order_release);
 }
-// pos_cnt (nullable): one count per work item, attn_items(d, B, T, pos0) of
-// them, item i belonging to (sequence * H + head) = i % (B * H): how many of
+// pos_cnt (nullable): one count per work item, attn_items(d, B, T, pos0,
+// rows) of them (rows: launch_attn_rows), item i belonging to (sequence * H + head) = i % (B * H): how many of
 // the item's causal scores q.k are > 0 (src/lib/fortran_attn.f90:247-300).
-int64_t attn_items(const Dims& d, int B, int T, int pos0);
+int64_t attn_items(const Dims& d, int B, int T, int pos0, bool rows);
 void launch_attn_mfma(hipStream_t s, const Dims& d, const uint16_t* qs, const uint16_t* ks,
                       const uint16_t* vt, int B, int T, int npos, int pos0, int64_t q_plane,
                       int64_t kv_plane, float* scratch, float* y, uint16_t* ys = nullptr,
                       int64_t ys_plane = 0, bool f16 = false, uint32_t* pos_cnt = nullptr);
+// The same attention for few query blocks (attn_rows_fits), from the rotated
+// queries q [B*T][H*hd] and the cache rows themselves ([B][maxT][KH*hd], fp32
+// or bf16 with kv16): no planes, no scratch, no merge launch.
+bool attn_rows_fits(const Dims& d, bool kv16, int B, int T, int pos0);
+int64_t attn_rows_most(const Dims& d);  // the most token rows it holds for (fp32 rows)
+void launch_attn_rows(hipStream_t s, const Dims& d, const float* q, const void* kc, const void* vc,
+                      bool kv16, int B, int T, int pos0, int maxT, float* y, uint16_t* ys,
+                      int64_t ys_plane, uint32_t* pos_cnt = nullptr);
 // Fill the hi/lo key/value planes for cache positions [0, n) from the cache
 // of one layer ([B][maxT][KH*hd], fp32, or bf16 with kv16: lo planes zero).
 void launch_split_cache(hipStream_t s, const Dims& d, const void* kc, const void* vc, bool kv16,

@@ -435,6 +435,273 @@ __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs p) {
   store_out<HD, P16>(p, (int64_t)b * p.T + tt, h * HD + d, v);
 }
 
+// ------------------------------------------------------------ few queries
+// The same attention for passes whose query blocks cannot fill the chip (a
+// prompt chunk, a short prefill). There the kernel above runs on a handful of
+// workgroups, each walking its keys in a serial chain of LDS stages, after a
+// launch of its own has split the cached keys and values into planes. Here a
+// workgroup takes 16 queries of one head and its 8 wavefronts every eighth
+// 32-key tile each, so a chain is an eighth as long; keys and values come
+// straight from the cache rows (fp32, split into bf16 hi + lo in registers, or
+// bf16) to MFMA operands, nothing is staged and no planes are needed. The
+// wavefronts' partial (O, max, sum) meet in LDS in wavefront order.
+//
+// v_mfma_f32_16x16x32_bf16 with S^T = K Q^T: lane l = 16 g + c holds query c
+// of keys 4g .. 4g+3 of both 16-key blocks of its tile, which are taken as
+// the 8 K slots of its B operand in O^T = V^T P^T; which head dims a lane's K
+// slots and rows of that product stand for is chosen so that its pieces of the
+// K and V rows are whole 16-byte loads (RowsTileKV).
+// Bound by that chain, 6 us a round of 8 tiles from an fp32 cache (the split's
+// arithmetic), 3 from a bf16 one; attn_rows_fits has the measurements.
+struct AttnRowsArgs {
+  const float* q;  // [B*T][H*HD], rotated
+  const void* kc;  // [B][maxT][KH*HD]
+  const void* vc;
+  int H, KH, T, pos0, maxT, nbh, nqb;
+  float* y;
+  uint16_t* ys;
+  int64_t ys_plane;
+  uint32_t* pos_cnt;  // as in AttnArgs
+};
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// One 32-key tile's raw K and V pieces of a lane, and their operand forms.
+// fp32 rows: a lane's 8 dims of K step s are 32 s + 4 g .. + 3 and 32 s + 16 +
+// 4 g .. + 3, its dims of a V row 64 i + 4 c .. + 3, so that the lanes of one
+// load instruction read 64 (K) or 256 (V) consecutive bytes of a row.
+template <int HD, class KT>
+struct RowsTileKV;
+template <int HD>
+struct RowsTileKV<HD, float> {
+  static constexpr int NS = HD / 32, VD = HD / 16, DK = 16, DG = 4;  // K piece stride, lane step
+  static constexpr bool LO = true;
+  static __device__ __forceinline__ int vdim(int c, int i) { return 64 * (i / 4) + 4 * c; }
+  float4 k[2][NS][2], v[8][VD / 4];
+  __device__ __forceinline__ void load_k(int kb, const float* row, int g) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      k[kb][s][0] = *(const float4*)(row + 32 * s + DG * g);
+      k[kb][s][1] = *(const float4*)(row + 32 * s + DG * g + DK);
+    }
+  }
+  __device__ __forceinline__ void load_v(int e, const float* row, int c) {
+#pragma unroll
+    for (int i = 0; i < VD / 4; ++i) v[e][i] = *(const float4*)(row + vdim(c, 4 * i));
+  }
+  __device__ __forceinline__ void kop(int kb, int s, bf16x8_t& h, bf16x8_t& l) const {
+    const float4 a = k[kb][s][0], b = k[kb][s][1];
+    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    split8(x, h, l);
+  }
+  __device__ __forceinline__ void vop(int i, bf16x8_t& h, bf16x8_t& l) const {
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float4 t = v[e][i / 4];
+      x[e] = i % 4 == 0 ? t.x : i % 4 == 1 ? t.y : i % 4 == 2 ? t.z : t.w;
+    }
+    split8(x, h, l);
+  }
+};
+template <int HD>
+struct RowsTileKV<HD, uint16_t> {
+  static constexpr int NS = HD / 32, VD = HD / 16, DK = 4, DG = 8;
+  static __device__ __forceinline__ int vdim(int c, int i) { return VD * c + i; }
+  static constexpr bool LO = false;  // (the cache's elements are exact in one term)
+  typedef uint16_t vrow_t __attribute__((ext_vector_type(VD)));
+  uint4 k[2][NS];
+  vrow_t v[8];
+  __device__ __forceinline__ void load_k(int kb, const uint16_t* row, int g) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) k[kb][s] = *(const uint4*)(row + 32 * s + 8 * g);
+  }
+  __device__ __forceinline__ void load_v(int e, const uint16_t* row, int c) {
+    v[e] = *(const vrow_t*)(row + VD * c);
+  }
+  __device__ __forceinline__ void kop(int kb, int s, bf16x8_t& h, bf16x8_t&) const {
+    h = __builtin_bit_cast(bf16x8_t, k[kb][s]);
+  }
+  __device__ __forceinline__ void vop(int i, bf16x8_t& h, bf16x8_t&) const {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) h[e] = __builtin_bit_cast(__bf16, (uint16_t)v[e][i]);
+  }
+};
+
+constexpr int RQ = 16, RWV = 8;  // queries and wavefronts of a workgroup
+
+template <int HD>
+constexpr int attn_rows_lds() { return (RWV * RQ * (HD + 4) + RWV * RQ * 2) * 4; }
+
+template <int HD, class KT>
+__global__ __launch_bounds__(64 * RWV) void k_attn_rows(AttnRowsArgs p) {
+  typedef RowsTileKV<HD, KT> TileKV;
+  constexpr int NS = TileKV::NS, VD = TileKV::VD, OST = HD + 4;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+  float* xo = reinterpret_cast<float*>(lds);  // [RWV][RQ][OST]
+  float* ml = xo + RWV * RQ * OST;            // [RWV][RQ] (max, sum)
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int bh = blockIdx.x % p.nbh, j = p.nqb - 1 - blockIdx.x / p.nbh;  // longest chains first
+  const int b = bh / p.H, h = bh % p.H, kvh = h / (p.H / p.KH);
+  const int t0 = j * RQ, tq = min(t0 + c, p.T - 1);  // (queries past T: the last one, not stored)
+  const int klim = p.pos0 + tq + 1;                  // keys below this are visible
+  const int kend = p.pos0 + min(t0 + RQ, p.T);       // to any query of the block
+  const int ntile = (kend + 31) / 32;
+  const int64_t kd = (int64_t)p.KH * HD;
+  const KT* kc = (const KT*)p.kc + (int64_t)b * p.maxT * kd + kvh * HD;
+  const KT* vc = (const KT*)p.vc + (int64_t)b * p.maxT * kd + kvh * HD;
+
+  TileKV kv;
+  // (keys past kend read the last row; they are masked)
+  auto load_k = [&](int tile) {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+      kv.load_k(kb, kc + min(32 * tile + 16 * kb + c, kend - 1) * kd, g);
+  };
+  auto load_v = [&](int tile) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      kv.load_v(e, vc + min(32 * tile + 16 * (e >> 2) + 4 * g + (e & 3), kend - 1) * kd, c);
+  };
+  if (wv < ntile) {
+    load_k(wv);
+    load_v(wv);
+  }
+  bf16x8_t qh[NS], ql[NS];
+  {
+    const float* qp = p.q + ((int64_t)b * p.T + tq) * p.H * HD + h * HD + TileKV::DG * g;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const float4 a = *(const float4*)(qp + 32 * s);
+      const float4 d = *(const float4*)(qp + 32 * s + TileKV::DK);
+      const float x[8] = {a.x, a.y, a.z, a.w, d.x, d.y, d.z, d.w};
+      split8(x, qh[s], ql[s]);
+    }
+  }
+  f32x4_t o[VD];
+#pragma unroll
+  for (int i = 0; i < VD; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m_run = -FLT_MAX, l_run = 0.f;  // log2 domain; l_run: this lane's keys
+  uint32_t npos = 0;  // this lane's positive causal scores (p.pos_cnt)
+  __shared__ float wpos[RWV];
+  const float cs = LOG2E / sqrtf((float)HD);
+  auto mma = [](const bf16x8_t& a, const bf16x8_t& x, const f32x4_t& acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, x, acc, 0, 0, 0);
+  };
+
+  for (int tile = wv; tile < ntile; tile += RWV) {
+    const int nx = min(tile + RWV, ntile - 1);  // (past the end: loaded, unused)
+    f32x4_t sc[2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      sc[kb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        bf16x8_t ah, al;
+        kv.kop(kb, s, ah, al);
+        sc[kb] = mma(ah, qh[s], sc[kb]);
+        if constexpr (TileKV::LO) sc[kb] = mma(al, qh[s], sc[kb]);
+        sc[kb] = mma(ah, ql[s], sc[kb]);
+      }
+    }
+    load_k(nx);
+    if (32 * tile + 31 > p.pos0 + t0) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          sc[kb][r] = 32 * tile + 16 * kb + 4 * g + r < klim ? sc[kb][r] : -INFINITY;
+    }
+    if (p.pos_cnt && t0 + c < p.T) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) npos += sc[e >> 2][e & 3] > 0.f ? 1u : 0u;
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, sc[e >> 2][e & 3]);
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * cs;
+    if (__any(mx > m_run + 8.f)) {  // (the lazy rescale of k_attn_mfma)
+      const float m_new = fmaxf(m_run, mx);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      l_run *= alpha;
+#pragma unroll
+      for (int i = 0; i < VD; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[i][r] *= alpha;
+      m_run = m_new;
+    }
+    float pv[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      pv[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[e >> 2][e & 3], cs, -m_run));
+      l_run += pv[e];
+    }
+    bf16x8_t ph, pl;
+    split8(pv, ph, pl);
+#pragma unroll
+    for (int i = 0; i < VD; ++i) {
+      bf16x8_t ah, al;
+      kv.vop(i, ah, al);
+      o[i] = mma(ah, ph, o[i]);
+      if constexpr (TileKV::LO) o[i] = mma(al, ph, o[i]);
+      o[i] = mma(ah, pl, o[i]);
+    }
+    load_v(nx);
+  }
+
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+  float* xr = xo + (wv * RQ + c) * OST;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int i = 0; i < VD; i += 4)
+      *(float4*)(xr + TileKV::vdim(4 * g + r, i)) =
+          make_float4(o[i][r], o[i + 1][r], o[i + 2][r], o[i + 3][r]);
+  if (g == 0) *(float2*)(ml + 2 * (wv * RQ + c)) = make_float2(m_run, l_run);
+  if (p.pos_cnt) {  // (a wavefront's count is below 2^24: its float sum is exact)
+    const float wc = wave_sum((float)npos);
+    if (lane == 0) wpos[wv] = wc;
+  }
+  __syncthreads();
+  if (p.pos_cnt && tid == 0) {
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < RWV; ++w) t += wpos[w];
+    p.pos_cnt[blockIdx.x] = (uint32_t)t;
+  }
+  const int qq = tid / (HD / 4), d = 4 * (tid % (HD / 4)), t = t0 + qq;
+  if (qq >= RQ || t >= p.T) return;
+  float2 w[RWV];
+  float m = -FLT_MAX, l = 0.f;
+#pragma unroll
+  for (int k = 0; k < RWV; ++k) {
+    w[k] = *(const float2*)(ml + 2 * (k * RQ + qq));
+    m = fmaxf(m, w[k].x);
+  }
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int k = 0; k < RWV; ++k) {
+    const float e = exp2f(w[k].x - m);
+    const float4 v = *(const float4*)(xo + (k * RQ + qq) * OST + d);
+    l += e * w[k].y;
+    acc.x += e * v.x;
+    acc.y += e * v.y;
+    acc.z += e * v.z;
+    acc.w += e * v.w;
+  }
+  const float inv = 1.0f / l;
+  const float v[4] = {acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv};
+  const int64_t row = (int64_t)b * p.T + t;
+  if (p.ys)
+    put4<false>(v, p.ys + tile_at(row, h * HD + d, p.H * HD), p.ys_plane);
+  else
+    *(float4*)(p.y + row * p.H * HD + h * HD + d) = make_float4(v[0], v[1], v[2], v[3]);
+}
+
 // Cache positions [0, n) of one layer, [B][maxT][KH*hd] -> hi/lo planes
 // (a bf16 cache: hi = the element, lo = 0).
 __device__ __forceinline__ float cache_elem(const float* c, int64_t i) { return c[i]; }
@@ -487,8 +754,9 @@ int attn_chunk_keys(int BH, int T, int pos0) {
   return best;
 }
 
-int64_t attn_items(const Dims& d, int B, int T, int pos0) {
+int64_t attn_items(const Dims& d, int B, int T, int pos0, bool rows) {
   const int nbh = B * d.H;
+  if (rows) return (int64_t)nbh * ((T + RQ - 1) / RQ);
   return (int64_t)nbh * attn_items_per_head(T, pos0, attn_chunk_keys(nbh, T, pos0));
 }
 
@@ -555,6 +823,53 @@ void launch_attn_mfma(hipStream_t s, const Dims& d, const uint16_t* qs, const ui
   } else {
     if (f16) launch_attn_hd<64, true>(s, p, grid, split);
     else launch_attn_hd<64, false>(s, p, grid, split);
+  }
+}
+
+// Where a pass attends from cache rows. Its chain grows with the keys, and past
+// one workgroup a CU with the workgroups, faster than k_attn_mfma's; against
+// that stands what the other way costs before it starts (the split of the
+// cached positions, on all KV heads; QKV's plane stores) and after (the merge
+// of split key ranges). Whole passes, us, planes -> rows:
+//   fp32 cache, 6 heads of their own K/V: 16 queries after 500 positions 662
+//   -> 480, after 2000 1031 -> 1004; 256 after 1500 1193 -> 1017; 512 after
+//   1500 1506 -> 1346; 1024 (384 workgroups) after 0 1381 -> 1301, after 1000
+//   1653 -> 1755; forwards of 150 486 -> 426, 1000 1205 -> 1202, 1365 (516)
+//   1378 -> 1527
+//   fp32, 10 heads on 2 KV heads (K/V rows split five times over): 128 after
+//   1000 1694 -> 1563, after 1900 1780 -> 1904; 512 (320) after 0 2525 -> 2315,
+//   after 512 2684 -> 2752
+//   bf16 cache (no split at all): 64 after 1900 984 -> 604 and, on 2 KV heads,
+//   1493 -> 1291; 1024 (640) after 0 3338 -> 3228; 1365 (860) 3771 -> 3804
+// Key counts above those measured stay on the kernel that spreads them.
+constexpr int64_t ROWS_MAX_WG = 512, ROWS_MAX_WG16 = 640;
+bool attn_rows_fits(const Dims& d, bool kv16, int B, int T, int pos0) {
+  const int64_t wg = (int64_t)B * d.H * ((T + RQ - 1) / RQ);
+  if (kv16) return wg <= ROWS_MAX_WG16 && pos0 + T <= 2560;
+  const int keys = d.H == d.KH ? 2560 : 1200;
+  return wg <= ROWS_MAX_WG && pos0 + T <= (wg > cu_count() ? keys / 2 : keys);
+}
+int64_t attn_rows_most(const Dims& d) { return ROWS_MAX_WG / d.H * RQ; }
+
+template <int HD, class KT>
+static void launch_attn_rows_t(hipStream_t s, const AttnRowsArgs& p) {
+  constexpr int lds = attn_rows_lds<HD>();
+  static std::atomic<uint64_t> lds_set{0};
+  raise_lds_once((const void*)k_attn_rows<HD, KT>, lds, &lds_set);
+  FG_LAUNCH((k_attn_rows<HD, KT>), dim3((unsigned)(p.nbh * p.nqb)), dim3(64 * RWV), lds, s, p);
+}
+
+void launch_attn_rows(hipStream_t s, const Dims& d, const float* q, const void* kc, const void* vc,
+                      bool kv16, int B, int T, int pos0, int maxT, float* y, uint16_t* ys,
+                      int64_t ys_plane, uint32_t* pos_cnt) {
+  const AttnRowsArgs p{q, kc, vc, d.H,      d.KH,   T, pos0, maxT, B * d.H, (T + RQ - 1) / RQ,
+                       y, ys, ys_plane, pos_cnt};
+  if (d.hd == 128) {
+    if (kv16) launch_attn_rows_t<128, uint16_t>(s, p);
+    else launch_attn_rows_t<128, float>(s, p);
+  } else {
+    if (kv16) launch_attn_rows_t<64, uint16_t>(s, p);
+    else launch_attn_rows_t<64, float>(s, p);
   }
 }
 

@@ -63,3 +63,26 @@ def test_step_rows(B):
     assert np.array_equal(nxt, lg.argmax(axis=1))
     kv.close()
     m.close()
+
+
+@pytest.mark.parametrize("d", [TINY, SMALL])
+@pytest.mark.parametrize("B,pos,T", [
+    (1, 0, 2), (1, 0, 16), (1, 0, 17), (2, 15, 2), (1, 16, 16), (1, 31, 33), (3, 32, 5),
+    (1, 255, 2), (1, 256, 16), (1, 257, 47), (2, 300, 20)])
+def test_chunk_attention_rows(d, B, pos, T):
+    """Chunks attended from the cache rows (k_attn_rows) at the edges of its
+    16-query blocks, 32-key tiles and 8-tile rounds. bf16 caches round K and V
+    to 8 bits (2^-9 of each at most; asked 4e-3 of max|logit|)."""
+    n = pos + T
+    m, w, c, s = model(d, n)
+    ids = uniform_ids(41 + n, B * n, d.vocab).reshape(B, n)
+    ref = O.gpt_forward(ids.reshape(-1), c, s, w, d, B, n).reshape(B, n, -1)[:, pos:]
+    for kv16, tol in ((False, 5e-5), (True, 4e-3)):
+        kv = m.kv(B, n + 3, bf16=kv16)
+        if pos:
+            kv.step_multi(ids[:, :pos], want_logits=False)
+        lg, nxt = kv.step_multi(ids[:, pos:])
+        assert rel(lg, ref) <= tol
+        assert np.array_equal(nxt, lg[:, -1].argmax(axis=1))
+        kv.close()
+    m.close()
