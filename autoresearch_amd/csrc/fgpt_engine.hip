@@ -670,6 +670,9 @@ struct PassOpts {
   int pos_host = -1;      // host value of the first position (timing model), -1: pos0
   bool embed = true;      // false: x already holds the embedded rows
   bool rows_single = false;  // every row as a single cached step (see layer_stack)
+  // chunk over a cache: only the last row of each sequence goes past the last
+  // layer's keys and values; logits takes B rows
+  bool last_only = false;
   const int32_t* d_rows = nullptr;  // rows_single: rows live, read on the device
   bool kv16 = false;      // the cache holds bf16 elements
   bool f16 = false;       // single-term fp16 MFMA pass where the MFMA path runs (> 128 rows)
@@ -697,8 +700,9 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
                  Work* ws_in = nullptr) {
   const Dims& d = m->d;
   Work& ws = ws_in ? *ws_in : m->ws;
-  const int rows = B * T;
-  const bool gm = !o.rows_single && use_gemm(d, rows);
+  int rows = B * T;
+  bool gm = !o.rows_single && use_gemm(d, rows);
+  float* x = ws.x;
   const bool f16 = !o.rows_single && pass_f16(m, rows, o.f16);
   // the GEMMs' weights: the operand-layout copies; the GEMV's: row-major
   auto W = [&](const bf16_t* p) {
@@ -710,11 +714,11 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
   const double pairs = (double)T * pos_host + 0.5 * (double)T * (T + 1);
   const double at_flops = 4.0 * d.hd * d.H * B * pairs;
   const double at_bytes = (double)B * (2.0 * T * d.qd() + 2.0 * (pos_host + T) * d.kvd()) * 4;
-  const int64_t prow = tile_rows(rows);
-  const int64_t xplane = prow * d.D, aplane = prow * d.qd(), hplane = prow * d.dff;
+  int64_t prow = tile_rows(rows);
+  int64_t xplane = prow * d.D, aplane = prow * d.qd(), hplane = prow * d.dff;
   const int64_t qplane = (int64_t)rows * d.qd();
   // ssq partials per row after the attention-output RESID
-  const int nt_resid = gemm_ssq_parts(rows, d.D, d.qd());
+  int nt_resid = gemm_ssq_parts(rows, d.D, d.qd());
   // chunk attention from the cache rows instead of split planes
   const bool few = chunk_few(d, o.kv16, B, T, pos0, f16) &&
                    !((T == 1 || o.rows_single) && kc != nullptr);
@@ -743,12 +747,13 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
     // q, k, v = rmsnorm(x) Wqkv^T, RoPE on q and k, k/v appended to the cache
     // (and, for a chunk, written as bf16 hi/lo planes for the MFMA attention)
     const bool one = (T == 1 || o.rows_single) && lk != nullptr;
+    const bool last = o.last_only && l == d.L - 1;  // (queries: one row a sequence, from q)
     const int npos = npos_pad(pos0 + T);
     if (few && !kc) {  // (gpt_forward: the layer's keys and values in scratch rows)
       a.kc = ws.fkv;
       a.vc = ws.fkv + (int64_t)rows * d.kvd();
     }
-    if (!one && !few) {
+    if (!one && !few && !last) {
       a.qs = m->qs;
       a.q_plane = qplane;
       a.ks = m->ks;
@@ -756,7 +761,7 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
       a.npos = npos;
       a.kv_plane = (int64_t)B * npos * d.kvd();
     }
-    a.x = ws.x; a.xs = ws.xs; a.xs_plane = xplane; a.ssq_in = ws.ssq; a.ssq_n = nt;
+    a.x = x; a.xs = ws.xs; a.xs_plane = xplane; a.ssq_in = ws.ssq; a.ssq_n = nt;
     a.f16 = f16 ? 1 : 0;
     a.ovf = f16 ? m->d_ovf : nullptr;
     a.wscale = m->w16_inv;
@@ -764,8 +769,35 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
     linear(m, s, GV_QKV, a, d_pos, gm);
     a.qs = nullptr;
     a.ks = a.vt = nullptr;
+    const float* q = ws.q;
+    if (last) {  // go on with the last row of each sequence
+      const int64_t qd = d.qd();
+      if (B == 1) {
+        x += (int64_t)(T - 1) * d.D;
+        q += (int64_t)(T - 1) * qd;
+      } else {  // (h past the B rows that fc writes: dff >= qd + D)
+        float* p = ws.h + (int64_t)B * d.dff;
+        launch_last_rows(s, ws.q, p, (int)qd, ws.x, p + B * qd, d.D, B, T);
+        q = p;
+        x = p + B * qd;
+      }
+      rows = a.M = B;
+      a.T = 1;
+      gm = use_gemm(d, rows);
+      prow = tile_rows(rows);
+      xplane = prow * d.D;
+      aplane = prow * qd;
+      hplane = prow * d.dff;
+      nt_resid = gemm_ssq_parts(rows, d.D, d.qd());
+    }
     uint16_t* aos = gm ? ws.aos : nullptr;
-    if (one) {
+    if (last) {
+      timed(m, s, FG_K_ATTN_DECODE, 4.0 * d.hd * d.H * B * (pos_host + T),
+            (double)B * (2.0 * d.qd() + 2.0 * (pos_host + T) * d.kvd()) * 4, [&] {
+        launch_attn_decode_pos(s, d, q, lk, lv, o.kv16, B, maxT, nullptr, pos0 + T, dec_part,
+                               o.dec_cnt, ws.ao, aos, aplane);
+      });
+    } else if (one) {
       timed(m, s, FG_K_ATTN_DECODE, at_flops, at_bytes, [&] {
         launch_attn_decode_pos(s, d, ws.q, lk, lv, o.kv16, B, maxT, d_pos, pos0 + 1, dec_part,
                                o.dec_cnt, ws.ao, aos,
@@ -791,25 +823,25 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
     }
     // x += attn_out Wproj^T (GEMM path: also the split x and its row sums)
     a.x = ws.ao; a.xs = ws.aos; a.xs_plane = aplane; a.ssq_n = 0;
-    a.w = W(m->w.proj(l)); a.N = d.D; a.K = d.qd(); a.norm = 0; a.y = ws.x;
+    a.w = W(m->w.proj(l)); a.N = d.D; a.K = d.qd(); a.norm = 0; a.y = x;
     a.ys = ws.xs; a.ys_plane = xplane; a.ssq_out = ws.ssq;
     linear(m, s, GV_RESID, a, d_pos, gm);
     nt = nt_resid;
     // h = relu(rmsnorm(x) Wfc^T)^2
-    a.x = ws.x; a.xs = ws.xs; a.xs_plane = xplane; a.ssq_in = ws.ssq; a.ssq_n = nt;
+    a.x = x; a.xs = ws.xs; a.xs_plane = xplane; a.ssq_in = ws.ssq; a.ssq_n = nt;
     a.w = W(m->w.fc(l)); a.N = d.dff; a.K = d.D; a.norm = 1; a.y = ws.h;
     a.ys = ws.hs; a.ys_plane = hplane; a.ssq_out = nullptr;
     linear(m, s, GV_RELU2, a, d_pos, gm);
     // x += h Wproj2^T
     a.x = ws.h; a.xs = ws.hs; a.xs_plane = hplane; a.ssq_n = 0;
-    a.w = W(m->w.proj2(l)); a.N = d.D; a.K = d.dff; a.norm = 0; a.y = ws.x;
+    a.w = W(m->w.proj2(l)); a.N = d.D; a.K = d.dff; a.norm = 0; a.y = x;
     a.ys = ws.xs; a.ys_plane = xplane; a.ssq_out = ws.ssq;
     linear(m, s, GV_RESID, a, d_pos, gm);
     nt = gemm_ssq_parts(rows, d.D, d.dff);
   }
   GemvArgs a = base_args(m, ws);
   a.M = rows; a.T = T; a.d_M = o.d_rows;
-  a.x = ws.x; a.xs = ws.xs; a.xs_plane = xplane; a.ssq_in = ws.ssq; a.ssq_n = nt;
+  a.x = x; a.xs = ws.xs; a.xs_plane = xplane; a.ssq_in = ws.ssq; a.ssq_n = nt;
   a.f16 = f16 ? 1 : 0;
   a.ovf = f16 ? m->d_ovf : nullptr;
   a.wscale = m->w16_inv;
@@ -1296,10 +1328,12 @@ int32_t kv_pass(fg_model* m, fg_kv* kv, const int32_t* h_ids, int TB, float* log
   PassOpts o;
   o.kv16 = kv->kv16;
   o.dec_cnt = kv->d_dcnt;
+  // a prompt chunk: nobody reads its rows' logits but the last one's argmax
+  o.last_only = TB > 1 && !logits && (B == 1 || m->d.dff >= m->d.qd() + m->d.D);
   layer_stack(m, s, m->ws.ids, B, TB, kv->len, nullptr, kv->k, kv->v, kv->maxT, lstride,
               kv->d_part, m->ws.logits, o);
   HIPCHK(hipGetLastError());
-  if (next_ids && TB == 1) {
+  if (next_ids && (TB == 1 || o.last_only)) {
     launch_argmax(s, m->ws.logits, B, m->d.V, m->ws.amax);
     HIPCHK(hipMemcpyAsync(next_ids, m->ws.amax, (size_t)B * 4, hipMemcpyDeviceToHost, s));
   } else if (next_ids) {

@@ -134,6 +134,10 @@ void launch_embed_norm(hipStream_t s, const Dims& d, const bf16_t* wte, const in
                        int64_t rows, float* x, uint16_t* xs = nullptr, int64_t plane = 0,
                        float* ssq = nullptr, const int32_t* d_rows = nullptr, bool f16 = false);
 
+// qo[b] = q[b * T + T - 1] (nq floats a row), xo likewise of x (nx), b < B.
+void launch_last_rows(hipStream_t s, const float* q, float* qo, int nq, const float* x, float* xo,
+                      int nx, int B, int T);
+
 // GEMV family for M <= GEMV_MAX_ROWS token rows, fp32 activations x bf16
 // weights (the MFMA GEMM shares the argument block).
 constexpr int GEMV_MAX_ROWS = 16;

@@ -115,6 +115,20 @@ void launch_to_f16(hipStream_t s, const bf16_t* src, uint16_t* dst, int64_t n, f
   FG_LAUNCH(k_to_f16, dim3((unsigned)blocks), dim3(256), 0, s, src, dst, n, scale);
 }
 
+__global__ __launch_bounds__(256) void k_last_rows(const float* __restrict__ q,
+                                                   float* __restrict__ qo, int nq,
+                                                   const float* __restrict__ x,
+                                                   float* __restrict__ xo, int nx, int T) {
+  const int64_t b = blockIdx.x, r = b * T + T - 1;
+  for (int k = threadIdx.x; k < nq; k += 256) qo[b * nq + k] = q[r * nq + k];
+  for (int k = threadIdx.x; k < nx; k += 256) xo[b * nx + k] = x[r * nx + k];
+}
+
+void launch_last_rows(hipStream_t s, const float* q, float* qo, int nq, const float* x, float* xo,
+                      int nx, int B, int T) {
+  FG_LAUNCH(k_last_rows, dim3((unsigned)B), dim3(256), 0, s, q, qo, nq, x, xo, nx, T);
+}
+
 void launch_embed_norm(hipStream_t s, const Dims& d, const bf16_t* wte, const int32_t* ids,
                        int64_t rows, float* x, uint16_t* xs, int64_t plane, float* ssq,
                        const int32_t* d_rows, bool f16) {

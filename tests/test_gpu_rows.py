@@ -86,3 +86,34 @@ def test_chunk_attention_rows(d, B, pos, T):
         assert np.array_equal(nxt, lg[:, -1].argmax(axis=1))
         kv.close()
     m.close()
+
+
+@pytest.mark.parametrize("d,B,T,pos,kv16", [
+    (TINY, 1, 2, 0, False), (TINY, 1, 40, 3, False), (SMALL, 2, 3, 0, False), (SMALL, 5, 9, 7, True),
+    (SMALL, 17, 20, 0, False), (TINY, 3, 300, 0, False)])
+def test_chunk_without_logits(d, B, T, pos, kv16):
+    """A chunk whose logits nobody takes runs its last layer and lm_head for
+    one row a sequence: the same cache bit for bit, and the id that the full
+    pass's last row has as its maximum (within the passes' 5e-5)."""
+    n = pos + T
+    m, w, c, s = model(d, n + 1)
+    ids = uniform_ids(51 + n, B * n, d.vocab).reshape(B, n)
+    full, fast = m.kv(B, n + 1, bf16=kv16), m.kv(B, n + 1, bf16=kv16)
+    for kv in (full, fast):
+        if pos:
+            kv.step_multi(ids[:, :pos])
+    lg, _ = full.step_multi(ids[:, pos:])
+    none, nxt = fast.step_multi(ids[:, pos:], want_logits=False)
+    assert none is None and fast.len == full.len == n
+    for a, b in zip(full.read(), fast.read()):
+        assert np.array_equal(a, b)
+    last = lg[:, -1]
+    best = last.max(axis=1)
+    assert np.all(best - last[np.arange(B), nxt] <= 1e-4 * np.abs(last).max())
+    # and on from there
+    a, _ = full.step(nxt)
+    b, _ = fast.step(nxt)
+    assert np.array_equal(a, b)
+    full.close()
+    fast.close()
+    m.close()
