@@ -1446,8 +1446,11 @@ bool fused_applies(const fg_model* m, const fg_kv* kv, int n_steps) {
 // n_steps positions are written in place. The launch's placement counters
 // are cleared first, and its error flag too when clear_err is set (a caller
 // running several launches clears it once and reads it after the last).
+// host_sd: draw each next id instead (the host's copy of kv->d_smp; ids_out =
+// kv->d_sids).
 int32_t fused_launch(fg_model* m, fg_kv* kv, const int32_t* d_id0, int len0, int n_steps,
-                     int32_t* ids_out, float* logits_out, bool clear_err) {
+                     int32_t* ids_out, float* logits_out, bool clear_err,
+                     const SampleDev* host_sd = nullptr) {
   hipStream_t s = m->stream;
   const uint32_t eps = fused_epochs(m->d, n_steps);
   if ((uint64_t)m->fused_ep + eps >= 0xFFFFFF00ull) {  // epochs would wrap: start over
@@ -1471,6 +1474,14 @@ int32_t fused_launch(fg_model* m, fg_kv* kv, const int32_t* d_id0, int len0, int
   a.d_id0 = d_id0;
   a.ids_out = ids_out;
   a.logits_out = logits_out;
+  a.sd = nullptr;
+  a.n_gen = 0;
+  if (host_sd) {
+    a.sd = kv->d_smp;
+    a.cfg = host_sd->cfg;
+    a.ids_out = ids_out + host_sd->n_known;
+    a.n_gen = host_sd->pp - host_sd->n_known;
+  }
   a.slots = m->fused_slots;
   a.ep_base = m->fused_ep;
   a.err = m->fused_err;
@@ -2022,7 +2033,13 @@ extern "C" int32_t fg_decode_sample(fg_model* m, fg_kv* kv, int32_t* ids, int32_
   int done = 0;
   const int total = n_total - n_known;
   const bool fused = fused_applies(m, kv, total);
-  if (fused) {
+  if (fused && m->fl.kind == 0 && !m->timing) {
+    // one launch for all the steps, the draws in it: no launch, no placement
+    // and no cold weight pipeline per id (timing brackets each step instead)
+    int32_t* inp = (int32_t*)((char*)kv->d_smp + offsetof(SampleDev, inp));
+    RCCHK(fused_launch(m, kv, inp, n_known - 1, total, kv->d_sids, nullptr, true, h));
+    done = total;
+  } else if (fused) {
     // each step the persistent kernel for one step (its logits; its own
     // argmax goes to the spare inp[1]), then the draw, which leaves the next
     // input in inp[0]; the error flag is cleared once and read at the end

@@ -427,6 +427,11 @@ struct FusedArgs {
   uint32_t* cnt;         // [8] workgroups placed per XCD so far; zeroed before
   int D, H, KH, L, V, dff;
   float eps;
+  // sampled loop (nullable; kind 0 only): its state in and out, its settings,
+  // and ids_out = the start of the history, n_gen ids of it known
+  SampleDev* sd;
+  SampleCfg cfg;
+  int n_gen;
   uint64_t* trace;       // null, or [256][L+1][32] phase timestamps of step trace_step
   int trace_step;
 };

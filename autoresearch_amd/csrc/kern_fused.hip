@@ -49,6 +49,7 @@
 #include <algorithm>
 
 #include "kern_fused.h"
+#include "kern_sample.h"
 
 namespace fgpt {
 
@@ -74,14 +75,20 @@ struct FusedShape {
   static constexpr int64_t OFF_LM = OFF_P2 + 2 * FUSED_NX * D;
   // (the argmax candidates: two step parities x FUSED_LMC copies)
   static constexpr int64_t OFF_AP = OFF_LM + 2 * FUSED_LMC * 2 * FUSED_NWG;
-  static constexpr int64_t SLOTS = OFF_AP + 2 * FUSED_NX * FUSED_SPLIT_WG * (HD + 2);
+  // (sampled loops: the row of logits and FUSED_LMC copies of the drawn id)
+  static constexpr int64_t OFF_SM = OFF_AP + 2 * FUSED_NX * FUSED_SPLIT_WG * (HD + 2);
+  static constexpr int64_t SLOTS = OFF_SM + 2 * (V + FUSED_LMC);
+  static_assert(4 * V + sample_wg_aux(V) <= WBUF, "the sampled row fits a weight buffer");
 };
 // The shapes the persistent decode is built for: depth-12's (d_model 768,
 // 6 heads, vocab 8192) and a small one the tests run.
 typedef FusedShape<768, 6, 8192> ShapeD12;
 typedef FusedShape<256, 2, 1024> ShapeSmall;
 
-template <class Sh, bool TRACE>
+// SAMPLE: the next id is drawn (a.sd) in place of the argmax: every workgroup
+// hands its logits to workgroup 0, which draws from the row (sample_wg, in the
+// weight buffer lm_head has just freed) and hands the id to all.
+template <class Sh, bool TRACE, bool SAMPLE>
 __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   constexpr int HD = Sh::HD;
@@ -168,7 +175,8 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
     }
     const int64_t nch = n / 1024, k0 = part * nch / 3, k1 = (part + 1) * nch / 3;
     for (int64_t k = off + 1024 * k0; k < off + 1024 * k1; k += 1024)
-      dma16(src + k + 16 * lane, lds_off(dst + k));
+      dma16(src + k + 16 * lane, SAMPLE ? __builtin_amdgcn_readfirstlane(lds_off(dst + k))
+                                        : lds_off(dst + k));
   };
   auto waitdma = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
 
@@ -198,6 +206,8 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
     }
   };
 
+  int64_t* rng = (int64_t*)(ired + 6);  // (SAMPLE, workgroup 0)
+  if (SAMPLE && tid == 0) *rng = a.sd->rng;
   if (loader) {
     issue(0, 0);
     issue(0, 1);
@@ -498,6 +508,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
       const uint32_t ep = a.ep_base + (uint32_t)(s * E + 8 * L);
       // argmax candidates of the 256 workgroups, [2][256][2] (value, index)
       uint64_t* LMC = S + Sh::OFF_LM + (int64_t)(s & 1) * FUSED_LMC * 2 * FUSED_NWG;
+      uint64_t* SMP = S + Sh::OFF_SM + (int64_t)(s & 1) * (V + FUSED_LMC);
       if (comp) {
         const float inv = 1.0f / sqrtf(sumsq<D>(x_lds, lane) / (float)D + eps);
         float bv = -INFINITY;
@@ -518,7 +529,11 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
           }
           const float v = multi_sum<8>(acc, scr, lane) * inv;
           const int r = r0 + 4 * (lane >> 3), id = b * LR + r;
-          if ((lane & 7) == 0 && r < LR && a.logits_out) a.logits_out[(int64_t)s * V + id] = v;
+          if (SAMPLE) {
+            if ((lane & 7) == 0 && r < LR) slot_put_dev(SMP + id, v, ep);
+          } else if ((lane & 7) == 0 && r < LR && a.logits_out) {
+            a.logits_out[(int64_t)s * V + id] = v;
+          }
           // rows in increasing order across the eight groups
 #pragma unroll
           for (int q = 0; q < 8; ++q)
@@ -532,6 +547,35 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
       }
       lds_barrier();  // B5
       if (loader && G + 1 < total) issue(G + 1, 1);
+      if (SAMPLE) {
+        if (b == 0) {
+          float* pr = (float*)(lds + (G & 1) * Sh::WBUF);
+          if (comp) {
+            constexpr int NB = V > 4096 ? 2 : 1;  // (16 slots a thread at once)
+            for (int k = 0; k < NB; ++k)
+              if (!gather_slots<V / 256 / NB>(SMP + k * (V / NB), V / NB, ep, pr + k * (V / NB), tid,
+                                              err))
+                *stop = 1;
+          }
+          lds_barrier();
+          if (!*stop) {
+            const int id = sample_wg<V>(pr, (uint8_t*)(pr + V), a.ids_out, s + a.n_gen, a.cfg, rng,
+                                        comp);
+            if (wv == 0 && lane < FUSED_LMC)
+              slot_put_dev(SMP + V + lane, __int_as_float(id), ep + 1);
+            if (tid == 0) {
+              ired[4] = id;
+              __hip_atomic_store(a.ids_out + a.n_gen + s, id, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+              asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the next draw's history)
+            }
+          }
+        } else if (wv == 0) {
+          float f;
+          if (!slots_wait<1, 0, 2>(SMP + V + b % FUSED_LMC, 0, 1, ep + 1, &f, err)) *stop = 1;
+          if (lane == 0) ired[4] = __float_as_int(f);
+        }
+      } else
       // the first-max argmax over all 256 candidates in one hand-over
       // across XCDs: every workgroup publishes its candidate (value in
       // slot b, index in slot 256 + b) into FUSED_LMC copies (lane k of
@@ -576,9 +620,16 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
       if (loader && G + 1 < total) issue(G + 1, 2);
       int id = ired[4];
       if (id == 0x7fffffff) id = 0;  // no finite candidate: position 1, as the scan starts there
-      if (b == 0 && tid == 0) a.ids_out[s] = id;
+      if (!SAMPLE && b == 0 && tid == 0) a.ids_out[s] = id;
       if (s + 1 < a.n_steps) embed(id, pos + 1);
     }
+  }
+  if (SAMPLE && b == 0 && tid == 0) {  // the loop's state after n_steps draws
+    SampleDev* sd = a.sd;
+    sd->rng = *rng;
+    sd->pp += a.n_steps;
+    sd->len += a.n_steps;
+    sd->inp[0] = ired[4];
   }
 done:
   if (loader) waitdma();  // no LDS-DMA may outlive the workgroup
@@ -634,7 +685,7 @@ FusedLayout fused_layout(const Dims& d, const char** why) {
   f.off_p2 = f.off_hl + 2 * FUSED_NX * (int64_t)f.HN;
   f.off_lm = f.off_p2 + 2 * FUSED_NX * (int64_t)d.D;
   f.off_ap = f.off_lm + 2 * FUSED_LMC * 2 * (int64_t)FUSED_NWG;
-  f.slots = f.off_ap + 2 * FUSED_NX * FUSED_SPLIT_WG * (int64_t)(d.hd + 2);
+  f.slots = f.off_ap + 2 * FUSED_NX * FUSED_SPLIT_WG * (int64_t)(d.hd + 2) + 2 * (d.V + FUSED_LMC);
   f.ok = true;
   return f;
 }
@@ -684,7 +735,9 @@ static hipError_t launch_shape(hipStream_t s, const FusedLayout& f, const FusedA
   if (f.slice != Sh::SLICE || f.lmb != Sh::LMB || f.wbuf != Sh::WBUF || f.wf != Sh::WF ||
       f.off_lm != Sh::OFF_LM || f.off_ap != Sh::OFF_AP || f.slots != Sh::SLOTS)
     return hipErrorInvalidValue;  // (host and device layouts disagree)
-  const void* k = a.trace ? (const void*)k_fused_decode<Sh, true> : (const void*)k_fused_decode<Sh, false>;
+  const void* k = a.sd      ? (const void*)k_fused_decode<Sh, false, true>
+                  : a.trace ? (const void*)k_fused_decode<Sh, true, false>
+                            : (const void*)k_fused_decode<Sh, false, false>;
   hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)f.lds_bytes);
   if (e != hipSuccess) return e;
   FusedArgs aa = a;

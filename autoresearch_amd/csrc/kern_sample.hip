@@ -19,25 +19,13 @@
 
 #include "fgpt_internal.h"
 #include "kern_common.h"
+#include "kern_sample.h"
 
 namespace fgpt {
 namespace {
 
 constexpr int ST = 1024;  // threads of a sampling workgroup
 constexpr int NW = ST / 64;
-
-// xorshift64* of rand_u01: the state advances, the top 24 bits of
-// state * 2685821657736338717 give u in [0, 1)
-__device__ float rand_u01(int64_t* st) {
-  uint64_t x = (uint64_t)*st;
-  if (x == 0) x = 2685821657736338717ull;
-  x ^= x << 13;
-  x ^= x >> 7;
-  x ^= x << 17;
-  *st = (int64_t)x;
-  const uint64_t y = x * 2685821657736338717ull;
-  return (float)((y >> 40) & 0xFFFFFFull) / 16777216.0f;
-}
 
 __device__ __forceinline__ void amax_pick(float& v, int& i, float v2, int i2) {
   if (v2 > v || (v2 == v && i2 < i)) {
@@ -115,13 +103,6 @@ __device__ void count_ids(const int32_t* gen, int lo, int hi, int V, int* cnt) {
     if (g >= 0 && g < V) atomicAdd(&cnt[g], 1);
   }
   __syncthreads();
-}
-
-// Sort keys: the probability's bits (p >= 0, so they order as p does) above,
-// 0x7fffffff - id below: descending key order is descending probability
-// with ties in ascending id; key 0 (padding past V) sorts last.
-__device__ __forceinline__ uint64_t prob_key(float p, int id) {
-  return ((uint64_t)__float_as_uint(p) << 32) | (uint32_t)(0x7fffffff - id);
 }
 
 // v of lane (lane ^ D), D a power of two below 64: DPP within quads, a

@@ -281,7 +281,8 @@ int32_t fg_decode_sample(fg_model *m, fg_kv *kv, int32_t *ids, int32_t n_known, 
 
 /* Handle options (no counterpart in the reference, which has one CPU path).
  *
- * FG_OPT_FUSED_DECODE: 1 (the default) lets fg_decode_greedy run a B=1 loop
+ * FG_OPT_FUSED_DECODE: 1 (the default) lets fg_decode_greedy (and, with one KV
+ * head per query head and timing off, fg_decode_sample) run a B=1 loop
  * on an fp32 cache as ONE persistent launch (all layers, lm_head and the
  * argmax of every step; the weights stream through LDS ahead of their use,
  * activations pass between workgroups through epoch-tagged slots), for the

@@ -210,6 +210,35 @@ def test_decode_sample_loop_persistent(d):
     m.close()
 
 
+@pytest.mark.parametrize("d", [SMALL_MHA, Dims(n_layer=1, d_model=768, n_head=6, n_kv_head=6,
+                                               head_dim=128, vocab=8192)], ids=["1k", "8k"])
+@pytest.mark.parametrize("cfg", [
+    dict(temp=0.05, topp=0.9), dict(temp=0.3, topp=0.5, rep=1.3, nblock=2),  # few ids kept
+    dict(temp=0.8, topp=0.95, pres=0.2, freq=0.1, nblock=3),
+    dict(temp=0.8, topp=0.9, pwin=5, plen=0.4, pres=0.3, freq=0.2, rep=1.2),
+    dict(temp=1.0, topp=1.0), dict(temp=50.0, topp=0.9999), dict(temp=3.0, topp=0.9),  # whole row
+    dict(temp=0.7, topp=1e-6), dict(temp=0.9, topp=0.9, byte_space=True), dict(temp=0.0, rep=1.5)])
+def test_sampling_inside_the_persistent_loop(d, cfg):
+    """One launch that draws between its steps against a launch and a
+    k_sample_step per id (what timing runs): the same logits, sums and order,
+    so the same ids and generator state, bit for bit."""
+    m = engine.Model(d, stacks=seeded_weights(d, 9))
+    prompt = uniform_ids(19, 9, d.vocab)
+    n_gen = 24
+    c, s = rope_tables(prompt.size + n_gen, d.head_dim)
+    m.set_rope(c.reshape(-1), s.reshape(-1))
+    outs = []
+    for timing in (True, False):
+        kv = m.kv(1, prompt.size + n_gen)
+        kv.step_multi(prompt[:-1], want_logits=False)
+        m.timing(timing)
+        outs.append(kv.decode_sample(prompt, n_gen, seed=1234567, **cfg))
+        m.timing(False)
+        kv.close()
+    assert np.array_equal(outs[0][0], outs[1][0]) and outs[0][1] == outs[1][1]
+    m.close()
+
+
 def test_sample_errors(m):
     with pytest.raises(engine.FgptError):
         m.sample(np.zeros(8193, np.float32))
