@@ -676,7 +676,11 @@ struct PassOpts {
   const int32_t* d_rows = nullptr;  // rows_single: rows live, read on the device
   bool kv16 = false;      // the cache holds bf16 elements
   bool f16 = false;       // single-term fp16 MFMA pass where the MFMA path runs (> 128 rows)
-  float* nll_part = nullptr;  // lm_head writes the cross-entropy's partials here (GEMM path)
+  // lm_head writes the cross-entropy's partials here, and the logits of tgt to
+  // tlogit (GEMM path)
+  float* nll_part = nullptr;
+  const int32_t* tgt = nullptr;
+  float* tlogit = nullptr;
   // (nullable) the chunk attention's positive-score counts, attn_items(...)
   // per layer, layer after layer
   uint32_t* pos_cnt = nullptr;
@@ -847,6 +851,8 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
   a.wscale = m->w16_inv;
   a.w = W(m->w.lm); a.N = d.V; a.K = d.D; a.norm = 1; a.y = logits;
   a.nll_part = gm ? o.nll_part : nullptr;
+  a.tgt = o.tgt;
+  a.tlogit = o.tlogit;
   linear(m, s, GV_STORE, a, d_pos, gm);
 }
 
@@ -874,13 +880,18 @@ int32_t forward_core(fg_model* m, const int32_t* d_ids, int B, int T, float* d_l
   // the cross-entropy from lm_head's log-sum-exp partials where the GEMM
   // writes them (no second pass over the logits), else from the logits
   const bool nll_parts = d_tgt && d_nll && m->ws.nllp && use_gemm(m->d, rows) &&
-                         gemm_store_nll(rows, m->d.V);
-  if (nll_parts) o.nll_part = m->ws.nllp;
+                         gemm_store_nll(rows, m->d.V, pass_f16(m, rows, m->fwd_f16));
+  if (nll_parts) {
+    o.nll_part = m->ws.nllp;
+    o.tgt = d_tgt;
+    o.tlogit = m->ws.stat;
+    if (!d_logits) logits = nullptr;  // (asked for the cross-entropy alone)
+  }
   o.pos_cnt = d_pos_cnt;
   layer_stack(m, s, d_ids, B, T, 0, nullptr, nullptr, nullptr, T, 0, nullptr, logits, o);
   if (nll_parts)
     timed(m, s, FG_K_OTHER, 0, (double)rows * (m->d.V / NLL_GROUP_COLS) * 8 + rows * 12, [&] {
-      launch_nll_parts(s, logits, m->ws.nllp, d_tgt, rows, m->d.V, d_nll);
+      launch_nll_parts(s, m->ws.stat, m->ws.nllp, d_tgt, rows, m->d.V, d_nll);
     });
   else if (d_tgt && d_nll)
     timed(m, s, FG_K_OTHER, 0, vb, [&] { launch_nll(s, logits, d_tgt, rows, m->d.V, d_nll); });
@@ -1061,7 +1072,7 @@ int32_t forward_host(fg_model* m, const int32_t* ids, int32_t B, int32_t T, floa
   HIPCHK(hipMemcpyAsync(m->ws.ids, ids, rows * 4, hipMemcpyHostToDevice, s));
   if (targets) HIPCHK(hipMemcpyAsync(m->ws.tgt, targets, rows * 4, hipMemcpyHostToDevice, s));
   if (m->fwd_f16) launch_zero_u32(s, m->d_ovf, 1);
-  RCCHK(forward_core(m, m->ws.ids, B, T, m->ws.logits, targets ? m->ws.tgt : nullptr,
+  RCCHK(forward_core(m, m->ws.ids, B, T, logits ? m->ws.logits : nullptr, targets ? m->ws.tgt : nullptr,
                      targets ? m->ws.nll : nullptr, s, npos ? m->d_pos : nullptr));
   RCCHK(check_f16_range(m, s));
   if (logits) RCCHK(copy_out(m, logits, m->ws.logits, (size_t)rows * m->d.V * 4, s));
@@ -1147,7 +1158,7 @@ extern "C" int32_t fg_eval_bpb(fg_model* m, const int32_t* rows, int32_t n_rows,
       HIPCHK(hipMemcpyAsync(m->ws.ids, ids.data(), n * 4, hipMemcpyHostToDevice, s));
       HIPCHK(hipMemcpyAsync(m->ws.tgt, tgt.data(), n * 4, hipMemcpyHostToDevice, s));
       if (m->fwd_f16) launch_zero_u32(s, m->d_ovf, 1);
-      RCCHK(forward_core(m, m->ws.ids, nb, T, m->ws.logits, m->ws.tgt, m->ws.nll, s));
+      RCCHK(forward_core(m, m->ws.ids, nb, T, nullptr, m->ws.tgt, m->ws.nll, s));
       timed(m, s, FG_K_OTHER, 0, (double)n * 12, [&] {
         launch_bpb_rows(s, m->ws.nll, m->ws.tgt, nb, T, d_tb, d_rn, d_rb);
       });

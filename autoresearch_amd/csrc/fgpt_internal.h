@@ -84,8 +84,8 @@ __host__ __device__ __forceinline__ int64_t tile_at(int64_t r, int k, int K) {
 __host__ __device__ __forceinline__ int64_t tile_rows(int64_t M) { return (M + 15) / 16 * 16; }
 
 // Columns of one log-sum-exp partial of lm_head's cross-entropy epilogue
-// (one wavefront row of the 128x256 register-epilogue tile).
-constexpr int NLL_GROUP_COLS = 128;
+// (a wavefront's of the 256x256 register-epilogue tile).
+constexpr int NLL_GROUP_COLS = 64;
 
 // Activation workspace for up to `rows` token rows.
 struct Work {
@@ -189,9 +189,13 @@ struct GemvArgs {
   float wscale;
   // lm_head with the cross-entropy to follow (STORE only, nullable): per row
   // and NLL_GROUP_COLS-column group, the group's maximum logit and sum of
-  // exp(logit - maximum), [M][N/NLL_GROUP_COLS][2]; the GEMM then runs where
-  // it can write them (gemm_store_nll says when)
+  // exp(logit - maximum), [M][N/NLL_GROUP_COLS][2], and tlogit[m] = the logit
+  // of tgt[m] (where that is an id); the logits themselves are not stored when
+  // y is null. The GEMM then runs where it can write them (gemm_store_nll says
+  // when)
   float* nll_part;
+  const int32_t* tgt;
+  float* tlogit;
   // single-term fp16 pass (nullable): set to 1 by any epilogue whose fp16
   // operand store would round a value to inf (|v| >= 65520 or not finite)
   uint32_t* ovf;
@@ -302,13 +306,13 @@ void launch_bpb_rows(hipStream_t s, const float* nll, const int32_t* tgt, int ro
 // Per-row nll = logsumexp - logit[tgt].
 void launch_nll(hipStream_t s, const float* logits, const int32_t* tgt, int64_t rows, int V,
                 float* out);
-// The same from lm_head's per-row partials (GemvArgs::nll_part,
-// V/NLL_GROUP_COLS groups a row) and the target's logit.
-void launch_nll_parts(hipStream_t s, const float* logits, const float* parts, const int32_t* tgt,
+// The same from lm_head's per-row partials and target logits
+// (GemvArgs::nll_part, tlogit; V/NLL_GROUP_COLS groups a row).
+void launch_nll_parts(hipStream_t s, const float* tlogit, const float* parts, const int32_t* tgt,
                       int64_t rows, int V, float* out);
 // Whether an lm_head GEMM of M rows over a vocabulary of N writes the
-// log-sum-exp partials when asked (1025 to 4096 rows, N a multiple of 256).
-bool gemm_store_nll(int64_t M, int N);
+// log-sum-exp partials when asked (f16: the single-term pass).
+bool gemm_store_nll(int64_t M, int N, bool f16);
 
 // ---- greedy speculative decoding
 // host side (fgpt_spec.hip)

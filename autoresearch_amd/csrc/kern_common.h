@@ -122,18 +122,26 @@ __device__ __forceinline__ float half_sum(float v) {
   return (threadIdx.x & 32) ? c + d : a + b;
 }
 
-// Maximum across each half-wavefront, in half_sum's pattern.
-__device__ __forceinline__ float half_max(float v) {
+// Sum and maximum across each half-wavefront without lane reads: the two 16-lane rows of a half
+// meet by gfx950's row swap (v_permlane16_swap: odd rows of the first operand
+// with even rows of the second).
+__device__ __forceinline__ float half_sum_swap(float v) {
+  v += dpp_f<0xB1>(v);
+  v += dpp_f<0x4E>(v);
+  v += dpp_f<0x141>(v);
+  v += dpp_f<0x140>(v);
+  const uint32_t u = __float_as_uint(v);
+  const auto w = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return __uint_as_float(w[0]) + __uint_as_float(w[1]);
+}
+__device__ __forceinline__ float half_max_swap(float v) {
   v = fmaxf(v, dpp_f<0xB1>(v));
   v = fmaxf(v, dpp_f<0x4E>(v));
   v = fmaxf(v, dpp_f<0x141>(v));
   v = fmaxf(v, dpp_f<0x140>(v));
-  const int iv = __builtin_bit_cast(int, v);
-  const float a = __builtin_bit_cast(float, __builtin_amdgcn_readlane(iv, 0));
-  const float b = __builtin_bit_cast(float, __builtin_amdgcn_readlane(iv, 16));
-  const float c = __builtin_bit_cast(float, __builtin_amdgcn_readlane(iv, 32));
-  const float d = __builtin_bit_cast(float, __builtin_amdgcn_readlane(iv, 48));
-  return (threadIdx.x & 32) ? fmaxf(c, d) : fmaxf(a, b);
+  const uint32_t u = __float_as_uint(v);
+  const auto w = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return fmaxf(__uint_as_float(w[0]), __uint_as_float(w[1]));
 }
 
 // Maximum across the 64 lanes, in wave_sum's pattern.

@@ -1397,7 +1397,7 @@ __global__ __launch_bounds__(256) void k_nll(const float* __restrict__ logits,
 // log-sum-exp partials (one (max, sum of exp(logit - max)) per
 // NLL_GROUP_COLS-column group, written by the GEMM's epilogue): one wavefront per row, the row
 // maximum and the rescaled sums reduced in a fixed order.
-__global__ __launch_bounds__(256) void k_nll_parts(const float* __restrict__ logits,
+__global__ __launch_bounds__(256) void k_nll_parts(const float* __restrict__ tlogit,
                                                    const float* __restrict__ parts,
                                                    const int32_t* __restrict__ tgt, int64_t rows,
                                                    int V, float* __restrict__ out) {
@@ -1413,14 +1413,14 @@ __global__ __launch_bounds__(256) void k_nll_parts(const float* __restrict__ log
   sum = wave_sum(sum);
   if (lane == 0) {
     const int t = tgt[row];
-    out[row] = (t >= 0 && t < V) ? (m + logf(sum)) - logits[row * V + t] : __builtin_nanf("");
+    out[row] = (t >= 0 && t < V) ? (m + logf(sum)) - tlogit[row] : __builtin_nanf("");
   }
 }
 
-void launch_nll_parts(hipStream_t s, const float* logits, const float* parts, const int32_t* tgt,
+void launch_nll_parts(hipStream_t s, const float* tlogit, const float* parts, const int32_t* tgt,
                       int64_t rows, int V, float* out) {
   if (rows <= 0) return;
-  FG_LAUNCH(k_nll_parts, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, logits, parts, tgt,
+  FG_LAUNCH(k_nll_parts, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, tlogit, parts, tgt,
             rows, V, out);
 }
 

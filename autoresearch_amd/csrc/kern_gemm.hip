@@ -506,6 +506,7 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm2(GemvArgs a,
   constexpr int STAGE_BYTES = GROUPS * 1024;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   __shared__ float sinv[BM];
+  __shared__ int stgt[EPI == GV_STORE ? BM : 1];  // the rows' targets (a.nll_part)
 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int wm = wid / NWN, wn = wid % NWN;
@@ -579,8 +580,10 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm2(GemvArgs a,
         for (int t = 0; t < a.ssq_n; ++t) ssum += a.ssq_in[(int64_t)(m0 + r) * a.ssq_n + t];
       sinv[r] = 1.0f / sqrtf(ssum / (float)K + a.eps);
     }
-    __syncthreads();
   }
+  if (EPI == GV_STORE && a.nll_part)
+    for (int r = tid; r < BM; r += NT) stgt[r] = m0 + r < M ? a.tgt[m0 + r] : -1;
+  __syncthreads();
 
   const int half = lane >> 5, cl = lane & 31;
   if constexpr (TR) {
@@ -606,61 +609,53 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm2(GemvArgs a,
     }
     return;
   }
+  // The cross-entropy's part (a.nll_part): per row and NLL_GROUP_COLS columns
+  // (this wavefront's), the maximum and the sum of exp(v - max) (the hardware
+  // exp2 of (v - max) log2 e: its relative error, a few ulp, is far below the
+  // tolerance of the nll), and the target's logit from whichever lane holds
+  // it. The values are the logits stored, bit for bit; a.y null: not stored.
+  // Row 8 (r / 4) + 4 half + r % 4 of a 32-row block is kept by lane r of the
+  // half, so a block's partials leave in one store.
+  constexpr bool CAN_NLL = EPI == GV_STORE && WN * 32 == NLL_GROUP_COLS;
+  const bool nll = CAN_NLL && a.nll_part;
 #pragma unroll
   for (int i = 0; i < WM; ++i) {
     const int rb = (wm * WM + i) * 32 + 4 * half;  // tile row of r = 0
+    float pm = 0.f, ps = 0.f;
 #pragma unroll
-    for (int j = 0; j < WN; ++j) {
-      const int n = n0 + (wn * WN + j) * 32 + cl;
+    for (int r = 0; r < 16; ++r) {
+      const int rl = rb + 8 * (r >> 2) + (r & 3), m = m0 + rl;
+      const float inv = a.norm ? sinv[rl] : 1.f;
+      float v[WN];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int rl = rb + 8 * (r >> 2) + (r & 3), m = m0 + rl;
-        const float u = P16 ? acc[i][j][r] * a.wscale : acc[i][j][r];
-        if (m < M)  // logits: read once, later
-          __builtin_nontemporal_store(a.norm ? u * sinv[rl] : u, a.y + (int64_t)m * a.N + n);
+      for (int j = 0; j < WN; ++j) {
+        v[j] = (P16 ? acc[i][j][r] * a.wscale : acc[i][j][r]) * inv;
+        if (m < M && (!CAN_NLL || a.y))  // logits: read once, later
+          __builtin_nontemporal_store(v[j], a.y + (int64_t)m * a.N + n0 + (wn * WN + j) * 32 + cl);
       }
-    }
-    if constexpr (EPI == GV_STORE) {
-      // the cross-entropy's log-sum-exp, per row and NLL_GROUP_COLS-column
-      // group (GB adjacent 32-column blocks of this wavefront): the group
-      // maximum over the lane's GB values and the half-wavefront's 32 lanes,
-      // then the sum of exp(v - max) (the hardware exp2 of (v - max) log2 e:
-      // its relative error, a few ulp, is far below the tolerance of the
-      // nll); the values are the logits just stored, bit for bit. Only
-      // tilings whose wavefront row holds whole groups generate it; the
-      // launcher picks one of those when nll_part is set.
-      constexpr int GB = NLL_GROUP_COLS / 32;
-      if constexpr (WN % GB == 0) {
-        if (a.nll_part) {
-          const int ng = a.N / NLL_GROUP_COLS;
+      if constexpr (CAN_NLL) {
+        if (nll) {
+          const int t = stgt[rl] - n0 - wn * WN * 32 - cl;  // (-1 for rows past M)
+          float mx = v[0], e = 0.f;
 #pragma unroll
-          for (int q = 0; q < WN / GB; ++q) {
-            const int grp = (n0 + (wn * WN + GB * q) * 32) / NLL_GROUP_COLS;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const int rl = rb + 8 * (r >> 2) + (r & 3);
-              float v[GB];
-#pragma unroll
-              for (int g = 0; g < GB; ++g) {
-                const float u = P16 ? acc[i][GB * q + g][r] * a.wscale : acc[i][GB * q + g][r];
-                v[g] = a.norm ? u * sinv[rl] : u;
-              }
-              float mx = v[0];
-#pragma unroll
-              for (int g = 1; g < GB; ++g) mx = fmaxf(mx, v[g]);
-              mx = half_max(mx);
-              float e = 0.f;
-#pragma unroll
-              for (int g = 0; g < GB; ++g) e += __expf(v[g] - mx);
-              const float sm = half_sum(e);
-              const int m = m0 + rl;
-              if (cl == 0 && m < M)
-                *reinterpret_cast<float2*>(a.nll_part + ((int64_t)m * ng + grp) * 2) =
-                    make_float2(mx, sm);
-            }
+          for (int j = 0; j < WN; ++j) {
+            if (t == 32 * j) a.tlogit[m] = v[j];
+            mx = fmaxf(mx, v[j]);
           }
+          mx = half_max_swap(mx);
+#pragma unroll
+          for (int j = 0; j < WN; ++j) e += __expf(v[j] - mx);
+          e = half_sum_swap(e);
+          pm = cl == r ? mx : pm;
+          ps = cl == r ? e : ps;
         }
       }
+    }
+    if constexpr (CAN_NLL) {
+      const int m = m0 + rb + 8 * (cl >> 2) + (cl & 3);
+      if (nll && cl < 16 && m < M)
+        *reinterpret_cast<float2*>(a.nll_part + ((int64_t)m * (a.N / NLL_GROUP_COLS) +
+                                                 n0 / NLL_GROUP_COLS + wn) * 2) = make_float2(pm, ps);
     }
   }
 }
@@ -697,6 +692,29 @@ void launch_cfg(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
 int tile_n(int64_t M, int N) {
   const int64_t mt64 = (M + 63) / 64;
   return (N % 128 == 0 && mt64 * (N / 128) >= 128) ? 128 : 64;
+}
+
+// The residual GEMMs whose 64x64 tiles fit the CUs in one round: no CU has
+// more to do, and none would idle for a wider tile (M = 1280, N = 768, 240
+// tiles against 160 of 64x96: fp16 proj2 18.4 -> 13.6 us, split 24.9 -> 19.5).
+bool resid_64(int64_t M, int N) {
+  return N % 64 == 0 && (M + 63) / 64 * (N / 64) <= cu_count();
+}
+
+// The residual GEMMs whose 128x128 tiles give half of the CUs or more one each
+// (and 64x96 or 64x160 tiles do not fit one round): M = 3072, N = 768 (144
+// tiles), against 64x128 ones: proj2 fp16 32.4 -> 27.9 us, split 58.5 -> 45.5;
+// M = 3072, N = 1280 (240) 59.3 -> 51.5, 103.7 -> 86.3.
+bool resid_128(int64_t M, int N) {
+  return N % 128 == 0 && 2 * ((M + 127) / 128 * (N / 128)) >= cu_count();
+}
+
+// lm_head on 256x256 tiles: past half a round of them over the CUs (three
+// quarters with split operands: at 160 tiles fp16 37.4 -> 29.9 us, split 40.9
+// -> 42.3 and more).
+bool store_256(int64_t M, int N, bool f16) {
+  const int64_t t = (M + 255) / 256 * (N / 256), ncu = cu_count();
+  return N % 256 == 0 && 4 * t > (f16 ? 2 : 3) * ncu;
 }
 
 // The residual GEMMs (proj, proj2) at prefill sizes, where 64x128 tiles
@@ -739,10 +757,19 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
     }
   }
   if constexpr (EPI == GV_STORE) {
-    // lm_head with the cross-entropy's partials: a register-epilogue tiling
-    // (the only one that writes them; gemm_store_nll guarantees the shape)
-    if (a.nll_part) {
-      launch_cfg2<EPI, 2, 2, 2, 4, 2, P16>(s, a, d_pos);
+    // lm_head: 256x256 tiles (also the ones whose epilogue writes the
+    // cross-entropy's partials); in front of them 128x256 where those cover
+    // most of the CUs once. us, before (128x256 in 4 wavefronts, 128x128) ->
+    // after, d_model 768, fp16 / split: M = 2048 51.0 -> 37.9 / 62.2 -> 52.7,
+    // 4096 98 -> 72 / 122 -> 101, 600 20.9 -> 16.0 / 25.6 -> 22.0, 800 25.7 ->
+    // 23.3 / 28.5 -> 26.6
+    if (store_256(a.M, a.N, P16)) {
+      launch_cfg2<EPI, 2, 4, 4, 2, 2, P16>(s, a, d_pos);
+      return;
+    }
+    const int64_t t256 = (a.M + 127) / 128 * (a.N / 256), ncu = cu_count();
+    if (a.N % 256 == 0 && 8 * t256 >= 5 * ncu && t256 <= ncu) {
+      launch_cfg2<EPI, 2, 4, 2, 2, 3, P16>(s, a, d_pos);
       return;
     }
   }
@@ -760,7 +787,7 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
   }
   const bool big = a.N % 128 == 0 && mt128 * (a.N / 128) >= 256;
   if constexpr (EPI == GV_RELU2 || EPI == GV_STORE) {
-    if (a.N % 256 == 0 && mt128 * (a.N / 256) >= (EPI == GV_STORE ? 384 : 768)) {
+    if (EPI == GV_RELU2 && a.N % 256 == 0 && mt128 * (a.N / 256) >= 768) {
       launch_cfg2<EPI, 2, 2, 2, 4, 2, P16>(s, a, d_pos);
       return;
     }
@@ -770,6 +797,18 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
     }
   }
   if constexpr (EPI == GV_RESID) {
+    if (resid_64(a.M, a.N)) {
+      // K over 4 wavefront groups (two wavefronts a SIMD) except where the
+      // split operands and a short K keep one group busy. us: fp16 M = 450
+      // proj2 (K = 3072) 15.6 -> 12.3, 1024 16.2 -> 12.8, M = 300 at K = 5120
+      // 22.9 -> 17.0, proj (K = 768) 6.5 -> 6.1; split M = 1024 proj2 18.9 ->
+      // 18.8, proj 7.9 on one group, more on four
+      if (a.K % 64 == 0 && (P16 || a.K >= 2048))
+        launch_cfg<EPI, 64, 64, 2, 1, 64, 4, 4, P16>(s, a, d_pos);
+      else
+        launch_cfg<EPI, 64, 64, 2, 2, 32, 4, 1, P16>(s, a, d_pos);
+      return;
+    }
     if (resid_k4(a.M, a.N, a.K)) {
       launch_cfg<EPI, 64, 96, 2, 1, 64, 3, 4, P16>(s, a, d_pos);
       return;
@@ -778,12 +817,33 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
       launch_cfg<EPI, 64, 160, 2, 1, 64, 3, 2, P16>(s, a, d_pos);
       return;
     }
+    if (resid_128(a.M, a.N) && !big) {
+      launch_cfg<EPI, 128, 128, 4, 2, 32, 3, 1, P16>(s, a, d_pos);
+      return;
+    }
   }
   const int bn = tile_n(a.M, a.N);
   if constexpr (EPI == GV_QKV) {
     // 128x128 tiles where they fit in one round and 64x128 ones would need
     // two (the depth-20 model at 2047 rows: 224 tiles against 448)
     const int64_t ncu = cu_count(), t128 = mt128 * (a.N / 128);
+    const int64_t t64 = (int64_t)((a.M + 63) / 64) * (a.N / 128);
+    // 64x64 tiles while 64x128 ones would leave CUs without one: us, fp16 /
+    // split: M = 450, N = 2304 12.4 -> 9.9 / 14.0 -> 12.0, 800 11.3 -> 9.8 /
+    // 14.2 -> 13.2
+    if (bn == 128 && t64 <= ncu) {
+      launch_cfg<EPI, 64, 64, 2, 2, 32, 4, 1, P16>(s, a, d_pos);
+      return;
+    }
+    // 64x128 tiles where 128x128 ones fill one or two rounds over the CUs and
+    // less than half of the next: M = 1800, N = 2304 (270) 20.4 -> 19.1 / 29.6
+    // -> 27.0, 2048 (288) 19.8 -> 19.9 / 28.6 -> 26.2, 4096 (576) 32.5 -> 31.2 /
+    // 44.1 -> 42.0; M = 3072, N = 1792 (336) 29.4 -> 27.6 / 43.6 -> 38.5
+    if (bn == 128 && a.K % 64 == 0 && t128 > ncu && t128 < 3 * ncu && 2 * (t128 % ncu) < ncu) {
+      if constexpr (P16) launch_cfg<EPI, 64, 128, 2, 2, 64, 2, 1, P16>(s, a, d_pos);
+      else launch_cfg<EPI, 64, 128, 2, 2, 32, 3, 1, P16>(s, a, d_pos);
+      return;
+    }
     if (bn == 128 && !big && t128 <= ncu && 2 * t128 > ncu) {
       launch_cfg<EPI, 128, 128, 4, 2, 32, 3, 1, P16>(s, a, d_pos);
       return;
@@ -837,18 +897,23 @@ int cu_count() {
   return v;
 }
 
-// lm_head writes the log-sum-exp partials over 1025 to 4096 rows. Measured
-// against the separate pass over the logits on the depth-12 forward: 10-30
-// us faster per pass at 2048 and 4096 rows, 10 us slower at 1024 (the pass
-// over 128 MB of logits is short there); beyond 4096 rows the 256x256 tiles
-// hold 64 rows a lane and the epilogue's reductions cost more than the pass.
-bool gemm_store_nll(int64_t M, int N) { return M > 1024 && M <= 4096 && N % 256 == 0; }
+// lm_head writes the log-sum-exp partials wherever it runs on 256x256 tiles
+// (a row's 64 columns of a wavefront meet by DPP and one row swap); where the
+// logits are not asked for it then stores none of them. Whole passes with the
+// tiles above: 2048 rows, logits and cross-entropy, fp16 1283 -> 1246 us; the
+// cross-entropy alone over 8 x 2048 5500 -> 5366 (a pass over 537 MB of logits
+// took 94, their store about as much).
+bool gemm_store_nll(int64_t M, int N, bool f16) {
+  return gemm_rows_tile(M, N).tm == 0 && store_256(M, N, f16);
+}
 
 // RESID: one sum-of-squares partial per row and N tile.
 int gemm_ssq_parts(int64_t M, int N, int K) {
   if (const RowsTile t = gemm_rows_tile(M, N); t.tm > 0) return N / (16 * t.tn);
+  if (resid_64(M, N)) return N / 64;
   if (resid_k4(M, N, K)) return N / 96;
   if (resid_160(M, N, K)) return N / 160;
+  if (resid_128(M, N)) return N / 128;
   return N / tile_n(M, N);
 }
 

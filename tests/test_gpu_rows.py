@@ -117,3 +117,35 @@ def test_chunk_without_logits(d, B, T, pos, kv16):
     full.close()
     fast.close()
     m.close()
+
+
+WIDE1 = Dims(n_layer=1, d_model=768, n_head=6, n_kv_head=6, head_dim=128, vocab=256)
+VOCAB = Dims(n_layer=1, d_model=128, n_head=1, n_kv_head=1, head_dim=128, vocab=8192)
+
+
+@pytest.mark.parametrize("d,B,T", [
+    (WIDE1, 1, 450),    # QKV on 64x64 tiles
+    (WIDE1, 2, 901),    # QKV on 64x128 tiles, a ragged last one
+    (WIDE1, 2, 1390),   # residual GEMMs on 128x128 tiles
+    (VOCAB, 1, 600),    # lm_head on 128x256 tiles
+    (VOCAB, 1, 1100),   # fp16 lm_head on 256x256 tiles
+    (VOCAB, 2, 801)])   # both
+def test_forward_tiles(d, B, T):
+    """Passes past the few-row GEMM at the tiles their sizes pick, and the
+    cross-entropy: from lm_head's epilogue or the stored logits, with and
+    without the logits asked for (the same bits), against the oracle's (a
+    logit's bound moves a cross-entropy by at most twice that)."""
+    m, w, c, s = model(d, T)
+    ids = uniform_ids(61 + T, B * (T + 1), d.vocab).reshape(B, T + 1)
+    x, tg = np.ascontiguousarray(ids[:, :-1]).reshape(-1), np.ascontiguousarray(ids[:, 1:]).reshape(-1)
+    ref = O.gpt_forward(x, c, s, w, d, B, T)
+    ref_nll = O.nll(ref.reshape(-1, d.vocab), tg, d.vocab)
+    top = float(np.abs(ref).max())
+    for f16, tol in ((False, 5e-5), (True, 2e-3)):
+        m.set_forward_f16(f16)
+        lg, nll = m.forward(x, B, T, targets=tg)
+        assert rel(lg, ref) <= tol
+        assert np.abs(nll.reshape(-1) - ref_nll).max() <= 2 * tol * top
+        alone = m.eval_bpb(ids, np.ones(d.vocab, np.int32), batch=B, want_nll=True)["nll"]
+        assert np.array_equal(alone.reshape(-1), nll.reshape(-1))
+    m.close()
