@@ -87,9 +87,13 @@ __global__ __launch_bounds__(RNT) void k_gemm_rows(GemvArgs a, const int32_t* __
 
   const uint16_t* ap[TM];
   const uint16_t* wp[TN];
+  // rows past M repeat the last one (never stored): their lanes ask for lines
+  // that others ask for, so a block of 7 rows takes in half of each A tile
 #pragma unroll
-  for (int i = 0; i < TM; ++i)  // (row blocks past M repeat the last one and are never stored)
-    ap[i] = a.xs + (int64_t)min((m0 >> 4) + i, (M - 1) >> 4) * K * 16 + lane * 8;
+  for (int i = 0; i < TM; ++i) {
+    const int rb = min((m0 >> 4) + i, (M - 1) >> 4), r = min(lane & 15, M - 1 - 16 * rb);
+    ap[i] = a.xs + (int64_t)rb * K * 16 + (lane >> 4) * 128 + r * 8;
+  }
 #pragma unroll
   for (int j = 0; j < TN; ++j)
     wp[j] = a.w + (int64_t)((n0 >> 4) + j) * K * 16 + lane * 8;
