@@ -702,11 +702,14 @@ bool resid_64(int64_t M, int N) {
 }
 
 // The residual GEMMs whose 128x128 tiles give half of the CUs or more one each
-// (and 64x96 or 64x160 tiles do not fit one round): M = 3072, N = 768 (144
-// tiles), against 64x128 ones: proj2 fp16 32.4 -> 27.9 us, split 58.5 -> 45.5;
-// M = 3072, N = 1280 (240) 59.3 -> 51.5, 103.7 -> 86.3.
+// (and 64x96, 64x128 or 64x160 ones do not fit one round): M = 3072, N = 768
+// (144 tiles), against 64x128 ones: proj2 fp16 32.4 -> 27.9 us, split 58.5 ->
+// 45.5; M = 3072, N = 1280 (240) 59.3 -> 51.5, 103.7 -> 86.3; but M = 1554, N =
+// 1280 (130) 69.3 split, where one round of 64x128 tiles (200 at M = 1280)
+// takes 48.0.
 bool resid_128(int64_t M, int N) {
-  return N % 128 == 0 && 2 * ((M + 127) / 128 * (N / 128)) >= cu_count();
+  return N % 128 == 0 && 2 * ((M + 127) / 128 * (N / 128)) >= cu_count() &&
+         (M + 63) / 64 * (N / 128) > cu_count();
 }
 
 // lm_head on 256x256 tiles: past half a round of them over the CUs (three
