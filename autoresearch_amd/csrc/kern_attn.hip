@@ -100,6 +100,22 @@ __device__ __forceinline__ void split8(const float* v, bf16x8_t& h, bf16x8_t& l)
   }
 }
 
+// Maximum and sum of v and the other half-wavefront's (lane l ^ 32), by
+// gfx950's half swap. A shuffle goes through the LDS crossbar, which at two
+// wavefronts a SIMD waits behind their operand reads: with the swap, one sum at
+// the end instead of one a tile, and scalar wave ids, 8 x 2048 eval 5617 -> 5541
+// us, a 2 x 777 split forward 1579 -> 1563.
+__device__ __forceinline__ float halves_max(float v) {
+  const uint32_t u = __float_as_uint(v);
+  const auto w = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return fmaxf(__uint_as_float(w[0]), __uint_as_float(w[1]));
+}
+__device__ __forceinline__ float halves_sum(float v) {
+  const uint32_t u = __float_as_uint(v);
+  const auto w = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __uint_as_float(w[0]) + __uint_as_float(w[1]);
+}
+
 // four consecutive output dims (d % 4 == 0): fp32, or the bf16 hi/lo planes
 // the next GEMM reads, one 8-byte store per plane
 template <int HD, bool P16>
@@ -125,7 +141,8 @@ __global__ __launch_bounds__(512) void k_attn_mfma(AttnArgs p) {
   static_assert(GPR >= 8 && GPR % 8 == 0, "region / wavefront mismatch");
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
 
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int qg = wv & 3, kp = wv >> 2, g = lane >> 5, qi = lane & 31;
 
   // work item: (sequence*head, query block j, key chunk c); items of one
@@ -170,19 +187,22 @@ __global__ __launch_bounds__(512) void k_attn_mfma(AttnArgs p) {
 
   // DMA sources of this lane, one per 1 KB group the wavefront fills:
   // group G = wv + 8q lies in region G / GPR = 8q / GPR (compile time)
-  const uint16_t* src[GPW];
+  // (a 32-bit element offset from a workgroup-uniform base)
+  uint32_t soff[GPW];
   int koff[GPW];
+  const uint16_t* kb0 = p.ks + bk * p.npos * HD;
+  const uint16_t* vb0 = p.vt + bk * p.npos * HD;
 #pragma unroll
   for (int q = 0; q < GPW; ++q) {
     const int region = 8 * q / GPR, gi = (wv + 8 * q) % GPR;
     if (region < NKR) {  // K rows: 1024 / RBK rows per group
       const int row = gi * (1024 / RBK) + lane / (HD / 8), slot = lane % (HD / 8);
       koff[q] = 32 * (row >> 5) + tile_key(row & 31);
-      src[q] = p.ks + (region ? p.kv_plane : 0) + bk * p.npos * HD + kslot<HD>(row, slot) * 8;
+      soff[q] = kslot<HD>(row, slot) * 8;
     } else {  // V^T rows (dims): 8 rows of 64 keys per group
       const int d = gi * 8 + lane / 8, slot = lane & 7;
       koff[q] = 0;
-      src[q] = p.vt + (region == 3 ? p.kv_plane : 0) + (bk * HD + d) * p.npos + vslot(d, slot) * 8;
+      soff[q] = d * p.npos + vslot(d, slot) * 8;
     }
   }
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_off(lds) + wv * 1024);
@@ -191,7 +211,9 @@ __global__ __launch_bounds__(512) void k_attn_mfma(AttnArgs p) {
     for (int q = 0; q < GPW; ++q) {
       const int region = 8 * q / GPR;
       const uint16_t* g0 =
-          region < NKR ? src[q] + (int64_t)min(k0 + koff[q], p.nvalid - 1) * HD : src[q] + k0;
+          region < NKR ? kb0 + (region ? p.kv_plane : 0) +
+                             (soff[q] + (uint32_t)min(k0 + koff[q], p.nvalid - 1) * HD)
+                       : vb0 + (region == 3 ? p.kv_plane : 0) + (soff[q] + (uint32_t)k0);
       dma16(g0, lds0 + stg * STAGE + 8 * q * 1024);
     }
   };
@@ -201,7 +223,7 @@ __global__ __launch_bounds__(512) void k_attn_mfma(AttnArgs p) {
   for (int i = 0; i < ND; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
-  float m_run = -FLT_MAX, l_run = 0.f;  // in the log2 domain
+  float m_run = -FLT_MAX, l_run = 0.f;  // in the log2 domain; l_run: this half's keys
   uint32_t npos = 0;  // this lane's positive causal scores (p.pos_cnt)
   __shared__ float wpos[8];
   const float cs = LOG2E / sqrtf((float)HD);
@@ -251,7 +273,7 @@ __global__ __launch_bounds__(512) void k_attn_mfma(AttnArgs p) {
     float mx = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[r]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * cs;  // log2 domain (cs > 0)
+    mx = halves_max(mx) * cs;  // log2 domain (cs > 0)
     // lazy rescale: the running max moves only when a score passes it by
     // 2^8, so most tiles skip rescaling O; probabilities stay below 2^8
     if (__any(mx > m_run + 8.f)) {
@@ -271,7 +293,7 @@ __global__ __launch_bounds__(512) void k_attn_mfma(AttnArgs p) {
       sc[r] = pr;
       ps += pr;
     }
-    l_run += ps + __shfl_xor(ps, 32, 64);
+    l_run += ps;
 
     // O^T += V^T P^T over two 16-key steps: this lane's 8 probabilities are
     // keys 16s + 8g .. +7, one 16-byte chunk of each V^T row
@@ -308,6 +330,7 @@ __global__ __launch_bounds__(512) void k_attn_mfma(AttnArgs p) {
     }
   }
 
+  l_run = halves_sum(l_run);
   if (p.pos_cnt) {  // (a wavefront's count is below 2^24: its float sum is exact)
     const float wc = wave_sum((float)npos);
     if (lane == 0) wpos[wv] = wc;
