@@ -160,6 +160,7 @@ struct fg_kv {
   // of speculative rounds keyed by (rounds, 100 + rows per pass); valid for gen
   std::map<std::pair<int, int>, hipGraphExec_t> graphs;
   int64_t graphs_gen = -1;
+  int32_t* h_out = nullptr;  // pinned: a step's ids [B padded to 4], then logits [B][V]
 };
 
 namespace {
@@ -1227,6 +1228,10 @@ extern "C" int32_t fg_kv_create_ex(fg_model* m, int32_t B, int32_t maxT, int32_t
   if (e == hipSuccess) e = hipMalloc((void**)&kv->d_part, part_bytes);
   const size_t cnt_bytes = (size_t)attn_decode_counters(m->d, std::max(B, GEMV_MAX_ROWS)) * 4;
   if (e == hipSuccess) e = hipMalloc((void**)&kv->d_dcnt, cnt_bytes);
+  // a step's ids and logits on the host, where a batch's are small
+  const size_t out_bytes = ((size_t)(B + 3) / 4 * 4 + (size_t)B * m->d.V) * 4;
+  if (e == hipSuccess && out_bytes <= ((size_t)1 << 20))
+    e = hipHostMalloc((void**)&kv->h_out, out_bytes, hipHostMallocDefault);
   // zeroed on the handle's stream, and finished before the cache is handed
   // out (its first user may be a caller's stream); the reference's callers
   // zero their caches too
@@ -1245,6 +1250,7 @@ extern "C" int32_t fg_kv_create_ex(fg_model* m, int32_t B, int32_t maxT, int32_t
     if (kv->d_ids) (void)hipFree(kv->d_ids);
     if (kv->d_part) (void)hipFree(kv->d_part);
     if (kv->d_dcnt) (void)hipFree(kv->d_dcnt);
+    if (kv->h_out) (void)hipHostFree(kv->h_out);
     delete kv;
     return seterr(FG_EHIP, "KV cache allocation (%zu bytes): %s", 2 * n * esz,
                   hipGetErrorString(e));
@@ -1263,6 +1269,7 @@ extern "C" int32_t fg_kv_destroy(fg_kv* kv) {
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (kv->h_sst) (void)hipHostFree(kv->h_sst);
+  if (kv->h_out) (void)hipHostFree(kv->h_out);
   if (kv->h_smp) (void)hipHostFree(kv->h_smp);
   delete kv;
   return FG_OK;
@@ -1344,6 +1351,20 @@ int32_t kv_pass(fg_model* m, fg_kv* kv, const int32_t* h_ids, int TB, float* log
   layer_stack(m, s, m->ws.ids, B, TB, kv->len, nullptr, kv->k, kv->v, kv->maxT, lstride,
               kv->d_part, m->ws.logits, o);
   HIPCHK(hipGetLastError());
+  if (kv->h_out && (next_ids || logits) && (TB == 1 || o.last_only)) {
+    // the argmax leaves the ids, and a step's logits, in pinned host memory: no
+    // copies to pageable memory queued behind it (a step 328 -> 289 us, a prompt
+    // of 500 in chunks of 64 4063 -> 3873)
+    float* hl = reinterpret_cast<float*>(kv->h_out) + (B + 3) / 4 * 4;
+    launch_argmax(s, m->ws.logits, B, m->d.V, kv->h_out, logits ? hl : nullptr);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(s));
+    if (next_ids) memcpy(next_ids, kv->h_out, (size_t)B * 4);
+    if (logits) memcpy(logits, hl, (size_t)B * m->d.V * 4);
+    kv->len += TB;
+    kv->filled = std::max(kv->filled, kv->len);
+    return FG_OK;
+  }
   if (next_ids && (TB == 1 || o.last_only)) {
     launch_argmax(s, m->ws.logits, B, m->d.V, m->ws.amax);
     HIPCHK(hipMemcpyAsync(next_ids, m->ws.amax, (size_t)B * 4, hipMemcpyDeviceToHost, s));

@@ -297,8 +297,10 @@ void launch_greedy_tail(hipStream_t s, const Dims& d, const float* logits, int r
                         const bf16_t* wte, int32_t* ids, int32_t* out2, int32_t* d_len,
                         const int32_t* d_len0, float* lgs_out, float* x);
 
-// Per-row argmax (first max) of logits [rows][V] -> out [rows].
-void launch_argmax(hipStream_t s, const float* logits, int64_t rows, int V, int32_t* out);
+// Per-row argmax (first max) of logits [rows][V] -> out [rows], the logits
+// copied to lgs_out on the way (nullable).
+void launch_argmax(hipStream_t s, const float* logits, int64_t rows, int V, int32_t* out,
+                   float* lgs_out = nullptr);
 // Per eval row (rows of T positions): byte-weighted nats and byte count
 // with the token byte-length table tbytes (targets already range-checked).
 void launch_bpb_rows(hipStream_t s, const float* nll, const int32_t* tgt, int rows, int T,

@@ -1035,10 +1035,10 @@ __device__ __forceinline__ void amax_merge(float& v, int& i, float v2, int i2) {
   }
 }
 
-// One block per row. With a step record (d_len/d_len0 set), the chosen id
-// also goes to out2[(len - len0) * rows + row] and, when lgs_out is set, the
-// whole logits row is copied to lgs_out at the same slot: a replayed greedy
-// graph then needs no per-step pointers.
+// One block per row; when lgs_out is set, the logits row is copied to it. With
+// a step record (d_len/d_len0 set), the chosen id also goes to out2[(len -
+// len0) * rows + row] and the logits row to that slot of lgs_out: a replayed
+// greedy graph then needs no per-step pointers.
 __global__ __launch_bounds__(256) void k_argmax(const float* __restrict__ logits, int V,
                                                 int32_t* __restrict__ out,
                                                 int32_t* __restrict__ out2,
@@ -1049,8 +1049,8 @@ __global__ __launch_bounds__(256) void k_argmax(const float* __restrict__ logits
   __shared__ int ri[4];
   const int64_t row = blockIdx.x, rows = gridDim.x;
   const float* l = logits + row * V;
-  const int64_t slot = d_len ? (int64_t)(*d_len - *d_len0) * rows + row : 0;
-  float* cp = (d_len && lgs_out) ? lgs_out + slot * V : nullptr;
+  const int64_t slot = d_len ? (int64_t)(*d_len - *d_len0) * rows + row : row;
+  float* cp = lgs_out ? lgs_out + slot * V : nullptr;
   float bv = -INFINITY;
   int bi = 0x7fffffff;
   auto take = [&](float v, int j) {
@@ -1356,8 +1356,9 @@ void launch_spec_commit(hipStream_t s, SpecDev* st, const float* logits, int V, 
   FG_LAUNCH(k_spec_commit, dim3(1), dim3(1024), 0, s, st, logits, V, ids);
 }
 
-void launch_argmax(hipStream_t s, const float* logits, int64_t rows, int V, int32_t* out) {
-  launch_argmax_step(s, logits, rows, V, out, nullptr, nullptr, nullptr, nullptr);
+void launch_argmax(hipStream_t s, const float* logits, int64_t rows, int V, int32_t* out,
+                   float* lgs_out) {
+  launch_argmax_step(s, logits, rows, V, out, nullptr, nullptr, nullptr, lgs_out);
 }
 
 // One block per row. Rows of up to 256*4*NV4 logits are read once, as
