@@ -1541,7 +1541,7 @@ int32_t fused_launch(fg_model* m, fg_kv* kv, const int32_t* d_id0, int len0, int
   const size_t tn = (size_t)FUSED_NWG * (d.L + 1) * 32;
   a.trace = nullptr;  // (null: the kernel built without timestamps)
   a.trace_step = n_steps > 1 ? 1 : 0;
-  if (tpath && *tpath) {
+  if (tpath && *tpath && !host_sd) {
     HIPCHK(hipMalloc((void**)&a.trace, tn * 8));
     HIPCHK(hipMemsetAsync(a.trace, 0, tn * 8, s));
   }
@@ -2065,29 +2065,50 @@ extern "C" int32_t fg_decode_sample(fg_model* m, fg_kv* kv, int32_t* ids, int32_
   int done = 0;
   const int total = n_total - n_known;
   const bool fused = fused_applies(m, kv, total);
-  if (fused && m->fl.kind == 0 && !m->timing) {
-    // one launch for all the steps, the draws in it: no launch, no placement
-    // and no cold weight pipeline per id (timing brackets each step instead)
-    int32_t* inp = (int32_t*)((char*)kv->d_smp + offsetof(SampleDev, inp));
-    RCCHK(fused_launch(m, kv, inp, n_known - 1, total, kv->d_sids, nullptr, true, h));
-    done = total;
-  } else if (fused) {
+  // The draws inside the persistent loop, one launch for all the steps (no
+  // launch, no placement and no cold weight pipeline per id), where the rows
+  // are peaked enough for it: a launch that meets one it had to sort whole ends
+  // with it, and the next 32 ids (then 64, 128, ..) take the launches below.
+  // A topp that no cut can pass takes them at once, and timing, which brackets
+  // each step.
+  const bool in_loop = fused && m->fl.kind == 0 && !m->timing && (c.temp <= 0.f || c.topp < 0.998f);
+  int32_t* inp = (int32_t*)((char*)kv->d_smp + offsetof(SampleDev, inp));
+  auto failed = [&](int32_t rc) {
+    (void)hipStreamSynchronize(s);
+    kv->len = n_known - 1;
+    return rc;
+  };
+  for (int single = in_loop ? 0 : total, next = 32; fused && done < total;) {
+    if (single == 0) {
+      h->pp = n_known + done;
+      int32_t rc = fused_launch(m, kv, inp, n_known - 1 + done, total - done, kv->d_sids, nullptr,
+                                true, h);
+      if (rc != FG_OK) return failed(rc);
+      HIPCHK(hipMemcpyAsync(h, kv->d_smp, sizeof *h, hipMemcpyDeviceToHost, s));
+      HIPCHK(hipStreamSynchronize(s));
+      rc = fused_check(m);
+      if (rc != FG_OK) return failed(rc);
+      done = h->pp - n_known;
+      single = next;
+      next *= 2;
+      continue;
+    }
     // each step the persistent kernel for one step (its logits; its own
     // argmax goes to the spare inp[1]), then the draw, which leaves the next
     // input in inp[0]; the error flag is cleared once and read at the end
-    int32_t* inp = (int32_t*)((char*)kv->d_smp + offsetof(SampleDev, inp));
     HIPCHK(hipMemsetAsync(m->fused_err, 0, 4, s));
-    for (; done < total; ++done) {
+    for (; done < total && single > 0; ++done, --single) {
       const int32_t rc = fused_launch(m, kv, inp, n_known - 1 + done, 1, inp + 1,
                                       m->ws.logits, false);
-      if (rc != FG_OK) {
-        (void)hipStreamSynchronize(s);
-        kv->len = n_known - 1;
-        return rc;
-      }
+      if (rc != FG_OK) return failed(rc);
       timed(m, s, FG_K_OTHER, 0, (double)m->d.V * 4, [&] {
         launch_sample_step(s, kv->d_smp, m->ws.logits, m->d.V, kv->d_sids);
       });
+    }
+    if (done < total) {  // (its error flag, before the next launch clears it)
+      HIPCHK(hipStreamSynchronize(s));
+      const int32_t rc = fused_check(m);
+      if (rc != FG_OK) return failed(rc);
     }
   }
   while (done < total) {

@@ -215,6 +215,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
   }
   embed(*a.d_id0, a.len0);
 
+  int drawn = 0;  // (SAMPLE) steps whose id is drawn
   for (int s = 0; s < a.n_steps; ++s) {
     const int pos = a.len0 + s;
     for (int l = 0; l <= L; ++l) {
@@ -565,7 +566,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
               slot_put_dev(SMP + V + lane, __int_as_float(id), ep + 1);
             if (tid == 0) {
               ired[4] = id;
-              __hip_atomic_store(a.ids_out + a.n_gen + s, id, __ATOMIC_RELAXED,
+              __hip_atomic_store(a.ids_out + a.n_gen + s, id & ~SAMPLE_WHOLE, __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
               asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the next draw's history)
             }
@@ -621,15 +622,19 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
       int id = ired[4];
       if (id == 0x7fffffff) id = 0;  // no finite candidate: position 1, as the scan starts there
       if (!SAMPLE && b == 0 && tid == 0) a.ids_out[s] = id;
+      if (SAMPLE) {
+        ++drawn;
+        if (id & SAMPLE_WHOLE) break;  // (the loop of steps)
+      }
       if (s + 1 < a.n_steps) embed(id, pos + 1);
     }
   }
-  if (SAMPLE && b == 0 && tid == 0) {  // the loop's state after n_steps draws
+  if (SAMPLE && b == 0 && tid == 0) {  // the loop's state after its draws
     SampleDev* sd = a.sd;
     sd->rng = *rng;
-    sd->pp += a.n_steps;
-    sd->len += a.n_steps;
-    sd->inp[0] = ired[4];
+    sd->pp += drawn;
+    sd->len += drawn;
+    sd->inp[0] = ired[4] & ~SAMPLE_WHOLE;
   }
 done:
   if (loader) waitdma();  // no LDS-DMA may outlive the workgroup

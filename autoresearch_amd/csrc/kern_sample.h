@@ -49,6 +49,11 @@ __device__ __forceinline__ uint64_t prob_key(float p, int id) {
 constexpr int SVT = 1024;  // threads that sample_row's sums are split over
 constexpr int64_t sample_wg_aux(int V) { return 2 * V + 4 * SVT + 256; }
 
+// Sorting it whole takes 240 us here (k_sample_step, on four times the threads,
+// draws in 52): SAMPLE_WHOLE is then set in the result, and the loop ends so that
+// the caller goes on with k_sample_step (24 ids at temperature 2: 227 us an id
+// against 218 with launches alone, 374 without the way out).
+constexpr int SAMPLE_WHOLE = 1 << 30;
 template <int V>
 __device__ int sample_wg(float* pr, uint8_t* aux, const int32_t* gen, int ngen, const SampleCfg& c,
                          int64_t* state, bool comp) {
@@ -352,7 +357,7 @@ __device__ int sample_wg(float* pr, uint8_t* aux, const int32_t* gen, int ngen, 
       if (pr[i] >= u && i < hit) hit = i;
   hit = block_min(hit);
   hit = hit < cut ? hit : cut - 1;
-  const int id = cut_row ? 0x7fffffff - (int)(uint32_t)keys[hit] : (int)id16[hit];
+  const int id = cut_row ? 0x7fffffff - (int)(uint32_t)keys[hit] : (int)id16[hit] | SAMPLE_WHOLE;
   lds_barrier();  // (pr and aux are free again)
   return id;
 }

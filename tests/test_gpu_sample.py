@@ -221,10 +221,11 @@ def test_decode_sample_loop_persistent(d):
 def test_sampling_inside_the_persistent_loop(d, cfg):
     """One launch that draws between its steps against a launch and a
     k_sample_step per id (what timing runs): the same logits, sums and order,
-    so the same ids and generator state, bit for bit."""
+    so the same ids and generator state, bit for bit. 48 ids: a row sorted whole
+    sends the next 32 to the launches, and the loop is tried again."""
     m = engine.Model(d, stacks=seeded_weights(d, 9))
     prompt = uniform_ids(19, 9, d.vocab)
-    n_gen = 24
+    n_gen = 48
     c, s = rope_tables(prompt.size + n_gen, d.head_dim)
     m.set_rope(c.reshape(-1), s.reshape(-1))
     outs = []
