@@ -1,4 +1,5 @@
-// kern_gemm.hip -- bf16 MFMA GEMM for prefill and batched decode (gfx950).
+// kern_gemm.hip -- MFMA GEMM for more than 256 token rows (gfx950; fewer run in
+// kern_rows.hip).
 //
 // C[M][N] = epi( s_m * (A[M][K] . W[N][K]^T) ), the y = x W^T of
 // linear3d_sgemm (src/lib/fortran_blas.f90:39-57) with rmsnorm0's row scale
@@ -900,14 +901,14 @@ int cu_count() {
   return v;
 }
 
-// lm_head writes the log-sum-exp partials wherever it runs on 256x256 tiles
-// (a row's 64 columns of a wavefront meet by DPP and one row swap); where the
-// logits are not asked for it then stores none of them. Whole passes with the
-// tiles above: 2048 rows, logits and cross-entropy, fp16 1283 -> 1246 us; the
-// cross-entropy alone over 8 x 2048 5500 -> 5366 (a pass over 537 MB of logits
-// took 94, their store about as much).
+// lm_head writes the log-sum-exp partials where it runs on 256x256 tiles, up to
+// 4096 rows (a row's 64 columns of a wavefront meet by DPP and one row swap),
+// and then stores no logits where none are asked for. Past that its reductions,
+// 11 us a round of tiles, cost more than a pass over stored logits: 16384 rows
+// 387 us against 271 + 94. Whole pass with the tiles above: 2048 rows, logits
+// and cross-entropy, fp16 1283 -> 1246 us.
 bool gemm_store_nll(int64_t M, int N, bool f16) {
-  return gemm_rows_tile(M, N).tm == 0 && store_256(M, N, f16);
+  return M <= 4096 && gemm_rows_tile(M, N).tm == 0 && store_256(M, N, f16);
 }
 
 // RESID: one sum-of-squares partial per row and N tile.

@@ -88,7 +88,8 @@ __global__ __launch_bounds__(RNT) void k_gemm_rows(GemvArgs a, const int32_t* __
   const uint16_t* ap[TM];
   const uint16_t* wp[TN];
   // rows past M repeat the last one (never stored): their lanes ask for lines
-  // that others ask for, so a block of 7 rows takes in half of each A tile
+  // that others ask for, so a block of 7 rows takes in half of each A tile (16
+  // decode steps of 7 sequences 6459 -> 6031 us)
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int rb = min((m0 >> 4) + i, (M - 1) >> 4), r = min(lane & 15, M - 1 - 16 * rb);
