@@ -105,6 +105,7 @@ struct fg_model {
   uint32_t* fused_err = nullptr;
   uint32_t fused_ep = 1;
   bool fused_on = true;  // fg_set_option(FG_OPT_FUSED_DECODE)
+  int32_t loop_ids = 0;  // FG_OPT_SAMPLED_IN_LOOP
   // FG_OPT_FORWARD_F16: the fp16 copy of the GEMM weights (the bf16 arena's
   // layout, each value times w16_scale, a power of 2; wte unused), made on
   // first use; w16_inv = 1 / w16_scale; wmax = max |w| of those weights
@@ -1479,7 +1480,8 @@ bool fused_applies(const fg_model* m, const fg_kv* kv, int n_steps) {
 // are cleared first, and its error flag too when clear_err is set (a caller
 // running several launches clears it once and reads it after the last).
 // host_sd: draw each next id instead (the host's copy of kv->d_smp; ids_out =
-// kv->d_sids).
+// kv->d_sids; logits_out takes the one row that ends the loop early, with the
+// ids drawn so far counted in kv->d_smp).
 int32_t fused_launch(fg_model* m, fg_kv* kv, const int32_t* d_id0, int len0, int n_steps,
                      int32_t* ids_out, float* logits_out, bool clear_err,
                      const SampleDev* host_sd = nullptr) {
@@ -1576,16 +1578,20 @@ int32_t fused_decode(fg_model* m, fg_kv* kv, const int32_t* ids, int n_steps, in
                       with_logits ? kv->d_lgs : nullptr, true);
 }
 
-// The persistent launch's error flag, after the device is idle: 0, or the
-// engine error for it.
-int32_t fused_check(fg_model* m) {
-  uint32_t err = 0;
-  HIPCHK(hipMemcpy(&err, m->fused_err, 4, hipMemcpyDeviceToHost));
+// The engine error for a persistent launch's error flag.
+int32_t fused_error(uint32_t err) {
   if (err != 0)
     return seterr(FG_EHIP, "persistent decode: %s",
                   err == 2 ? "an XCD held more than 32 of its workgroups"
                            : "a hand-over between workgroups timed out");
   return FG_OK;
+}
+
+// The flag itself, after the device is idle.
+int32_t fused_check(fg_model* m) {
+  uint32_t err = 0;
+  HIPCHK(hipMemcpy(&err, m->fused_err, 4, hipMemcpyDeviceToHost));
+  return fused_error(err);
 }
 
 }  // namespace
@@ -2033,6 +2039,7 @@ extern "C" int32_t fg_decode_sample(fg_model* m, fg_kv* kv, int32_t* ids, int32_
     return seterr(FG_EFULL, "cache full (raise maxT): n_total %d > %d", n_total, kv->maxT);
   RCCHK(check_ids(m, ids, n_known));
   GUARD(m);
+  m->loop_ids = 0;
   if (n_total == n_known) return FG_OK;
   RCCHK(check_rope(m, n_total));
   RCCHK(ensure_work(m, 1));
@@ -2043,7 +2050,8 @@ extern "C" int32_t fg_decode_sample(fg_model* m, fg_kv* kv, int32_t* ids, int32_
   if (!kv->d_smp) {
     HIPCHK(hipMalloc((void**)&kv->d_smp, sizeof(SampleDev)));
     RCCHK(dev_zero(m, kv->d_smp, sizeof(SampleDev)));
-    HIPCHK(hipHostMalloc((void**)&kv->h_smp, sizeof(SampleDev), hipHostMallocDefault));
+    // (and, behind it, a persistent launch's error flag)
+    HIPCHK(hipHostMalloc((void**)&kv->h_smp, sizeof(SampleDev) + 4, hipHostMallocDefault));
   }
   if (kv->graphs_gen != m->gen) {
     for (auto& g : kv->graphs) (void)hipGraphExecDestroy(g.second);
@@ -2067,10 +2075,12 @@ extern "C" int32_t fg_decode_sample(fg_model* m, fg_kv* kv, int32_t* ids, int32_
   const bool fused = fused_applies(m, kv, total);
   // The draws inside the persistent loop, one launch for all the steps (no
   // launch, no placement and no cold weight pipeline per id), where the rows
-  // are peaked enough for it: a launch that meets one it had to sort whole ends
-  // with it, and the next 32 ids (then 64, 128, ..) take the launches below.
-  // A topp that no cut can pass takes them at once, and timing, which brackets
-  // each step.
+  // are peaked enough for it: a launch that meets one that has to be sorted
+  // whole ends there with the row's logits, k_sample_step draws from them, and
+  // the next 32 ids (then 64, 128, ..) take the launches below (256 ids at
+  // temperature 2, d12, us an id: 209.4 so, 209.5 with launches alone, 221 when
+  // the loop sorted such a row itself). A topp that no cut can pass takes them
+  // at once, and timing, which brackets each step.
   const bool in_loop = fused && m->fl.kind == 0 && !m->timing && (c.temp <= 0.f || c.topp < 0.998f);
   int32_t* inp = (int32_t*)((char*)kv->d_smp + offsetof(SampleDev, inp));
   auto failed = [&](int32_t rc) {
@@ -2078,25 +2088,37 @@ extern "C" int32_t fg_decode_sample(fg_model* m, fg_kv* kv, int32_t* ids, int32_
     kv->len = n_known - 1;
     return rc;
   };
+  // the persistent launches' error flag, cleared once: every launch leaves its
+  // failure in it until it is read
+  if (fused) HIPCHK(hipMemsetAsync(m->fused_err, 0, 4, s));
   for (int single = in_loop ? 0 : total, next = 32; fused && done < total;) {
     if (single == 0) {
       h->pp = n_known + done;
-      int32_t rc = fused_launch(m, kv, inp, n_known - 1 + done, total - done, kv->d_sids, nullptr,
-                                true, h);
+      int32_t rc = fused_launch(m, kv, inp, n_known - 1 + done, total - done, kv->d_sids,
+                                m->ws.logits, false, h);
       if (rc != FG_OK) return failed(rc);
+      // k_sample_step runs (on a row the loop ended at; it does nothing once
+      // every id is drawn) while the host learns how far the loop came
+      uint32_t* herr = reinterpret_cast<uint32_t*>(h + 1);
       HIPCHK(hipMemcpyAsync(h, kv->d_smp, sizeof *h, hipMemcpyDeviceToHost, s));
-      HIPCHK(hipStreamSynchronize(s));
-      rc = fused_check(m);
+      HIPCHK(hipMemcpyAsync(herr, m->fused_err, 4, hipMemcpyDeviceToHost, s));
+      hipEvent_t ev = get_event(m);
+      HIPCHK(hipEventRecord(ev, s));
+      launch_sample_step(s, kv->d_smp, m->ws.logits, m->d.V, kv->d_sids);
+      const hipError_t e = hipEventSynchronize(ev);
+      m->evpool.push_back(ev);
+      HIPCHK(e);
+      rc = fused_error(*herr);
       if (rc != FG_OK) return failed(rc);
-      done = h->pp - n_known;
+      m->loop_ids += h->pp - n_known - done;
+      done = std::min(h->pp - n_known + 1, total);
       single = next;
       next *= 2;
       continue;
     }
     // each step the persistent kernel for one step (its logits; its own
     // argmax goes to the spare inp[1]), then the draw, which leaves the next
-    // input in inp[0]; the error flag is cleared once and read at the end
-    HIPCHK(hipMemsetAsync(m->fused_err, 0, 4, s));
+    // input in inp[0]
     for (; done < total && single > 0; ++done, --single) {
       const int32_t rc = fused_launch(m, kv, inp, n_known - 1 + done, 1, inp + 1,
                                       m->ws.logits, false);
@@ -2104,11 +2126,6 @@ extern "C" int32_t fg_decode_sample(fg_model* m, fg_kv* kv, int32_t* ids, int32_
       timed(m, s, FG_K_OTHER, 0, (double)m->d.V * 4, [&] {
         launch_sample_step(s, kv->d_smp, m->ws.logits, m->d.V, kv->d_sids);
       });
-    }
-    if (done < total) {  // (its error flag, before the next launch clears it)
-      HIPCHK(hipStreamSynchronize(s));
-      const int32_t rc = fused_check(m);
-      if (rc != FG_OK) return failed(rc);
     }
   }
   while (done < total) {
@@ -2188,8 +2205,8 @@ extern "C" int32_t fg_set_option(fg_model* m, int32_t key, int32_t value) {
 extern "C" int32_t fg_get_option(fg_model* m, int32_t key, int32_t* value, char* why,
                                  int32_t len) {
   if (!m || !value) return seterr(FG_EARG, "NULL argument");
-  if (key == FG_OPT_FORWARD_F16) {
-    *value = m->fwd_f16 ? 1 : 0;
+  if (key == FG_OPT_FORWARD_F16 || key == FG_OPT_SAMPLED_IN_LOOP) {
+    *value = key == FG_OPT_SAMPLED_IN_LOOP ? m->loop_ids : m->fwd_f16 ? 1 : 0;
     if (why && len > 0) why[0] = '\0';
     return FG_OK;
   }

@@ -87,7 +87,8 @@ typedef FusedShape<256, 2, 1024> ShapeSmall;
 
 // SAMPLE: the next id is drawn (a.sd) in place of the argmax: every workgroup
 // hands its logits to workgroup 0, which draws from the row (sample_wg, in the
-// weight buffer lm_head has just freed) and hands the id to all.
+// weight buffer lm_head has just freed) and hands the id to all. A row that
+// would have to be sorted whole goes to a.logits_out and ends the loop.
 template <class Sh, bool TRACE, bool SAMPLE>
 __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
   }
   embed(*a.d_id0, a.len0);
 
-  int drawn = 0;  // (SAMPLE) steps whose id is drawn
+  int drawn = 0, last = 0;  // (SAMPLE) ids drawn, the last of them
   for (int s = 0; s < a.n_steps; ++s) {
     const int pos = a.len0 + s;
     for (int l = 0; l <= L; ++l) {
@@ -564,9 +565,13 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
                                         comp);
             if (wv == 0 && lane < FUSED_LMC)
               slot_put_dev(SMP + V + lane, __int_as_float(id), ep + 1);
-            if (tid == 0) {
-              ired[4] = id;
-              __hip_atomic_store(a.ids_out + a.n_gen + s, id & ~SAMPLE_WHOLE, __ATOMIC_RELAXED,
+            if (tid == 0) ired[4] = id;
+            if (id == SAMPLE_WHOLE) {  // (pr holds penalised values; the slots still the logits)
+              if (comp)
+                for (int i = tid; i < V; i += 256)
+                  a.logits_out[i] = __uint_as_float((uint32_t)slot_load(SMP + i));
+            } else if (tid == 0) {
+              __hip_atomic_store(a.ids_out + a.n_gen + s, id, __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
               asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the next draw's history)
             }
@@ -623,8 +628,9 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
       if (id == 0x7fffffff) id = 0;  // no finite candidate: position 1, as the scan starts there
       if (!SAMPLE && b == 0 && tid == 0) a.ids_out[s] = id;
       if (SAMPLE) {
+        if (id == SAMPLE_WHOLE) break;  // (the loop of steps)
         ++drawn;
-        if (id & SAMPLE_WHOLE) break;  // (the loop of steps)
+        last = id;
       }
       if (s + 1 < a.n_steps) embed(id, pos + 1);
     }
@@ -634,7 +640,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
     sd->rng = *rng;
     sd->pp += drawn;
     sd->len += drawn;
-    sd->inp[0] = ired[4] & ~SAMPLE_WHOLE;
+    if (drawn > 0) sd->inp[0] = last;
   }
 done:
   if (loader) waitdma();  // no LDS-DMA may outlive the workgroup

@@ -41,19 +41,18 @@ __device__ __forceinline__ uint64_t prob_key(float p, int id) {
 // least 2^-k of the largest, for the first k whose mass passes topp (by 1e-3,
 // far more than the sums' rounding). The cut is in probabilities, so no run of
 // equal ones straddles it, and the kept prefix of the order, its cumulative
-// sums included, is that of the whole row. Only where no such cut keeps V / 8
-// ids or fewer (flat rows, topp near 1 or above) is the row sorted whole.
+// sums included, is that of the whole row. Where no such cut keeps V / 8 ids or
+// fewer (flat rows, topp near 1 or above) the row would have to be sorted whole,
+// 240 us on 256 threads against k_sample_step's 52 on 1024: SAMPLE_WHOLE is
+// returned instead, nothing drawn, and the loop ends so that the caller goes on
+// with that kernel.
 // A drawn id of the depth-12 model after 120 positions: 222 us with a launch
 // of the step and one of k_sample_step (52 us) an id, 163 in the loop, of
 // which a step with its argmax takes 137.
 constexpr int SVT = 1024;  // threads that sample_row's sums are split over
 constexpr int64_t sample_wg_aux(int V) { return 2 * V + 4 * SVT + 256; }
+constexpr int SAMPLE_WHOLE = 1 << 30;  // (no id: vocabularies are far smaller)
 
-// Sorting it whole takes 240 us here (k_sample_step, on four times the threads,
-// draws in 52): SAMPLE_WHOLE is then set in the result, and the loop ends so that
-// the caller goes on with k_sample_step (24 ids at temperature 2: 227 us an id
-// against 218 with launches alone, 374 without the way out).
-constexpr int SAMPLE_WHOLE = 1 << 30;
 template <int V>
 __device__ int sample_wg(float* pr, uint8_t* aux, const int32_t* gen, int ngen, const SampleCfg& c,
                          int64_t* state, bool comp) {
@@ -63,7 +62,6 @@ __device__ int sample_wg(float* pr, uint8_t* aux, const int32_t* gen, int ngen, 
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   uint32_t* cnt = (uint32_t*)aux;       // 16-bit counts, two a word (histories are below 2^16)
   uint64_t* keys = (uint64_t*)aux;      // [MAXC]
-  uint16_t* id16 = (uint16_t*)aux;      // [V]
   float* tot = (float*)(aux + 2 * V);   // [SVT]
   float* red = tot + SVT;               // [16]
   int* ri = (int*)(red + 16);           // [16]
@@ -224,7 +222,7 @@ __device__ int sample_wg(float* pr, uint8_t* aux, const int32_t* gen, int ngen, 
   }
   lds_barrier();
   float tau = 0.f;
-  int nc = 0;  // ids kept, 0: the whole row
+  int nc = 0;  // ids kept
 #pragma unroll
   for (int k = NK - 1; k >= 0; --k) {
     const float mass = (tot[k] + tot[8 + k]) + (tot[16 + k] + tot[24 + k]);
@@ -234,73 +232,47 @@ __device__ int sample_wg(float* pr, uint8_t* aux, const int32_t* gen, int ngen, 
       nc = (int)n;
     }
   }
-  int np = V;  // entries of the order that are used
-  if (nc > 0) {
-    int n2 = 64;
-    while (n2 < nc) n2 <<= 1;
-    if (comp) {
-      for (int i = tid; i < V; i += NT)
-        if (pr[i] >= tau) keys[atomicAdd(&ri[15], 1)] = prob_key(pr[i], i);
-      for (int i = nc + tid; i < n2; i += NT) keys[i] = 0ull;
-    }
-    lds_barrier();
-    // bitonic, descending; steps of j < 128 stay within the 128 keys that a
-    // wavefront's 64 pairs span
-    for (int k = 2; k <= n2; k <<= 1)
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        if (comp)
-          for (int q = tid; q < n2 / 2; q += NT) {
-            const int i = 2 * q - (q & (j - 1));
-            const uint64_t x = keys[i], y = keys[i + j];
-            if ((x < y) == ((i & k) == 0)) {
-              keys[i] = y;
-              keys[i + j] = x;
-            }
-          }
-        if (j >= 128 || (j == 1 && k >= 128))
-          lds_barrier();
-        else
-          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      }
-    lds_barrier();
-    np = nc;
-  } else {
-    if (comp)
-      for (int i = tid; i < V; i += NT) id16[i] = (uint16_t)i;
-    lds_barrier();
-    for (int k = 2; k <= V; k <<= 1)
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        if (comp)
-          for (int q = tid; q < V / 2; q += NT) {
-            const int i = 2 * q - (q & (j - 1));
-            const uint32_t px = __float_as_uint(pr[i]), py = __float_as_uint(pr[i + j]);
-            const uint16_t ix = id16[i], iy = id16[i + j];
-            const bool after = px < py || (px == py && ix > iy);  // x sorts after y
-            if (after == ((i & k) == 0)) {
-              pr[i] = __uint_as_float(py);
-              pr[i + j] = __uint_as_float(px);
-              id16[i] = iy;
-              id16[i + j] = ix;
-            }
-          }
-        if (j >= 128 || (j == 1 && k >= 128))
-          lds_barrier();
-        else
-          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      }
-    lds_barrier();
+  if (nc == 0) {
+    lds_barrier();  // (pr and aux are free again)
+    return SAMPLE_WHOLE;
   }
-  const bool cut_row = nc > 0;
+  int n2 = 64;
+  while (n2 < nc) n2 <<= 1;
+  if (comp) {
+    for (int i = tid; i < V; i += NT)
+      if (pr[i] >= tau) keys[atomicAdd(&ri[15], 1)] = prob_key(pr[i], i);
+    for (int i = nc + tid; i < n2; i += NT) keys[i] = 0ull;
+  }
+  lds_barrier();
+  // bitonic, descending; steps of j < 128 stay within the 128 keys that a
+  // wavefront's 64 pairs span
+  for (int k = 2; k <= n2; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      if (comp)
+        for (int q = tid; q < n2 / 2; q += NT) {
+          const int i = 2 * q - (q & (j - 1));
+          const uint64_t x = keys[i], y = keys[i + j];
+          if ((x < y) == ((i & k) == 0)) {
+            keys[i] = y;
+            keys[i + j] = x;
+          }
+        }
+      if (j >= 128 || (j == 1 && k >= 128))
+        lds_barrier();
+      else
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+  lds_barrier();
   // cumulative sums, into pr: PER entries a (sample_row) thread, 64 threads'
   // totals, then the groups of 64
-  const int ngrp = (np + 64 * PER - 1) / (64 * PER), nv = comp ? 64 * ngrp : 0;
+  const int ngrp = (nc + 64 * PER - 1) / (64 * PER), nv = comp ? 64 * ngrp : 0;
 #pragma unroll 1
   for (int v = tid; v < nv; v += NT) {
     float run = 0.f;
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
       const int i = v * PER + q;
-      run += !cut_row ? pr[i] : i < np ? __uint_as_float((uint32_t)(keys[i] >> 32)) : 0.f;
+      run += i < nc ? __uint_as_float((uint32_t)(keys[i] >> 32)) : 0.f;
       pr[i] = run;
     }
     tot[v] = run;
@@ -353,11 +325,11 @@ __device__ int sample_wg(float* pr, uint8_t* aux, const int32_t* gen, int ngen, 
   const float u = mred[4];
   int hit = 0x7fffffff;
   if (comp)
-    for (int i = tid; i < min(cut, np); i += NT)
+    for (int i = tid; i < min(cut, nc); i += NT)
       if (pr[i] >= u && i < hit) hit = i;
   hit = block_min(hit);
   hit = hit < cut ? hit : cut - 1;
-  const int id = cut_row ? 0x7fffffff - (int)(uint32_t)keys[hit] : (int)id16[hit] | SAMPLE_WHOLE;
+  const int id = 0x7fffffff - (int)(uint32_t)keys[hit];
   lds_barrier();  // (pr and aux are free again)
   return id;
 }

@@ -41,6 +41,7 @@ KERNEL_KINDS = {0: "gemm", 1: "gemv", 2: "attn_chunk", 3: "attn_decode", 4: "oth
                 5: "decode_fused"}
 FG_OPT_FUSED_DECODE = 1
 FG_OPT_FORWARD_F16 = 2
+FG_OPT_SAMPLED_IN_LOOP = 3
 
 
 FG_KV_BF16 = 1  # fg_kv_create_ex flag: bf16 K/V cache
@@ -276,6 +277,13 @@ class Model:
         buf = C.create_string_buffer(256)
         _check(_LIB.fg_get_option(self._h, FG_OPT_FUSED_DECODE, C.byref(v), buf, 256))
         return bool(v.value), buf.value.decode(errors="replace")
+
+    def sampled_in_loop(self) -> int:
+        """FG_OPT_SAMPLED_IN_LOOP: ids that the last decode_sample drew inside
+        the persistent loop."""
+        v = C.c_int32()
+        _check(_LIB.fg_get_option(self._h, FG_OPT_SAMPLED_IN_LOOP, C.byref(v), None, 0))
+        return v.value
 
     def set_forward_f16(self, enable: bool):
         """FG_OPT_FORWARD_F16: forward / eval passes of more than 128 token

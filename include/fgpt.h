@@ -307,8 +307,13 @@ int32_t fg_decode_sample(fg_model *m, fg_kv *kv, int32_t *ids, int32_t n_known, 
  * split format. 0 (the default) is the split format everywhere. Enabling it
  * makes the fp16 copy (the weight arena's size again) and fails with
  * FG_EARG when the weights exceed the fp16 range; disabling it waits for
- * the device's queued work (any stream) and frees the copy. */
-enum { FG_OPT_FUSED_DECODE = 1, FG_OPT_FORWARD_F16 = 2 };
+ * the device's queued work (any stream) and frees the copy.
+ *
+ * FG_OPT_SAMPLED_IN_LOOP (read only): how many ids the handle's last
+ * fg_decode_sample drew inside persistent launches (the others by a launch
+ * each: rows too flat for the loop's cut sort, and every id where the loop
+ * does not run). */
+enum { FG_OPT_FUSED_DECODE = 1, FG_OPT_FORWARD_F16 = 2, FG_OPT_SAMPLED_IN_LOOP = 3 };
 int32_t fg_set_option(fg_model *m, int32_t key, int32_t value);
 /* *value = the option's effective value (for FG_OPT_FUSED_DECODE: 1 when
  * the persistent decode is set up and enabled); why (nullable, len bytes)

@@ -240,6 +240,37 @@ def test_sampling_inside_the_persistent_loop(d, cfg):
     m.close()
 
 
+@pytest.mark.parametrize("d", [SMALL_MHA, Dims(n_layer=1, d_model=768, n_head=6, n_kv_head=6,
+                                               head_dim=128, vocab=8192)], ids=["1k", "8k"])
+@pytest.mark.parametrize("cfg,share", [
+    (dict(temp=0.0), 1), (dict(temp=0.02, topp=0.5), 1),     # every row has a cut that passes
+    (dict(temp=50.0, topp=0.9), 0), (dict(temp=50.0, topp=0.5, rep=1.2), 0),  # none has
+    (dict(temp=50.0, topp=1.0), 0)])                         # the loop does not run
+def test_flat_rows_are_not_sorted_in_the_loop(d, cfg, share):
+    """Ids drawn inside the persistent loop: all of a peaked run, none of a
+    flat one, whose rows go back as they are for k_sample_step to sort (48 ids:
+    the loop is tried at the first and again after 33). Either way the ids and
+    the state are those of one launch per id."""
+    m = engine.Model(d, stacks=seeded_weights(d, 9))
+    assert m.fused_decode()[0], m.fused_decode()[1]
+    prompt = uniform_ids(19, 9, d.vocab)
+    n_gen = 48
+    c, s = rope_tables(prompt.size + n_gen, d.head_dim)
+    m.set_rope(c.reshape(-1), s.reshape(-1))
+    outs = []
+    for timing in (True, False):
+        kv = m.kv(1, prompt.size + n_gen)
+        kv.step_multi(prompt[:-1], want_logits=False)
+        m.timing(timing)
+        outs.append(kv.decode_sample(prompt, n_gen, seed=4321, **cfg))
+        m.timing(False)
+        assert m.sampled_in_loop() == (0 if timing else share * n_gen)
+        assert kv.len == prompt.size + n_gen - 1
+        kv.close()
+    assert np.array_equal(outs[0][0], outs[1][0]) and outs[0][1] == outs[1][1]
+    m.close()
+
+
 def test_sample_errors(m):
     with pytest.raises(engine.FgptError):
         m.sample(np.zeros(8193, np.float32))
