@@ -2159,6 +2159,21 @@ extern "C" int32_t fg_decode_sample(fg_model* m, fg_kv* kv, int32_t* ids, int32_
 
 namespace {
 
+// Elements of an operand-layout copy: the layers' matrices and lm_head.
+size_t gemm_weight_elems(const fg_model* m) {
+  return m->w.layer_stride * m->d.L + (size_t)m->d.V * m->d.D;
+}
+
+// Every copy of the weights that the handle holds: the row-major arena, the
+// GEMMs' operand layout, the persistent decode's slices, the fp16 copy.
+int64_t weight_copies_bytes(const fg_model* m) {
+  const int64_t gemm = 2 * (int64_t)gemm_weight_elems(m);
+  int64_t n = (int64_t)m->w.bytes + gemm;
+  if (m->fused_w) n += (int64_t)FUSED_NWG * m->fl.cu_bytes;
+  if (m->w16) n += gemm;
+  return n;
+}
+
 // The fp16 copy of the GEMM weights for FG_OPT_FORWARD_F16: every bf16
 // weight times 2^k, k the largest integer <= 15 with max|w| 2^k <= 32768,
 // so the copy holds each weight exactly unless it is below ~2^-(24+k-7)
@@ -2169,7 +2184,7 @@ int32_t ensure_w16(fg_model* m) {
   while (k > -15 && m->wmax * std::ldexp(1.0f, k) > 32768.f) --k;
   if (m->wmax * std::ldexp(1.0f, k) > 32768.f)
     return seterr(FG_EARG, "weights up to %g exceed what fp16 holds", (double)m->wmax);
-  const size_t n = m->w.layer_stride * m->d.L + (size_t)m->d.V * m->d.D;  // layers + lm_head
+  const size_t n = gemm_weight_elems(m);
   HIPCHK(hipMalloc((void**)&m->w16, n * 2));  // (the arena's offsets, in the operand layout)
   m->w16_scale = std::ldexp(1.0f, k);
   m->w16_inv = std::ldexp(1.0f, -k);
@@ -2268,7 +2283,13 @@ extern "C" int32_t fg_timing_read(fg_model* m, int32_t kind, int64_t* launches, 
 
 extern "C" int32_t fg_model_bytes(const fg_model* m, int64_t* weight_bytes, int64_t* work_bytes) {
   if (!m) return seterr(FG_EARG, "NULL argument");
-  if (weight_bytes) *weight_bytes = (int64_t)m->w.bytes * (m->w16 ? 2 : 1);  // + the fp16 copy
-  if (work_bytes) *work_bytes = m->work_bytes;
+  if (weight_bytes) *weight_bytes = weight_copies_bytes(m);
+  if (work_bytes) {
+    int64_t n = m->work_bytes + m->samp_bytes + 4 * m->pos_cap + 4;  // (+ the overflow flag)
+    n += 2 * 4 * m->split_kv_elems + 4 * m->attn_floats;
+    n += (int64_t)2 * m->rope_cap * (m->d.hd / 2) * 4;
+    if (m->fused_w) n += 8 * m->fl.slots + 4 * (1 + FUSED_NX);
+    *work_bytes = n;
+  }
   return FG_OK;
 }

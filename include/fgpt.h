@@ -305,7 +305,7 @@ int32_t fg_decode_sample(fg_model *m, fg_kv *kv, int32_t *ids, int32_t n_known, 
  * instead of 2 (linears) or 3 (attention). Logits move by ~4e-4 x max|logit|
  * instead of ~5e-6; passes that fill a KV cache (fg_step_multi) keep the
  * split format. 0 (the default) is the split format everywhere. Enabling it
- * makes the fp16 copy (the weight arena's size again) and fails with
+ * makes the fp16 copy (the weights again, but for the embedding) and fails with
  * FG_EARG when the weights exceed the fp16 range; disabling it waits for
  * the device's queued work (any stream) and frees the copy.
  *
@@ -347,8 +347,14 @@ int32_t fg_timing(fg_model *m, int32_t enable);
 int32_t fg_timing_read(fg_model *m, int32_t kind, int64_t *launches, double *ms, double *flops,
                        double *bytes);
 
-/* Bytes of HBM the handle holds (weights, workspace, tables). Diagnostic,
- * the counterpart of gpublas_count / gpublas_bufs (gpu_shim.cpp:172-186). */
+/* Bytes of HBM the handle holds; KV caches hold their own. weight_bytes: every
+ * copy of the weights: the bf16 arena, the GEMMs' operand layout of its layers
+ * and lm_head (as large again but for the embedding), the persistent decode's
+ * copy where FG_OPT_FUSED_DECODE is available (likewise), and the fp16 copy
+ * while FG_OPT_FORWARD_F16 is on (likewise): up to four times the weights.
+ * work_bytes: workspace, attention planes and scratch, exchange slots, tables.
+ * Diagnostic, the counterpart of gpublas_count / gpublas_bufs
+ * (gpu_shim.cpp:172-186). */
 int32_t fg_model_bytes(const fg_model *m, int64_t *weight_bytes, int64_t *work_bytes);
 
 #ifdef __cplusplus

@@ -9,6 +9,7 @@ own top-2 margin is below twice the largest logit error measured, the
 bound under which a flip is possible at all. Passes of 128 rows or fewer,
 cached steps and chunked prefill keep the split format bit for bit.
 """
+import ctypes as C
 import json
 import os
 
@@ -66,12 +67,46 @@ def test_option_round_trip(d12):
     m.set_forward_f16(True)
     assert m.forward_f16() is True
     wb1, _ = m.bytes()
-    assert wb1 == 2 * wb0  # the fp16 copy has the arena's size
+    assert wb1 - wb0 == 2 * (sum(w[k].size for k in w) - w["wte"].size)  # all but the embedding
     m.set_forward_f16(False)
     assert m.forward_f16() is False
     assert m.bytes()[0] == wb0  # the copy is released with the option
     with pytest.raises(engine.FgptError):
         engine._check(engine._LIB.fg_set_option(m._h, 99, 1))
+
+
+@pytest.mark.parametrize("d", [D12, Dims(n_layer=4, d_model=1024, n_head=8, n_kv_head=2, head_dim=128,
+                                         vocab=8192)], ids=["persistent", "per-kernel"])
+def test_model_bytes_are_what_the_device_gave(d):
+    """bytes() against the device's free memory: every copy of the weights
+    (arena, operand layout, the persistent decode's, fp16) and the workspace.
+    hipMalloc rounds an allocation up to 2 MiB at most, and there are about
+    30: 60 MiB; the smallest copy here takes 100."""
+    hip = C.CDLL("libamdhip64.so.7")  # (the runtime that libfgpt.so is linked against)
+    w = seeded_weights(d, 5)
+    engine.Model(d, stacks=w).close()  # (code objects, context, staging)
+    ids = uniform_ids(3, 2 * 700, d.vocab)
+
+    def free():
+        n, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipDeviceSynchronize() == 0
+        assert hip.hipMemGetInfo(C.byref(n), C.byref(total)) == 0
+        return n.value
+
+    f0 = free()
+    m = engine.Model(d, stacks=w)
+    m.set_rope(*tables(d, 800))
+    last = 0
+    for step in ("weights", "fp16 copy", "a pass"):
+        if step == "fp16 copy":
+            m.set_forward_f16(True)
+        if step == "a pass":
+            m.forward(ids, 2, 700)
+        held, said = f0 - free(), sum(m.bytes())
+        print(step, "held", held, "reported", m.bytes(), flush=True)
+        assert said > last and -(4 << 20) <= held - said <= (60 << 20), step
+        last = said
+    m.close()
 
 
 def test_prefill_d12_T2048_f16_vs_oracle(d12):
