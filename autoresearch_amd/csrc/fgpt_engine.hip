@@ -424,12 +424,8 @@ int32_t upload_weights(fg_model* m, const float* const st[8]) {
 }
 
 void free_work(fg_model* m) {
-  Work& ws = m->ws;
-  void* ptrs[] = {ws.x, ws.q, ws.ao, ws.h, ws.logits, ws.ids, ws.tgt, ws.nll, ws.stat, ws.amax,
-                  ws.xs, ws.aos, ws.hs, ws.fkv, ws.ssq, ws.nllp, m->qs};
-  for (void* p : ptrs)
-    if (p) (void)hipFree(p);
-  ws = Work();
+  if (m->ws.slab) (void)hipFree(m->ws.slab);
+  m->ws = Work();
   m->qs = nullptr;
   m->work_bytes = 0;
 }
@@ -556,31 +552,47 @@ int32_t ensure_work(fg_model* m, int64_t rows) {
   free_work(m);
   const Dims& d = m->d;
   Work& ws = m->ws;
-  int64_t total = 0;
-  auto alloc = [&](void** p, int64_t bytes) -> int32_t {
-    total += bytes;
-    HIPCHK(hipMalloc(p, (size_t)bytes));
-    return dev_zero(m, *p, (size_t)bytes);
-  };
-  RCCHK(alloc((void**)&ws.x, rows * d.D * 4));
-  RCCHK(alloc((void**)&ws.q, rows * d.qd() * 4));
-  RCCHK(alloc((void**)&ws.ao, rows * d.qd() * 4));
-  RCCHK(alloc((void**)&ws.h, rows * d.dff * 4));
-  RCCHK(alloc((void**)&ws.logits, rows * d.V * 4));
-  RCCHK(alloc((void**)&ws.ids, rows * 4));
-  RCCHK(alloc((void**)&ws.tgt, rows * 4));
-  RCCHK(alloc((void**)&ws.nll, rows * 4));
-  RCCHK(alloc((void**)&ws.stat, rows * 4));
-  RCCHK(alloc((void**)&ws.amax, rows * 4));
-  RCCHK(alloc((void**)&m->qs, rows * d.qd() * 2 * 2));
   const int64_t prow = tile_rows(rows);  // (operand planes hold whole 16-row tiles)
-  RCCHK(alloc((void**)&ws.xs, prow * d.D * 2 * 2));
-  RCCHK(alloc((void**)&ws.aos, prow * d.qd() * 2 * 2));
-  RCCHK(alloc((void**)&ws.hs, prow * d.dff * 2 * 2));
-  RCCHK(alloc((void**)&ws.fkv, std::min(rows, attn_rows_most(d)) * d.kvd() * 2 * 4));
-  RCCHK(alloc((void**)&ws.ssq, rows * (d.D / 16) * 4));
-  if (d.V % 256 == 0) RCCHK(alloc((void**)&ws.nllp, rows * (d.V / NLL_GROUP_COLS) * 2 * 4));
-  HIPCHK(hipStreamSynchronize(m->stream));  // the clears, before any caller stream's work
+  const int64_t nrow = d.V % 256 == 0 ? std::min<int64_t>(rows, GEMM_NLL_ROWS) : 0;
+  struct Part {
+    void** p;
+    int64_t bytes;
+  };
+  const Part parts[] = {
+      {(void**)&ws.x, rows * d.D * 4},
+      {(void**)&ws.q, rows * d.qd() * 4},
+      {(void**)&ws.ao, rows * d.qd() * 4},
+      {(void**)&ws.h, rows * d.dff * 4},
+      {(void**)&ws.logits, rows * d.V * 4},
+      {(void**)&ws.ids, rows * 4},
+      {(void**)&ws.tgt, rows * 4},
+      {(void**)&ws.nll, rows * 4},
+      {(void**)&ws.stat, rows * 4},
+      {(void**)&ws.amax, rows * 4},
+      {(void**)&m->qs, rows * d.qd() * 2 * 2},
+      {(void**)&ws.xs, prow * d.D * 2 * 2},
+      {(void**)&ws.aos, prow * d.qd() * 2 * 2},
+      {(void**)&ws.hs, prow * d.dff * 2 * 2},
+      {(void**)&ws.ssq, gemm_ssq_floats(rows, d.D) * 4},
+      {(void**)&ws.nllp, nrow * (d.V / NLL_GROUP_COLS) * 2 * 4},
+  };
+  // One allocation for all of them: an allocation and its clear cost the host
+  // 60-350 us each, most after a handle of the process was closed, and a new
+  // handle's first pass pays for all (T = 2048, d12, handles opened and closed in
+  // turn, host us of that pass, medians: 1590 fp16 and 1860 split with one each,
+  // 844 and 950 with one for all).
+  constexpr int64_t ALIGN = 1 << 16;
+  auto room = [](int64_t bytes) { return (bytes + ALIGN - 1) / ALIGN * ALIGN; };
+  int64_t total = 0;
+  for (const Part& p : parts) total += room(p.bytes);
+  HIPCHK(hipMalloc((void**)&ws.slab, (size_t)total));
+  RCCHK(dev_zero(m, ws.slab, (size_t)total));
+  HIPCHK(hipStreamSynchronize(m->stream));  // the clear, before any caller stream's work
+  char* at = ws.slab;
+  for (const Part& p : parts) {
+    if (p.bytes > 0) *p.p = at;
+    at += room(p.bytes);
+  }
   ws.rows = rows;
   m->work_bytes = total;
   m->gen++;
@@ -755,9 +767,10 @@ void layer_stack(fg_model* m, hipStream_t s, const int32_t* ids, int B, int T, i
     const bool one = (T == 1 || o.rows_single) && lk != nullptr;
     const bool last = o.last_only && l == d.L - 1;  // (queries: one row a sequence, from q)
     const int npos = npos_pad(pos0 + T);
-    if (few && !kc) {  // (gpt_forward: the layer's keys and values in scratch rows)
-      a.kc = ws.fkv;
-      a.vc = ws.fkv + (int64_t)rows * d.kvd();
+    if (few && !kc) {  // (gpt_forward: the layer's keys and values in scratch rows: in
+                       // h [rows][4 D], which only fc and proj2 use)
+      a.kc = ws.h;
+      a.vc = ws.h + (int64_t)rows * d.kvd();
     }
     if (!one && !few && !last) {
       a.qs = m->qs;

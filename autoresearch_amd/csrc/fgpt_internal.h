@@ -90,6 +90,7 @@ constexpr int NLL_GROUP_COLS = 64;
 // Activation workspace for up to `rows` token rows.
 struct Work {
   int64_t rows = 0;
+  char* slab = nullptr;     // the allocation that all of these lie in
   float* x = nullptr;       // residual stream [rows][D]
   float* q = nullptr;       // rotated queries [rows][H*hd]
   float* ao = nullptr;      // attention output [rows][H*hd]
@@ -102,15 +103,13 @@ struct Work {
   int32_t* amax = nullptr;  // [rows]
   // the MFMA path's activations in the split format (hi plane, then lo
   // plane; each in the GEMM operand layout, tile_at, its rows padded to 16)
-  // and the residual's per-row partial sums of squares, up to [rows][D/16]
+  // and the residual's per-row partial sums of squares (gemm_ssq_floats)
   uint16_t* xs = nullptr;   // residual [rows][D]
   uint16_t* aos = nullptr;  // attention output [rows][H*hd]
   uint16_t* hs = nullptr;   // relu2(fc) [rows][4D]
-  // one layer's key, then value rows [rows][KH*hd] of a forward without a
-  // cache that attends from rows (attn_rows_fits)
-  float* fkv = nullptr;
   float* ssq = nullptr;
-  float* nllp = nullptr;    // lm_head's log-sum-exp partials [rows][V/NLL_GROUP_COLS][2]
+  // lm_head's log-sum-exp partials [rows up to GEMM_NLL_ROWS][V/NLL_GROUP_COLS][2]
+  float* nllp = nullptr;
 };
 
 struct KVCacheDev {
@@ -205,15 +204,18 @@ void launch_gemv(hipStream_t s, GemvEpi epi, const GemvArgs& a);
 // MFMA GEMM, C[M][N] = epi(rowscale * (A[M][K] . W[N][K]^T)), A in the
 // split format (xs), W bf16, fp32 accumulation. K must be a multiple of 128.
 void launch_gemm(hipStream_t s, GemvEpi epi, const GemvArgs& a);
-// Number of ssq_out partials per row that a RESID GEMM of M x N x K writes
-// (at most N / 16).
+// Number of ssq_out partials per row that a RESID GEMM of M x N x K writes (at
+// most N / 16, past the few-row GEMM's row range N / 64), and the floats that
+// hold them for any pass of up to M rows.
 int gemm_ssq_parts(int64_t M, int N, int K);
+int64_t gemm_ssq_floats(int64_t M, int N);
 // The same GEMM for few token rows (kern_rows.hip); gemm_rows_tile: the tile
 // it takes for M x N outputs, in units of 16 rows and columns (tm = 0: the
 // pass is not its).
 struct RowsTile {
   int tm, tn;
 };
+constexpr int64_t ROWS_MAX_M = 256;
 RowsTile gemm_rows_tile(int64_t M, int N);
 void launch_gemm_rows(hipStream_t s, GemvEpi epi, const GemvArgs& a, const int32_t* d_pos);
 // dst = the GEMM operand layout (tile_at) of the row-major matrix src [N][K].
@@ -252,7 +254,6 @@ void launch_attn_mfma(hipStream_t s, const Dims& d, const uint16_t* qs, const ui
 // queries q [B*T][H*hd] and the cache rows themselves ([B][maxT][KH*hd], fp32
 // or bf16 with kv16): no planes, no scratch, no merge launch.
 bool attn_rows_fits(const Dims& d, bool kv16, int B, int T, int pos0);
-int64_t attn_rows_most(const Dims& d);  // the most token rows it holds for (fp32 rows)
 void launch_attn_rows(hipStream_t s, const Dims& d, const float* q, const void* kc, const void* vc,
                       bool kv16, int B, int T, int pos0, int maxT, float* y, uint16_t* ys,
                       int64_t ys_plane, uint32_t* pos_cnt = nullptr);
@@ -313,7 +314,9 @@ void launch_nll(hipStream_t s, const float* logits, const int32_t* tgt, int64_t 
 void launch_nll_parts(hipStream_t s, const float* tlogit, const float* parts, const int32_t* tgt,
                       int64_t rows, int V, float* out);
 // Whether an lm_head GEMM of M rows over a vocabulary of N writes the
-// log-sum-exp partials when asked (f16: the single-term pass).
+// log-sum-exp partials when asked (f16: the single-term pass): never past
+// GEMM_NLL_ROWS.
+constexpr int64_t GEMM_NLL_ROWS = 4096;
 bool gemm_store_nll(int64_t M, int N, bool f16);
 
 // ---- greedy speculative decoding

@@ -872,7 +872,6 @@ bool attn_rows_fits(const Dims& d, bool kv16, int B, int T, int pos0) {
   const int keys = d.H == d.KH ? 2560 : 1200;
   return wg <= ROWS_MAX_WG && pos0 + T <= (wg > cu_count() ? keys / 2 : keys);
 }
-int64_t attn_rows_most(const Dims& d) { return ROWS_MAX_WG / d.H * RQ; }
 
 template <int HD, class KT>
 static void launch_attn_rows_t(hipStream_t s, const AttnRowsArgs& p) {

@@ -30,6 +30,8 @@
 // staged through LDS 64 rows at a time so each thread owns a column pair
 // (coalesced stores; a QKV rotation pair in one thread). The host picks the
 // tile per shape (launch_tile) so that one round of tiles covers the CUs.
+#include <algorithm>
+
 #include "fgpt_internal.h"
 #include "kern_common.h"
 #include "kern_epi.h"
@@ -908,7 +910,7 @@ int cu_count() {
 // 387 us against 271 + 94. Whole pass with the tiles above: 2048 rows, logits
 // and cross-entropy, fp16 1283 -> 1246 us.
 bool gemm_store_nll(int64_t M, int N, bool f16) {
-  return M <= 4096 && gemm_rows_tile(M, N).tm == 0 && store_256(M, N, f16);
+  return M <= GEMM_NLL_ROWS && gemm_rows_tile(M, N).tm == 0 && store_256(M, N, f16);
 }
 
 // RESID: one sum-of-squares partial per row and N tile.
@@ -919,6 +921,10 @@ int gemm_ssq_parts(int64_t M, int N, int K) {
   if (resid_160(M, N, K)) return N / 160;
   if (resid_128(M, N)) return N / 128;
   return N / tile_n(M, N);
+}
+
+int64_t gemm_ssq_floats(int64_t M, int N) {
+  return std::max(std::min(M, ROWS_MAX_M) * (N / 16), M * (N / 64));
 }
 
 void launch_gemm_pos(hipStream_t s, GemvEpi epi, const GemvArgs& a, const int32_t* d_pos) {

@@ -278,7 +278,6 @@ __global__ __launch_bounds__(256) void k_tile_weights(const bf16_t* __restrict__
 // past one round the next larger tile moves fewer bytes: M = 64, N = 3072 on
 // 192 blocks of 32x32 4.5 us, on 384 of 16x32 5.9, on 96 of 32x64 5.0).
 RowsTile gemm_rows_tile(int64_t M, int N) {
-  constexpr int64_t ROWS_MAX_M = 256;
   if (M > ROWS_MAX_M) return {0, 0};
   static const RowsTile tiles[] = {{1, 1}, {1, 2}, {2, 2}, {2, 4}, {4, 4}};
   for (const RowsTile& t : tiles) {

@@ -149,3 +149,24 @@ def test_forward_tiles(d, B, T):
         alone = m.eval_bpb(ids, np.ones(d.vocab, np.int32), batch=B, want_nll=True)["nll"]
         assert np.array_equal(alone.reshape(-1), nll.reshape(-1))
     m.close()
+
+
+@pytest.mark.parametrize("d,T", [(SMALL, 600), (VOCAB, 1500), (TINY, 40)])
+def test_workspace_is_what_a_pass_uses(d, T):
+    """A new handle's first pass allocates and clears its workspace: fp32 rows
+    and logits, the operand planes, the row norms' partial sums (a 16th of
+    d_model up to 256 rows, a 64th past them), lm_head's partials, and nothing
+    a pass of these rows never touches; 16 parts, rounded up to 64 KiB each. (A
+    chunk whose attention reads the cache rows has no other scratch.)"""
+    m, w, c, s = model(d, T)
+    kv = m.kv(1, T)
+    base = m.bytes()[1]
+    kv.step_multi(uniform_ids(71, T, d.vocab).reshape(1, T), want_logits=False)
+    D, qd, V = d.d_model, d.n_head * d.head_dim, d.vocab
+    rows, prow = T, (T + 15) // 16 * 16
+    need = 4 * rows * (D + 2 * qd + 4 * D + V + 5) + 4 * rows * qd + 4 * prow * (D + qd + 4 * D)
+    need += 4 * max(min(rows, 256) * D // 16, rows * D // 64) + 8 * rows * V // 64
+    said = m.bytes()[1] - base
+    assert need <= said <= need + 16 * 65536, (need, said)
+    kv.close()
+    m.close()
