@@ -2104,6 +2104,7 @@ extern "C" int32_t fg_decode_sample(fg_model* m, fg_kv* kv, int32_t* ids, int32_
   // the persistent launches' error flag, cleared once: every launch leaves its
   // failure in it until it is read
   if (fused) HIPCHK(hipMemsetAsync(m->fused_err, 0, 4, s));
+  bool ended = false;  // the loop drew the last id: h and the error flag are read
   for (int single = in_loop ? 0 : total, next = 32; fused && done < total;) {
     if (single == 0) {
       h->pp = n_known + done;
@@ -2124,6 +2125,7 @@ extern "C" int32_t fg_decode_sample(fg_model* m, fg_kv* kv, int32_t* ids, int32_
       rc = fused_error(*herr);
       if (rc != FG_OK) return failed(rc);
       m->loop_ids += h->pp - n_known - done;
+      ended = h->pp == n_total;
       done = std::min(h->pp - n_known + 1, total);
       single = next;
       next *= 2;
@@ -2152,11 +2154,11 @@ extern "C" int32_t fg_decode_sample(fg_model* m, fg_kv* kv, int32_t* ids, int32_
     }
     done += run;
   }
-  HIPCHK(hipMemcpyAsync(h, kv->d_smp, sizeof *h, hipMemcpyDeviceToHost, s));
+  if (!ended) HIPCHK(hipMemcpyAsync(h, kv->d_smp, sizeof *h, hipMemcpyDeviceToHost, s));
   HIPCHK(hipMemcpyAsync(ids + n_known, kv->d_sids + n_known, (size_t)total * 4,
                         hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
-  if (fused) {
+  if (fused && !ended) {
     const int32_t rc = fused_check(m);
     if (rc != FG_OK) {
       kv->len = n_known - 1;
