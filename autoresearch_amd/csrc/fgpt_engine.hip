@@ -1244,8 +1244,11 @@ extern "C" int32_t fg_kv_create_ex(fg_model* m, int32_t B, int32_t maxT, int32_t
   if (e == hipSuccess) e = hipMalloc((void**)&kv->d_dcnt, cnt_bytes);
   // a step's ids and logits on the host, where a batch's are small
   const size_t out_bytes = ((size_t)(B + 3) / 4 * 4 + (size_t)B * m->d.V) * 4;
-  if (e == hipSuccess && out_bytes <= ((size_t)1 << 20))
-    e = hipHostMalloc((void**)&kv->h_out, out_bytes, hipHostMallocDefault);
+  if (e == hipSuccess && out_bytes <= ((size_t)1 << 20) &&
+      hipHostMalloc((void**)&kv->h_out, out_bytes, hipHostMallocDefault) != hipSuccess) {
+    kv->h_out = nullptr;  // (no pinned memory left: steps copy instead)
+    (void)hipGetLastError();
+  }
   // zeroed on the handle's stream, and finished before the cache is handed
   // out (its first user may be a caller's stream); the reference's callers
   // zero their caches too
