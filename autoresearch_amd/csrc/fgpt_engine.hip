@@ -1554,12 +1554,13 @@ int32_t fused_launch(fg_model* m, fg_kv* kv, const int32_t* d_id0, int len0, int
     flops += wbytes + (double)d.L * 4 * d.hd * d.H * len;
   }
   // FGPT_FUSED_TRACE=<file>: append the phase timestamps of one step (the
-  // second, when there is one) of every workgroup to <file> (diagnostic)
+  // second, when there is one; a sampled loop that ended before it leaves
+  // nothing) of every workgroup to <file> (diagnostic)
   const char* tpath = getenv("FGPT_FUSED_TRACE");
   const size_t tn = (size_t)FUSED_NWG * (d.L + 1) * 32;
   a.trace = nullptr;  // (null: the kernel built without timestamps)
   a.trace_step = n_steps > 1 ? 1 : 0;
-  if (tpath && *tpath && !host_sd) {
+  if (tpath && *tpath) {
     HIPCHK(hipMalloc((void**)&a.trace, tn * 8));
     HIPCHK(hipMemsetAsync(a.trace, 0, tn * 8, s));
   }
@@ -1572,7 +1573,7 @@ int32_t fused_launch(fg_model* m, fg_kv* kv, const int32_t* d_id0, int len0, int
     if (e == hipSuccess) e = hipMemcpyAsync(ht.data(), a.trace, tn * 8, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     (void)hipFree(a.trace);
-    if (e == hipSuccess) {
+    if (e == hipSuccess && std::any_of(ht.begin(), ht.end(), [](uint64_t t) { return t != 0; })) {
       FILE* fp = fopen(tpath, "ab");
       if (fp) {
         const int32_t hdr[4] = {FUSED_NWG, d.L + 1, 32 | (m->fl.kind << 16), n_steps};

@@ -560,9 +560,11 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_fused_decode(FusedArgs a) {
                 *stop = 1;
           }
           lds_barrier();
+          mark(s, L, 4);
           if (!*stop) {
             const int id = sample_wg<V>(pr, (uint8_t*)(pr + V), a.ids_out, s + a.n_gen, a.cfg, rng,
                                         comp);
+            mark(s, L, 5);
             if (wv == 0 && lane < FUSED_LMC)
               slot_put_dev(SMP + V + lane, __int_as_float(id), ep + 1);
             if (tid == 0) ired[4] = id;
@@ -746,9 +748,10 @@ static hipError_t launch_shape(hipStream_t s, const FusedLayout& f, const FusedA
   if (f.slice != Sh::SLICE || f.lmb != Sh::LMB || f.wbuf != Sh::WBUF || f.wf != Sh::WF ||
       f.off_lm != Sh::OFF_LM || f.off_ap != Sh::OFF_AP || f.slots != Sh::SLOTS)
     return hipErrorInvalidValue;  // (host and device layouts disagree)
-  const void* k = a.sd      ? (const void*)k_fused_decode<Sh, false, true>
-                  : a.trace ? (const void*)k_fused_decode<Sh, true, false>
-                            : (const void*)k_fused_decode<Sh, false, false>;
+  const void* k = a.sd ? (a.trace ? (const void*)k_fused_decode<Sh, true, true>
+                                  : (const void*)k_fused_decode<Sh, false, true>)
+                       : (a.trace ? (const void*)k_fused_decode<Sh, true, false>
+                                  : (const void*)k_fused_decode<Sh, false, false>);
   hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)f.lds_bytes);
   if (e != hipSuccess) return e;
   FusedArgs aa = a;

@@ -1,11 +1,12 @@
 """Phase timings of the persistent B=1 decode loop (kern_fused.hip).
 
-With FGPT_FUSED_TRACE=<file> set, fg_decode_greedy's persistent launch
-appends one record per call to <file>: a header of four int32 (workgroups,
-pseudo-layers L+1, slots per layer 32 with the kernel's kind in bits 16 and
-up, steps) and then, for one step (the second of the call when it has two or
-more), per workgroup and layer, 32 uint64 device-clock stamps (100 MHz,
-s_memrealtime; 0 = not taken). Stamp k of a layer marks, for the kernel with
+With FGPT_FUSED_TRACE=<file> set, every persistent launch (fg_decode_greedy's,
+fg_decode_sample's loops and single steps) appends one record to <file>: a
+header of four int32 (workgroups, pseudo-layers L+1, slots per layer 32 with
+the kernel's kind in bits 16 and up, steps) and then, for one step (the second
+of the launch when it has two or more; a sampled loop that ended before it
+leaves no record), per workgroup and layer, 32 uint64 device-clock stamps (100
+MHz, s_memrealtime; 0 = not taken). Stamp k of a layer marks, for the kernel with
 one KV head per query head (kern_fused.hip, kind 0):
 
     0  layer start (after the barrier that opens the layer)
@@ -37,7 +38,9 @@ and for the grouped-KV kernel (kern_fused_gqa.hip, kind 1):
 
 For the lm_head pseudo-layer: 1 logits + candidates, 2 the argmax exchanged,
 3 barrier B6 (kind 0; kind 1: 0 rows landed, 1 logits + candidates, 2 the
-argmax exchanged, 3 the barrier after it).
+argmax exchanged, 3 the barrier after it). In a loop that draws its ids, 2 is
+the id received, and workgroup 0, which draws, has 4 the row gathered, 5 the id
+drawn.
 
     python -m autoresearch_amd.trace FILE [--json]
 """
@@ -100,7 +103,7 @@ def summary(t: np.ndarray, kind: int = 0) -> dict:
     out["layer_start_us"] = ls
     out["layer_us_mean"] = float(np.diff(ls[:L]).mean()) if L > 1 else None
     lm = {}
-    for k in (1, 2, 3):
+    for k in (1, 2, 3, 4, 5):
         v = t[:, L, k]
         ok = v > 0
         if ok.any():

@@ -331,8 +331,10 @@ int32_t fg_sync(fg_model *m);
 /* Kernel timing, the device-side counterpart of chat_text --stats
  * (src/app/chat_text.f90:250-282,465-468). With timing on, every launch the
  * handle makes outside graph capture (fg_decode_greedy then runs its steps
- * eagerly) is bracketed by HIP events on the stream it runs on, and tagged
- * with its kernel kind and its algorithmic flops and HBM bytes. Enabling or
+ * eagerly, and fg_decode_sample draws every id by a launch of its own, not
+ * inside the persistent loop: FGPT_FUSED_TRACE shows that loop's phases) is
+ * bracketed by HIP events on the stream it runs on, and tagged with its kernel
+ * kind and its algorithmic flops and HBM bytes. Enabling or
  * disabling clears the records. fg_timing_read sums one kind. */
 enum {
   FG_K_GEMM = 0,        /* MFMA GEMM (prefill, batched decode linears)   */

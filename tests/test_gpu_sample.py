@@ -12,7 +12,7 @@ stepping the engine one position at a time with the oracle choosing ids.
 import numpy as np
 import pytest
 
-from autoresearch_amd import engine
+from autoresearch_amd import engine, trace
 from autoresearch_amd.weights import Dims, rope_tables, seeded_weights, uniform_ids
 from oracle import sample as S
 
@@ -268,6 +268,36 @@ def test_flat_rows_are_not_sorted_in_the_loop(d, cfg, share):
         assert kv.len == prompt.size + n_gen - 1
         kv.close()
     assert np.array_equal(outs[0][0], outs[1][0]) and outs[0][1] == outs[1][1]
+    m.close()
+
+
+def test_trace_of_a_sampled_loop(tmp_path, monkeypatch):
+    """FGPT_FUSED_TRACE on sampled decoding: one record of the loop's second
+    step, with the draw's stamps from workgroup 0; from flat rows, whose loop
+    ends at its first, one for each of the single launches."""
+    d = SMALL_MHA
+    m = engine.Model(d, stacks=seeded_weights(d, 9))
+    prompt = uniform_ids(19, 9, d.vocab)
+    c, s = rope_tables(prompt.size + 6, d.head_dim)
+    m.set_rope(c.reshape(-1), s.reshape(-1))
+    for name, cfg, n in (("peaked", dict(temp=0.02, topp=0.5), 1), ("flat", dict(temp=50.0, topp=0.9), 5)):
+        p = tmp_path / name
+        kv = m.kv(1, prompt.size + 6)
+        kv.step_multi(prompt[:-1], want_logits=False)
+        monkeypatch.setenv("FGPT_FUSED_TRACE", str(p))
+        kv.decode_sample(prompt, 6, seed=5, **cfg)
+        monkeypatch.delenv("FGPT_FUSED_TRACE")
+        kv.close()
+        recs = trace.read(str(p))
+        assert len(recs) == n and all(kind == 0 for kind, _ in recs)
+        t = recs[0][1]
+        head = t[0, d.n_layer]  # workgroup 0's lm_head stamps
+        assert head[0] > 0 and np.all(t[:, d.n_layer, 2] > 0)
+        if name == "peaked":
+            assert head[0] < head[1] < head[4] < head[5] <= head[2]
+            assert {4, 5} <= set(trace.summary(t)["lm_head_us"])
+        else:
+            assert head[4] == head[5] == 0
     m.close()
 
 
