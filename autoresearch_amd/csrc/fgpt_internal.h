@@ -203,7 +203,9 @@ void launch_gemv(hipStream_t s, GemvEpi epi, const GemvArgs& a);
 
 // MFMA GEMM, C[M][N] = epi(rowscale * (A[M][K] . W[N][K]^T)), A in the
 // split format (xs), W bf16, fp32 accumulation. K must be a multiple of 128.
-void launch_gemm(hipStream_t s, GemvEpi epi, const GemvArgs& a);
+// d_pos (nullable): the first position, read on the device (a captured step
+// replays at successive positions).
+void launch_gemm_pos(hipStream_t s, GemvEpi epi, const GemvArgs& a, const int32_t* d_pos);
 // Number of ssq_out partials per row that a RESID GEMM of M x N x K writes (at
 // most N / 16, past the few-row GEMM's row range N / 64), and the floats that
 // hold them for any pass of up to M rows.
@@ -263,10 +265,9 @@ void launch_split_cache(hipStream_t s, const Dims& d, const void* kc, const void
                         int B, int maxT, int n, int npos, int64_t kv_plane, uint16_t* ks,
                         uint16_t* vt);
 
-// Variants whose position / cache length comes from device memory (so a
-// captured decode step replays at successive positions).
+// The GEMV with its position from device memory (so a captured decode step
+// replays at successive positions).
 void launch_gemv_pos(hipStream_t s, GemvEpi epi, const GemvArgs& a, const int32_t* d_pos);
-void launch_gemm_pos(hipStream_t s, GemvEpi epi, const GemvArgs& a, const int32_t* d_pos);
 // Single-query attention over the cache: q [B*qpr][H][hd] -> y [B*qpr][H*hd]
 // (or its split format in ys). Query row j of sequence b (row b*qpr + j)
 // sits at position len-1+j of cache b and sees positions 0..len-1+j: qpr

@@ -17,7 +17,7 @@
 // comes from per-row sums of squares of the fp32 values, also written by
 // the producer (one partial per producer N tile, summed here in order).
 //
-// Pipeline: NST stages of BK-wide K slices (BK = 32, 64 or 128) in LDS,
+// Pipeline: NST stages of BK-wide K slices (BK = 32 or 64) in LDS,
 // filled by global_load_lds_dwordx4 (memory -> LDS without registers),
 // NST-1 slices in flight while the MFMAs consume the oldest. Both operands
 // are stored in 1 KB tiles of 16 rows x 32 K (tile_at), so each DMA reads 1 KB
@@ -497,8 +497,7 @@ __device__ __forceinline__ void frag_mma(const Frag<WM, WN>& f, f32x16_t (&acc)[
 }
 
 template <int EPI, int NWM, int NWN, int WM, int WN, int NST, bool P16 = false, int BK = 32>
-__global__ __launch_bounds__(64 * NWM * NWN) void k_gemm2(GemvArgs a,
-                                                         const int32_t* __restrict__ d_pos) {
+__global__ __launch_bounds__(64 * NWM * NWN) void k_gemm2(GemvArgs a) {
   static_assert(EPI == GV_RELU2 || EPI == GV_STORE, "register epilogues");
   constexpr bool TR = EPI == GV_RELU2;
   constexpr int BM = NWM * WM * 32, BN = NWN * WN * 32;
@@ -664,15 +663,14 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm2(GemvArgs a,
 }
 
 template <int EPI, int NWM, int NWN, int WM, int WN, int NST, bool P16, int BK = 32>
-void launch_cfg2(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
+void launch_cfg2(hipStream_t s, const GemvArgs& a) {
   constexpr int BM = NWM * WM * 32, BN = NWN * WN * 32;
   constexpr size_t lds = (size_t)NST * ((P16 ? 1 : 2) * BM + BN) * 2 * BK;
   static_assert(lds + BM * sizeof(float) <= 160 * 1024, "tile exceeds the LDS");
   static std::atomic<uint64_t> attr{0};
   raise_lds_once((const void*)k_gemm2<EPI, NWM, NWN, WM, WN, NST, P16, BK>, lds, &attr);
   const dim3 g(a.N / BN, (unsigned)((a.M + BM - 1) / BM));
-  FG_LAUNCH((k_gemm2<EPI, NWM, NWN, WM, WN, NST, P16, BK>), g, dim3(64 * NWM * NWN), lds, s, a,
-                     d_pos);
+  FG_LAUNCH((k_gemm2<EPI, NWM, NWN, WM, WN, NST, P16, BK>), g, dim3(64 * NWM * NWN), lds, s, a);
 }
 
 template <int EPI, int BM, int BN, int NWM, int NWN, int BK, int NST, int KG, bool P16>
@@ -743,10 +741,13 @@ bool resid_160(int64_t M, int N, int K) {
          2 * t160 > ncu;
 }
 
-// Tile choice. The LDS-staged epilogue (k_gemm) serves QKV and RESID,
-// whose outputs are scattered or need per-row reductions; the register
-// epilogue (k_gemm2) serves the plain stores of RELU2 and lm_head, with
-// 128x256 tiles (wave 64x128) when there are >= 1.5 blocks per CU.
+// Tile choice. The LDS-staged epilogue (k_gemm) serves QKV and RESID at every
+// size, whose outputs are scattered or need per-row reductions, the 128x192
+// tiles of RELU2, and both plain stores below 256 tiles of 128x128; the register
+// epilogue (k_gemm2) serves the larger RELU2 and lm_head GEMMs: 128x128 tiles,
+// RELU2 on 128x256 ones (wave 64x128) from 3 blocks per CU on, lm_head on
+// 256x256 or (8 wavefronts) 128x256 ones by the rules below, and either on
+// 256x256 past 4096 rows in fp16.
 
 template <int EPI, bool P16>
 void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
@@ -758,7 +759,7 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
     // barriers per K: 0.8 % of the 8 x 2048 eval forward (identical bits; at
     // 2048 rows the 128x256 tiles are 1.5 % slower with them)
     if (a.M > 4096 && a.N % 256 == 0) {
-      launch_cfg2<EPI, 2, 4, 4, 2, 2, P16, 64>(s, a, d_pos);
+      launch_cfg2<EPI, 2, 4, 4, 2, 2, P16, 64>(s, a);
       return;
     }
   }
@@ -770,12 +771,12 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
     // 4096 98 -> 72 / 122 -> 101, 600 20.9 -> 16.0 / 25.6 -> 22.0, 800 25.7 ->
     // 23.3 / 28.5 -> 26.6
     if (store_256(a.M, a.N, P16)) {
-      launch_cfg2<EPI, 2, 4, 4, 2, 2, P16>(s, a, d_pos);
+      launch_cfg2<EPI, 2, 4, 4, 2, 2, P16>(s, a);
       return;
     }
     const int64_t t256 = (a.M + 127) / 128 * (a.N / 256), ncu = cu_count();
     if (a.N % 256 == 0 && 8 * t256 >= 5 * ncu && t256 <= ncu) {
-      launch_cfg2<EPI, 2, 4, 2, 2, 3, P16>(s, a, d_pos);
+      launch_cfg2<EPI, 2, 4, 2, 2, 3, P16>(s, a);
       return;
     }
   }
@@ -794,11 +795,11 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
   const bool big = a.N % 128 == 0 && mt128 * (a.N / 128) >= 256;
   if constexpr (EPI == GV_RELU2 || EPI == GV_STORE) {
     if (EPI == GV_RELU2 && a.N % 256 == 0 && mt128 * (a.N / 256) >= 768) {
-      launch_cfg2<EPI, 2, 2, 2, 4, 2, P16>(s, a, d_pos);
+      launch_cfg2<EPI, 2, 2, 2, 4, 2, P16>(s, a);
       return;
     }
     if (big) {
-      launch_cfg2<EPI, 4, 2, 1, 2, 3, P16>(s, a, d_pos);
+      launch_cfg2<EPI, 4, 2, 1, 2, 3, P16>(s, a);
       return;
     }
   }
@@ -830,8 +831,9 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
   }
   const int bn = tile_n(a.M, a.N);
   if constexpr (EPI == GV_QKV) {
-    // 128x128 tiles where they fit in one round and 64x128 ones would need
-    // two (the depth-20 model at 2047 rows: 224 tiles against 448)
+    // 128x128 tiles from where 64x128 ones would need a second round (the
+    // depth-20 model at 2047 rows: 224 tiles against 448), but for the second
+    // case here
     const int64_t ncu = cu_count(), t128 = mt128 * (a.N / 128);
     const int64_t t64 = (int64_t)((a.M + 63) / 64) * (a.N / 128);
     // 64x64 tiles while 64x128 ones would leave CUs without one: us, fp16 /
@@ -850,7 +852,7 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
       else launch_cfg<EPI, 64, 128, 2, 2, 32, 3, 1, P16>(s, a, d_pos);
       return;
     }
-    if (bn == 128 && !big && t128 <= ncu && 2 * t128 > ncu) {
+    if (bn == 128 && !big) {
       launch_cfg<EPI, 128, 128, 4, 2, 32, 3, 1, P16>(s, a, d_pos);
       return;
     }
@@ -868,9 +870,9 @@ void launch_tile_p(hipStream_t s, const GemvArgs& a, const int32_t* d_pos) {
     // (half the stage hand-overs) measured ~4 us a launch faster than 32-wide
     // ones at any depth
     launch_cfg<EPI, 64, 128, 2, 2, 64, 3, 1, P16>(s, a, d_pos);
-  else if (bn == 128)
-    launch_cfg<EPI, 64, 128, 2, 2, 32, 4, 1, P16>(s, a, d_pos);
-  else
+  else if (bn == 128) {
+    if constexpr (EPI != GV_QKV) launch_cfg<EPI, 64, 128, 2, 2, 32, 4, 1, P16>(s, a, d_pos);
+  } else
     launch_cfg<EPI, 64, 64, 2, 2, 32, 4, 1, P16>(s, a, d_pos);
 }
 
@@ -934,10 +936,6 @@ void launch_gemm_pos(hipStream_t s, GemvEpi epi, const GemvArgs& a, const int32_
     case GV_RELU2: launch_tile<GV_RELU2>(s, a, d_pos); break;
     default: launch_tile<GV_STORE>(s, a, d_pos); break;
   }
-}
-
-void launch_gemm(hipStream_t s, GemvEpi epi, const GemvArgs& a) {
-  launch_gemm_pos(s, epi, a, nullptr);
 }
 
 }  // namespace fgpt

@@ -19,8 +19,11 @@
 // 4.5, proj2 9.3 -> 5.3; M = 7 8.3 -> 4.0, 6.8 -> 3.4, 8.2 -> 3.9, 7.9 -> 5.4;
 // M = 150 in fp16 against 64x64 LDS tiles 10.2 -> 5.9, 7.8 -> 3.5, 9.5 -> 4.8,
 // 17.7 -> 5.4.
-// Which wavefront takes which K range depends on K alone, so a row's result
-// does not depend on the tile or on the other rows of the pass.
+// Which wavefront takes which K range depends on K alone, so a row's products
+// are summed in the same order on every tile. The row norm is not: RESID leaves
+// one sum of squares per tile of columns, and those are added 512 / (16 TM)
+// threads at a time, so the row count of the pass, which picks the tile, moves
+// the last bits of a row.
 #include "fgpt_internal.h"
 #include "kern_common.h"
 #include "kern_epi.h"
