@@ -114,10 +114,10 @@ def test_forward_d12_vs_oracle(d12):
 
 @pytest.mark.parametrize("B,T", [(1, 48), (1, 1500), (2, 700)])
 def test_forward_d12_gemm_shapes(d12, B, T):
-    """Row counts that reach the other GEMM tilings: split-K partials and their
-    reduce (48 rows), and the 64x96 residual tiles whose K is split over
-    wavefront groups, with a partial last row tile (1400 and 1500 rows) and,
-    at B=2, a sequence boundary inside a tile."""
+    """Row counts that reach the other GEMM tilings: the few-row GEMM (48 rows),
+    and the 64x96 residual tiles whose K is split over wavefront groups, with a
+    partial last row tile (1400 and 1500 rows) and, at B=2, a sequence boundary
+    inside a tile."""
     d, w, m, c, s = d12
     ids = uniform_ids(40 + T, B * T, d.vocab).reshape(B, T)
     lg, _ = m.forward(ids, B, T)

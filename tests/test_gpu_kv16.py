@@ -139,14 +139,13 @@ def test_batched_bf16_chunks_merged():
     m.close()
 
 
-def test_batched_qkv_fold_gqa_vs_single_rows():
+def test_batched_steps_gqa_vs_single_rows():
     """B=40 sequences of the 5:1 GQA shape (5 query heads over one KV head,
     head_dim 128) on a bf16 cache, 400-id prompts: 200 (sequence, head)
-    rows take the looped decode attention (3 blocks of 128 positions per
-    workgroup, 2 chunks and a merge), which also finishes the QKV's split-K
-    sums (five workgroups per KV head fold the query, one of them appends
-    k/v). One plain step and two graph-replayed steps, against each
-    sequence decoded alone (single-row GEMV path, no fold): the appended
+    rows take the few-row GEMM, whose QKV epilogue appends k/v, and the looped
+    decode attention (3 blocks of 128 positions per workgroup, 2 chunks and a
+    merge). One plain step and two graph-replayed steps, against each
+    sequence decoded alone (single-row GEMV path): the appended
     layer-0 rows within one bf16 unit (the two paths sum the projection in
     different orders; elements near zero within 1e-5 of the row's largest),
     the logits within the bar, ids equal but at near-ties."""
@@ -190,7 +189,7 @@ def test_batched_qkv_fold_gqa_vs_single_rows():
                 # difference of the projection (elements near zero)
                 bar = 2.0 ** -7 * np.abs(r) + 1e-5 * np.abs(r).max()
                 assert np.all(np.abs(a - r) <= bar), (b, p, float(np.abs(a - r).max()))
-    record("qkv_fold_gqa5_b40", relerr=worst, flips=flips)
+    record("batched_steps_gqa5_b40", relerr=worst, flips=flips)
     assert worst < TOL
     for b, t, marg in flips:
         assert marg < 2 * TOL * np.abs(got_lg).max(), (b, t, marg)

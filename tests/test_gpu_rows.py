@@ -119,6 +119,60 @@ def test_chunk_without_logits(d, B, T, pos, kv16):
     m.close()
 
 
+@pytest.mark.parametrize("d,B,pos,T,kv16", [
+    (TINY, 1, 1190, 40, False),    # grouped KV: 1200 keys at most
+    (TINY, 1, 1200, 65, False),    # head_dim 64, two query blocks, split key ranges
+    (TINY, 1, 2540, 40, True), (SMALL, 1, 2530, 47, True),
+    (SMALL, 70, 33, 50, False), (SMALL, 70, 33, 50, True)])  # 840 workgroups
+def test_chunk_attention_from_planes(d, B, pos, T, kv16):
+    """Chunks past what the cache-row attention takes (attn_rows_fits): the
+    cached positions split into planes, k_attn_mfma after them, with the logits
+    and without (the last layer then skips the planes: the same cache, and the
+    id of the full pass's last row). Bounds as for the cache-row attention."""
+    n = pos + T
+    m, w, c, s = model(d, n)
+    ids = uniform_ids(81 + n, B * n, d.vocab).reshape(B, n)
+    ref = O.gpt_forward(ids.reshape(-1), c, s, w, d, B, n).reshape(B, n, -1)[:, pos:]
+    full, fast = m.kv(B, n, bf16=kv16), m.kv(B, n, bf16=kv16)
+    for kv in (full, fast):
+        for p in range(0, pos, 1000 if B == 1 else 25):
+            kv.step_multi(ids[:, p:min(p + (1000 if B == 1 else 25), pos)], want_logits=False)
+    held = m.bytes()[1]
+    lg, nxt = full.step_multi(ids[:, pos:])
+    if B == 1:  # (no more rows than before: what grew are the planes)
+        assert m.bytes()[1] - held >= 8 * n * d.n_kv_head * d.head_dim
+    else:
+        assert B * d.n_head * ((T + 15) // 16) > 640
+    assert rel(lg, ref) <= (4e-3 if kv16 else 5e-5)
+    assert np.array_equal(nxt, lg[:, -1].argmax(axis=1))
+    none, nx2 = fast.step_multi(ids[:, pos:], want_logits=False)
+    assert none is None
+    for a, b in zip(full.read(), fast.read()):
+        assert np.array_equal(a, b)
+    last = lg[:, -1]
+    assert np.all(last.max(axis=1) - last[np.arange(B), nx2] <= 1e-4 * np.abs(last).max())
+    full.close()
+    fast.close()
+    m.close()
+
+
+@pytest.mark.parametrize("d,B,T", [(TINY, 1, 1300), (TINY, 3, 1201), (SMALL, 2, 1400)])
+def test_forward_attention_from_planes(d, B, T):
+    """Forwards past the cache-row attention in split operands (head_dim 64 and
+    128), with and without the positive-score counts: the same logits bit for
+    bit; the counts differ from the oracle's at most by the scores whose sign is
+    within rounding (1e-4 of sum |q_d k_d|: 16 bits of each operand)."""
+    m, w, c, s = model(d, T)
+    ids = uniform_ids(91 + T, B * T, d.vocab)
+    ref, cnt, amb = O.gpt_forward_pos(ids, c, s, w, d, B, T, rel_tol=1e-4)
+    lg, _ = m.forward(ids, B, T)
+    assert rel(lg, ref) <= 5e-5
+    lgp, npos = m.forward_pos(ids, B, T)
+    assert np.array_equal(lg, lgp)
+    assert np.all(np.abs(npos.astype(np.int64) - cnt) <= amb)
+    m.close()
+
+
 WIDE1 = Dims(n_layer=1, d_model=768, n_head=6, n_kv_head=6, head_dim=128, vocab=256)
 VOCAB = Dims(n_layer=1, d_model=128, n_head=1, n_kv_head=1, head_dim=128, vocab=8192)
 

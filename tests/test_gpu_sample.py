@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 from autoresearch_amd import engine, trace
-from autoresearch_amd.weights import Dims, rope_tables, seeded_weights, uniform_ids
+from autoresearch_amd.weights import Dims, rope_tables, round_bf16, seeded_weights, uniform_ids
 from oracle import sample as S
 
 pytestmark = pytest.mark.gpu
@@ -224,6 +224,7 @@ def test_sampling_inside_the_persistent_loop(d, cfg):
     so the same ids and generator state, bit for bit. 48 ids: a row sorted whole
     sends the next 32 to the launches, and the loop is tried again."""
     m = engine.Model(d, stacks=seeded_weights(d, 9))
+    assert m.fused_decode()[0], m.fused_decode()[1]
     prompt = uniform_ids(19, 9, d.vocab)
     n_gen = 48
     c, s = rope_tables(prompt.size + n_gen, d.head_dim)
@@ -235,6 +236,8 @@ def test_sampling_inside_the_persistent_loop(d, cfg):
         m.timing(timing)
         outs.append(kv.decode_sample(prompt, n_gen, seed=1234567, **cfg))
         m.timing(False)
+        if cfg["temp"] in (0.0, 0.05):  # (the other rows of seeded weights are mostly flat)
+            assert m.sampled_in_loop() == (0 if timing else n_gen)
         kv.close()
     assert np.array_equal(outs[0][0], outs[1][0]) and outs[0][1] == outs[1][1]
     m.close()
@@ -266,6 +269,53 @@ def test_flat_rows_are_not_sorted_in_the_loop(d, cfg, share):
         m.timing(False)
         assert m.sampled_in_loop() == (0 if timing else share * n_gen)
         assert kv.len == prompt.size + n_gen - 1
+        kv.close()
+    assert np.array_equal(outs[0][0], outs[1][0]) and outs[0][1] == outs[1][1]
+    m.close()
+
+
+def peaked_weights(d, seed):
+    """Seeded weights whose lm_head gives every id six likely successors, 15,
+    14.5, .. 12.5 above the others' logits (of standard deviation 0.02
+    sqrt(d_model)), from its own block of 32 ids: rows of which a cut keeps a
+    few ids, and histories that repeat."""
+    w = seeded_weights(d, seed)
+    V, D = d.vocab, d.d_model
+    lm, wte = w["lm_head"].reshape(V, D).copy(), w["wte"].reshape(V, D)
+    i = np.arange(V)
+    for k, step in enumerate((1, 3, 7, 12, 20, 27)):
+        lm[i // 32 * 32 + (i + step) % 32] += (15 - 0.5 * k) / (0.02 * D) * wte
+    w["lm_head"] = round_bf16(lm.reshape(-1))
+    return w
+
+
+@pytest.mark.parametrize("d", [SMALL_MHA, Dims(n_layer=1, d_model=768, n_head=6, n_kv_head=6,
+                                               head_dim=128, vocab=8192)], ids=["1k", "8k"])
+@pytest.mark.parametrize("cfg", [
+    dict(temp=0.8, topp=0.9), dict(temp=0.8, topp=0.98), dict(temp=0.8, topp=1e-6),
+    dict(temp=0.9, topp=0.95, pres=0.4, freq=0.3),
+    dict(temp=0.8, topp=0.9, pwin=5, pres=0.3, freq=0.2, rep=1.2),
+    dict(temp=0.8, topp=0.9, pwin=100, plen=0.4, freq=0.2), dict(temp=0.9, topp=0.9, rep=1.3),
+    dict(temp=0.9, topp=0.9, nblock=2), dict(temp=0.8, topp=0.9, pres=0.1, freq=0.1, rep=1.1, nblock=3),
+    dict(temp=0.8, topp=0.9, byte_space=True, freq=0.5), dict(temp=0.0, pres=0.5, rep=1.2, nblock=2)])
+def test_every_id_drawn_in_the_loop(d, cfg):
+    """Peaked rows, with each penalty, window and ban at work on a growing
+    history: all 96 ids are drawn inside the persistent loop, and are, with the
+    generator's state, those of one launch and one k_sample_step per id."""
+    m = engine.Model(d, stacks=peaked_weights(d, 9))
+    assert m.fused_decode()[0], m.fused_decode()[1]
+    prompt = uniform_ids(19, 9, 96)  # (ids that byte_space allows, and their blocks)
+    n_gen = 96
+    c, s = rope_tables(prompt.size + n_gen, d.head_dim)
+    m.set_rope(c.reshape(-1), s.reshape(-1))
+    outs = []
+    for timing in (True, False):
+        kv = m.kv(1, prompt.size + n_gen)
+        kv.step_multi(prompt[:-1], want_logits=False)
+        m.timing(timing)
+        outs.append(kv.decode_sample(prompt, n_gen, seed=20240, **cfg))
+        m.timing(False)
+        assert m.sampled_in_loop() == (0 if timing else n_gen)
         kv.close()
     assert np.array_equal(outs[0][0], outs[1][0]) and outs[0][1] == outs[1][1]
     m.close()
