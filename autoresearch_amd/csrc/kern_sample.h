@@ -1,6 +1,7 @@
 // kern_sample.h -- sample_next of src/lib/sample.f90:153-233 for one row of
-// logits: the generator and sort keys of both device forms, and the form that
-// the persistent decode runs between two of its steps (sample_wg).
+// logits: what both device forms share (the generator, the sort keys, the
+// penalties), and the form that the persistent decode runs between two of its
+// steps (sample_wg).
 #pragma once
 #include <float.h>
 
@@ -29,6 +30,91 @@ __device__ __forceinline__ float rand_u01(int64_t* st) {
 __device__ __forceinline__ uint64_t prob_key(float p, int id) {
   return ((uint64_t)__float_as_uint(p) << 32) | (uint32_t)(0x7fffffff - id);
 }
+
+// The row's penalties, n-gram ban and byte mask, in the reference's order:
+// presence and frequency over the whole history or its last pwin ids (:33-51,
+// :77-104), the repetition penalty (:56-71), the no-repeat n-gram ban
+// (:109-130), the byte-level ids (:141-151). X is how the caller's threads
+// split an index range (each), meet (sync), read an id of the history (id) and
+// count it from an index on (count, then n_of).
+template <class X>
+__device__ __forceinline__ void penalise(X& x, float* pr, int V, int ngen, const SampleCfg& c) {
+#pragma clang fp contract(off)
+  const int lo = c.pwin > 0 && ngen > c.pwin ? ngen - c.pwin : 0;
+  if ((c.pres != 0.f || c.freq != 0.f) && ngen > 0) {  // l - pres - freq * count
+    x.count(lo);
+    x.each(0, V, [&](int i) {
+#pragma clang fp contract(off)
+      const int n = x.n_of(i);
+      if (n > 0) pr[i] = (pr[i] - c.pres) - c.freq * (float)n;
+    });
+    x.sync();
+  }
+  if (c.pwin > 0 && ngen > 0 && c.plen != 0.f && ngen < c.pwin) {
+    if (threadIdx.x == 0) pr[0] = pr[0] - (c.plen * (float)(c.pwin - ngen)) / (float)c.pwin;
+    x.sync();
+  }
+  if (c.rep > 1.f && ngen > 0) {  // over the whole history: l / theta
+    x.count(0);
+    x.each(0, V, [&](int i) {
+      if (x.n_of(i) > 0) pr[i] = pr[i] / c.rep;
+    });
+    x.sync();
+  }
+  const int nn = c.nblock;
+  if (nn >= 2 && ngen >= nn) {  // ids that would complete an n-gram of the history
+    x.each(0, ngen - nn + 1, [&](int s) {
+      int k = 0;
+      while (k < nn - 1 && x.id(s + k) == x.id(ngen - nn + 1 + k)) ++k;
+      if (k == nn - 1) {
+        const int t = x.id(s + nn - 1);
+        if (t >= 0 && t < V) pr[t] = -FLT_MAX;
+      }
+    });
+    x.sync();
+  }
+  if (c.byte_space) {
+    x.each(0, V, [&](int i) {
+      if (!(i < 128 || (i >= 256 && i < 512))) pr[i] = -FLT_MAX;
+    });
+    x.sync();
+  }
+}
+
+// How 256 of a workgroup's threads (comp; the others only keep the barriers) go
+// through penalise().
+template <int V>
+struct WalkWG {
+  uint32_t* cnt;  // [V / 2]: 16-bit counts, two a word (histories are below 2^16)
+  const int32_t* gen;
+  int ngen;
+  bool comp;
+  int counted = -1;  // history start that cnt holds
+  template <class F>
+  __device__ __forceinline__ void each(int lo, int hi, F&& f) {
+    if (comp)
+      for (int i = lo + (int)threadIdx.x; i < hi; i += 256) f(i);
+  }
+  __device__ __forceinline__ void sync() { lds_barrier(); }
+  // (the history is this workgroup's own stores of earlier steps)
+  __device__ __forceinline__ int id(int j) {
+    return __hip_atomic_load(gen + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ __forceinline__ void count(int lo) {
+    if (counted == lo) return;
+    counted = lo;
+    each(0, V / 2, [&](int i) { cnt[i] = 0; });
+    lds_barrier();
+    each(lo, ngen, [&](int j) {
+      const int g = id(j);
+      if (g >= 0 && g < V) atomicAdd(&cnt[g >> 1], 1u << (16 * (g & 1)));
+    });
+    lds_barrier();
+  }
+  __device__ __forceinline__ int n_of(int i) {
+    return (int)((cnt[i >> 1] >> (16 * (i & 1))) & 0xFFFFu);
+  }
+};
 
 // The sampling of one row by 256 of a workgroup's threads (comp; the others
 // only keep the barriers), V a power of two, from pr[V] in LDS, which is
@@ -60,72 +146,13 @@ __device__ int sample_wg(float* pr, uint8_t* aux, const int32_t* gen, int ngen, 
   constexpr int NT = 256, PER = V / SVT, MAXC = V / 8, NK = 6;
   static_assert(V >= SVT && (V & (V - 1)) == 0 && 8 * MAXC <= 2 * V, "V a power of two");
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  uint32_t* cnt = (uint32_t*)aux;       // 16-bit counts, two a word (histories are below 2^16)
   uint64_t* keys = (uint64_t*)aux;      // [MAXC]
   float* tot = (float*)(aux + 2 * V);   // [SVT]
   float* red = tot + SVT;               // [16]
   int* ri = (int*)(red + 16);           // [16]
   float* mred = (float*)(ri + 16);      // [4] and a broadcast
-  // (the history is this workgroup's own stores of earlier steps)
-  auto G = [&](int j) {
-    return __hip_atomic_load(gen + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  int counted = -1;  // history start that cnt holds
-  auto count = [&](int lo) {
-    if (counted == lo) return;
-    counted = lo;
-    if (comp)
-      for (int i = tid; i < V / 2; i += NT) cnt[i] = 0;
-    lds_barrier();
-    if (comp)
-      for (int j = lo + tid; j < ngen; j += NT) {
-        const int g = G(j);
-        if (g >= 0 && g < V) atomicAdd(&cnt[g >> 1], 1u << (16 * (g & 1)));
-      }
-    lds_barrier();
-  };
-  auto n_of = [&](int i) { return (int)((cnt[i >> 1] >> (16 * (i & 1))) & 0xFFFFu); };
-  // penalties, the n-gram ban and the byte mask, in sample_row's order
-  const int lo = c.pwin > 0 && ngen > c.pwin ? ngen - c.pwin : 0;
-  if ((c.pres != 0.f || c.freq != 0.f) && ngen > 0) {
-    count(lo);
-    if (comp)
-      for (int i = tid; i < V; i += NT) {
-        const int n = n_of(i);
-        if (n > 0) pr[i] = (pr[i] - c.pres) - c.freq * (float)n;
-      }
-    lds_barrier();
-  }
-  if (c.pwin > 0 && ngen > 0 && c.plen != 0.f && ngen < c.pwin) {
-    if (tid == 0) pr[0] = pr[0] - (c.plen * (float)(c.pwin - ngen)) / (float)c.pwin;
-    lds_barrier();
-  }
-  if (c.rep > 1.f && ngen > 0) {
-    count(0);
-    if (comp)
-      for (int i = tid; i < V; i += NT)
-        if (n_of(i) > 0) pr[i] = pr[i] / c.rep;
-    lds_barrier();
-  }
-  const int nn = c.nblock;
-  if (nn >= 2 && ngen >= nn) {
-    if (comp)
-      for (int s = tid; s <= ngen - nn; s += NT) {
-        int k = 0;
-        while (k < nn - 1 && G(s + k) == G(ngen - nn + 1 + k)) ++k;
-        if (k == nn - 1) {
-          const int t = G(s + nn - 1);
-          if (t >= 0 && t < V) pr[t] = -FLT_MAX;
-        }
-      }
-    lds_barrier();
-  }
-  if (c.byte_space) {
-    if (comp)
-      for (int i = tid; i < V; i += NT)
-        if (!(i < 128 || (i >= 256 && i < 512))) pr[i] = -FLT_MAX;
-    lds_barrier();
-  }
+  WalkWG<V> walk{(uint32_t*)aux, gen, ngen, comp};
+  penalise(walk, pr, V, ngen, c);
   if (c.temp <= 0.f) {  // the first maximum, no draw
     float bv = -INFINITY;
     int bi = 0x7fffffff;

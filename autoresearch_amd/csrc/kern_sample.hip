@@ -94,16 +94,32 @@ __device__ int block_min(int v, int* red) {
   return v;
 }
 
-// per-id counts of gen[lo:hi) into cnt[0:V) (ids outside [0, V) ignored)
-__device__ void count_ids(const int32_t* gen, int lo, int hi, int V, int* cnt) {
-  for (int i = threadIdx.x; i < V; i += ST) cnt[i] = 0;
-  __syncthreads();
-  for (int j = lo + threadIdx.x; j < hi; j += ST) {
-    const int g = gen[j];
-    if (g >= 0 && g < V) atomicAdd(&cnt[g], 1);
+// How the ST threads of a sampling workgroup go through penalise(): counts in
+// cnt[0:V) (ids outside [0, V) ignored).
+struct WalkST {
+  int* cnt;
+  const int32_t* __restrict__ gen;
+  int ngen, V;
+  int counted = -1;  // history start that cnt holds
+  template <class F>
+  __device__ __forceinline__ void each(int lo, int hi, F&& f) {
+    for (int i = lo + (int)threadIdx.x; i < hi; i += ST) f(i);
   }
-  __syncthreads();
-}
+  __device__ __forceinline__ void sync() { __syncthreads(); }
+  __device__ __forceinline__ int id(int j) { return gen[j]; }
+  __device__ __forceinline__ void count(int lo) {
+    if (counted == lo) return;
+    counted = lo;
+    each(0, V, [&](int i) { cnt[i] = 0; });
+    __syncthreads();
+    each(lo, ngen, [&](int j) {
+      const int g = gen[j];
+      if (g >= 0 && g < V) atomicAdd(&cnt[g], 1);
+    });
+    __syncthreads();
+  }
+  __device__ __forceinline__ int n_of(int i) { return cnt[i]; }
+};
 
 // v of lane (lane ^ D), D a power of two below 64: DPP within quads, a
 // swizzle within 32-lane halves, a permute across them
@@ -235,54 +251,10 @@ __device__ int sample_row(const float* __restrict__ logits, int V, int np2,
   __shared__ int ri[NW];
   __shared__ float bcast;
   const int tid = threadIdx.x;
-  int* cnt = (int*)aux;
   for (int i = tid; i < V; i += ST) pr[i] = logits[i];
   __syncthreads();
-  // presence + frequency: once per distinct id, l - pres - freq * count
-  if (c.pwin > 0) {
-    if (ngen > 0) {
-      const int lo = ngen - c.pwin > 0 ? ngen - c.pwin : 0;
-      if (c.pres != 0.f || c.freq != 0.f) {
-        count_ids(gen, lo, ngen, V, cnt);
-        for (int i = tid; i < V; i += ST)
-          if (cnt[i] > 0) pr[i] = (pr[i] - c.pres) - c.freq * (float)cnt[i];
-        __syncthreads();
-      }
-      if (c.plen != 0.f && ngen < c.pwin && tid == 0)
-        pr[0] = pr[0] - (c.plen * (float)(c.pwin - ngen)) / (float)c.pwin;
-      __syncthreads();
-    }
-  } else if ((c.pres != 0.f || c.freq != 0.f) && ngen > 0) {
-    count_ids(gen, 0, ngen, V, cnt);
-    for (int i = tid; i < V; i += ST)
-      if (cnt[i] > 0) pr[i] = (pr[i] - c.pres) - c.freq * (float)cnt[i];
-    __syncthreads();
-  }
-  // repetition penalty over the whole history: l / theta
-  if (c.rep > 1.f && ngen > 0) {
-    count_ids(gen, 0, ngen, V, cnt);
-    for (int i = tid; i < V; i += ST)
-      if (cnt[i] > 0) pr[i] = pr[i] / c.rep;
-    __syncthreads();
-  }
-  // no-repeat n-gram: ids that would complete an n-gram seen in history
-  const int nn = c.nblock;
-  if (nn >= 2 && ngen >= nn) {
-    for (int s = tid; s <= ngen - nn; s += ST) {
-      int k = 0;
-      while (k < nn - 1 && gen[s + k] == gen[ngen - nn + 1 + k]) ++k;
-      if (k == nn - 1) {
-        const int t = gen[s + nn - 1];
-        if (t >= 0 && t < V) pr[t] = -FLT_MAX;
-      }
-    }
-    __syncthreads();
-  }
-  if (c.byte_space) {
-    for (int i = tid; i < V; i += ST)
-      if (!(i < 128 || (i >= 256 && i < 512))) pr[i] = -FLT_MAX;
-    __syncthreads();
-  }
+  WalkST walk{(int*)aux, gen, ngen, V};
+  penalise(walk, pr, V, ngen, c);
   if (c.temp <= 0.f) return block_argmax(pr, V, rv, ri);
 
   // temperature softmax
